@@ -398,7 +398,7 @@ def main() -> int:
         alg = BAND_FWD_BYTES["fp64"] * case.npts
         achieved = alg / (t * 1e-3) / 1e9
         line["roofline"] = {
-            "bound": "hbm", "kernel": "k_band_ring<fwd,double> (LU-SGS forward band sweep, LDS-ring form)",
+            "bound": "hbm", "kernel": "k_band<3,fwd,double> (LU-SGS forward band sweep)",
             "achieved": round(achieved, 3), "peak": PEAK_HBM_GBS, "unit": "GB/s",
             "frac": round(achieved / PEAK_HBM_GBS, 6),
             "traffic": round(BAND_FWD_TRAFFIC["fp64"] * case.npts),

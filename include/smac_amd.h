@@ -167,9 +167,9 @@ smac_status smac_timings(smac_handle *h, double out[7]);
 /* Options: "keep_lhs" (1: keep a copy of the five assembled blocks of each pass for
  * smac_get_array), "timing" (1: time kernel families with HIP events on the handle's
  * stream), "lusgs_rows" (1..64, default 64: grid rows per wavefront band of the LU-SGS
- * sweeps), "lusgs_prefetch" / "lusgs_prefetch_sa" (1, 2, 3, 4, 6 or 8; defaults 4 and 8:
- * steps of operand prefetch in the 3x3 / scalar LU-SGS sweeps), "lusgs_ring" (0 or 1, default 1:
- * the 3x3 sweeps stream their operands through an LDS ring fed by loader wavefronts),
+ * sweeps; the 3x3 sweeps take at most 16), "lusgs_prefetch" / "lusgs_prefetch_sa" (1, 2, 3, 4,
+ * 6 or 8) and "lusgs_ring" (0 or 1) (accepted, without effect: the sweeps have one form, fed
+ * through an LDS ring),
  * "lr_lines" (1..64, default 64: lines per workgroup of the line-relaxation
  * factorisations), "adj_restart" (4..400, default 100: GMRES restart length of
  * smac_adjoint), "adj_prec_steps" (1..8, default 3: steps of the transposed update per

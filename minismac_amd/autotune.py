@@ -4,10 +4,9 @@ The tunable knobs change how the work is cut into workgroups, never the arithmet
 are bit-identical for every setting):
 
 * ``lusgs_rows``        grid rows per wavefront band of the LU-SGS hyperplane sweeps;
-* ``lusgs_prefetch``    steps of operand prefetch in the 3x3 (mean-flow) band sweeps;
-* ``lusgs_prefetch_sa`` the same for the scalar (Spalart-Allmaras) band sweeps;
-* ``lusgs_ring``        1: the 3x3 sweeps stream their operands through an LDS ring fed by
-                        loader wavefronts (then ``lusgs_prefetch`` is not used);
+* ``lusgs_prefetch``, ``lusgs_prefetch_sa``, ``lusgs_ring``
+                        accepted by the library without effect (the sweeps have one form), so
+                        each has one value here;
 * ``lr_lines``          lines per workgroup of the line-relaxation factorisations.
 
 ``tune(case)`` times candidate settings on a private copy of the case (its own device
@@ -27,10 +26,10 @@ from .solver import Solver
 
 CACHE_ENV = "MINISMAC_AMD_TUNE_CACHE"
 
-LUSGS_ROWS = (16, 24, 32, 48, 64)
-LUSGS_PREFETCH = (2, 3, 4, 6, 8)
-LUSGS_PREFETCH_SA = (2, 4, 6, 8)
-LUSGS_RING = (0, 1)
+LUSGS_ROWS = (16, 32, 64)
+LUSGS_PREFETCH = (4,)
+LUSGS_PREFETCH_SA = (8,)
+LUSGS_RING = (1,)
 LR_LINES = (8, 16, 32, 64)
 # a setting replaces the current one only when it is faster by more than this fraction
 # (wall-clock noise of a few passes)

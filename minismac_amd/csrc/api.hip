@@ -70,7 +70,6 @@ struct smac_handle {
     WakePairs wake = {};
     LusgsWs lws = {};          // LU-SGS sheared workspace (impsch = 2)
     int lusgs_rows = 64;
-    int lusgs_ring = 1;    // the 3x3 sweeps stream their operands through an LDS ring
     int lr_lines = 64;     // lines per workgroup of the line-relaxation factor kernels
     int lr_refactor = 1;   // scan/zebra forms: factor the lines every this many passes
     long lr_factored = -1; // the pass whose blocks the line operands hold (-1: none)
@@ -147,30 +146,24 @@ static void free_lusgs_ws(smac_handle *h)
 
 static smac_status alloc_one_ws(smac_handle *h, int rows, int neqs, LusgsWs &w)
 {
-    const int pf3 = w.pf3, pf1 = w.pf1, ring = w.ring;
     hipEvent_t e0 = w.ev_fwd[0], e1 = w.ev_fwd[1];
     w = LusgsWs{};
-    w.pf3 = pf3;
-    w.pf1 = pf1;
-    w.ring = ring;
     w.ev_fwd[0] = e0;
     w.ev_fwd[1] = e1;
-    lusgs_ws_shape(h->d.jm, h->d.km, rows, w);
-    if (!lusgs_ws_fits(w)) return fail(SMAC_ERR_SIZE, "grid too large for the LU-SGS workspace");
-    void *p[4] = {};
-    size_t sz[4] = {(size_t)lusgs_ws_lhs_bytes(w, neqs), (size_t)lusgs_ws_vec_bytes(w, neqs),
-                    (size_t)lusgs_ws_vec_bytes(w, neqs), (size_t)(w.nedge * 8)};
-    for (int i = 0; i < 4; ++i) {
+    lusgs_ws_shape(h->d.jm, h->d.km, rows, neqs, w);
+    if (!lusgs_size_ok(h->d.jm, h->d.km, rows))
+        return fail(SMAC_ERR_SIZE, "grid too large for the LU-SGS workspace");
+    void *p[2] = {};
+    size_t sz[2] = {(size_t)lusgs_ws_lhs_bytes(w, neqs), (size_t)(w.nedge * 8)};
+    for (int i = 0; i < 2; ++i) {
         HIP_TRY(hipMalloc(&p[i], sz[i] + 256));
         h->lws_allocs.push_back(p[i]);
-        // the padding of the sheared planes is read (and ignored) by idle lanes, and the
-        // hand-over padding must not hold the sentinel: start from zeros
+        // the padding of the chunks is read by lanes without a row, and the hand-over padding
+        // must not hold the sentinel: start from zeros
         HIP_TRY(hipMemset(p[i], 0, sz[i] + 256));
     }
     w.lhs = p[0];
-    w.r = p[1];
-    w.dq = p[2];
-    w.edge = (unsigned long long *)p[3];
+    w.edge = (unsigned long long *)p[1];
     w.stall = &h->st->stall;
     return SMAC_OK;
 }
@@ -178,20 +171,15 @@ static smac_status alloc_one_ws(smac_handle *h, int rows, int neqs, LusgsWs &w)
 // LU-SGS workspaces: the mean flow (neqs = 3) and the SA (neqs = 1), which may run at once
 static smac_status alloc_lusgs_ws(smac_handle *h, int rows)
 {
-    const LusgsWs keep = h->lws, keep_sa = h->lws_sa;
+    const LusgsWs keep = h->lws;
     free_lusgs_ws(h);
     h->lws.ev_fwd[0] = keep.ev_fwd[0];
     h->lws.ev_fwd[1] = keep.ev_fwd[1];
-    h->lws.pf3 = keep.pf3;
-    h->lws.pf1 = keep.pf1;
-    h->lws.ring = h->lusgs_ring;
-    h->lws_sa.pf3 = keep_sa.pf3;
-    h->lws_sa.pf1 = keep_sa.pf1;
     smac_status rc = alloc_one_ws(h, rows, 3, h->lws);
     if (rc) return rc;
     rc = alloc_one_ws(h, rows, 1, h->lws_sa);
     if (rc) return rc;
-    h->lusgs_rows = h->lws.rows;
+    h->lusgs_rows = rows;
     return SMAC_OK;
 }
 
@@ -439,19 +427,14 @@ smac_status smac_set_option(smac_handle *h, const char *name, int value)
         return SMAC_OK;
     }
     if (!std::strcmp(name, "lusgs_prefetch") || !std::strcmp(name, "lusgs_prefetch_sa")) {
-        const bool mean = !std::strcmp(name, "lusgs_prefetch");
         const bool ok = value == 1 || value == 2 || value == 3 || value == 4 || value == 6 ||
                         value == 8;
         if (!ok) return fail(SMAC_ERR_ARG, std::string(name) + ": unsupported prefetch distance");
-        if (mean) h->lws.pf3 = value;
-        else h->lws_sa.pf1 = value;
-        return SMAC_OK;
+        return SMAC_OK;   // the sweeps have one form; the setting is accepted and has no effect
     }
     if (!std::strcmp(name, "lusgs_ring")) {
         if (value != 0 && value != 1) return fail(SMAC_ERR_ARG, "lusgs_ring must be 0 or 1");
-        h->lusgs_ring = value;
-        h->lws.ring = value;
-        return SMAC_OK;
+        return SMAC_OK;   // as above
     }
     if (!std::strcmp(name, "lr_solve")) {
         if (value != 0 && value != 1) return fail(SMAC_ERR_ARG, "lr_solve must be 0 or 1");
@@ -923,7 +906,6 @@ static smac_status adj_prepare(smac_handle *h, int m)
     if (h->p.impsch != 1)
         for (LusgsWs *ws : {&h->adj_ws, &h->adj_ws2})
             if (!ws->lhs) {
-                ws->ring = 1;
                 smac_status rc = alloc_one_ws(h, 64, 3, *ws);
                 if (rc) return rc;
             }
@@ -1053,7 +1035,7 @@ struct BandGroup {
     std::vector<int> members;        // indices into cases
     BandJob *jobs = nullptr;         // device
     int2 *map = nullptr;             // device
-    int nblk = 0, pf = 3;
+    int nblk = 0;
 };
 
 // streams over which the per-case kernels of a batch phase are spread
@@ -1203,12 +1185,10 @@ static void free_batch(smac_batch *b)
 
 static bool same_ws(const LusgsWs &a, const LusgsWs &c)
 {
-    return a.lhs == c.lhs && a.r == c.r && a.dq == c.dq && a.edge == c.edge &&
-           a.nband == c.nband && a.rows == c.rows && a.pf3 == c.pf3 && a.pf1 == c.pf1 &&
-           a.ring == c.ring;
+    return a.lhs == c.lhs && a.edge == c.edge && a.nband == c.nband && a.rows == c.rows;
 }
 
-static smac_status build_group(BandGroup &g, const std::vector<BandJob> &jobs, int pf)
+static smac_status build_group(BandGroup &g, const std::vector<BandJob> &jobs)
 {
     free_group(g);
     if (g.members.size() != jobs.size()) return fail(SMAC_ERR_ARG, "batch table mismatch");
@@ -1216,7 +1196,6 @@ static smac_status build_group(BandGroup &g, const std::vector<BandJob> &jobs, i
     for (size_t i = 0; i < jobs.size(); ++i)
         for (int blk = 0; blk < jobs[i].w.nband; ++blk) map.push_back(make_int2((int)i, blk));
     g.nblk = (int)map.size();
-    g.pf = pf;
     if (jobs.empty()) return SMAC_OK;
     if (hipMalloc(&g.jobs, jobs.size() * sizeof(BandJob)) != hipSuccess ||
         hipMalloc(&g.map, map.size() * sizeof(int2)) != hipSuccess)
@@ -1258,10 +1237,10 @@ static smac_status build_multi(smac_batch *b)
             sd.v.push_back(sa_deriv_args(d, h->q, h->met, h->dj, a));
             sas.v.push_back(sa_asm_args(d, dp, 0, h->q, h->met, h->dj, a));
             sa_bc_args(d, (int)h->regs.size(), h->regs.data(), a, sbc.v);
-            ssh.v.push_back(shear_args<double>(d, h->lws_sa, a.sf, a.stc, a.sjm, a.sjp, a.skm,
+            ssh.v.push_back(shear_args<double, 1>(d, h->lws_sa, a.sf, a.stc, a.sjm, a.sjp, a.skm,
                                              a.skp, (double *)nullptr));
             smid.v.push_back(mid_args<double, 1>(d, h->lws_sa));
-            sun.v.push_back(unshear_args(d, h->lws_sa, h->lws_sa.dq, a.ds));
+            sun.v.push_back(unshear_args(d, h->lws_sa, a.ds));
             swk.v.push_back(wake_args(d, 1, h->wake, a.anut, a.ds, a.sf));
             sup.v.push_back(sa_upd_args(d, dp, h->w, a));
             stu.v.push_back(sa_tur_args(h->w, h->st));
@@ -1274,7 +1253,7 @@ static smac_status build_multi(smac_batch *b)
                                             fb[3], fb[4]));
             bc_args<float>(d, dp, h->regs.data(), (int)h->regs.size(), h->st, h->x, h->y, h->met,
                            h->q, h->s, fb[0], fb[1], fb[2], fb[3], fb[4], bc[g].v);
-            sh[g].v.push_back(shear_args<float>(d, h->lws, h->s, fb[0], fb[1], fb[2], fb[3], fb[4],
+            sh[g].v.push_back(shear_args<float, 3>(d, h->lws, h->s, fb[0], fb[1], fb[2], fb[3], fb[4],
                                               (float *)nullptr));
             mid[g].v.push_back(mid_args<float, 3>(d, h->lws));
         } else {
@@ -1283,11 +1262,11 @@ static smac_status build_multi(smac_batch *b)
                                              db[2], db[3], db[4]));
             bc_args<double>(d, dp, h->regs.data(), (int)h->regs.size(), h->st, h->x, h->y,
                             h->met, h->q, h->s, db[0], db[1], db[2], db[3], db[4], bc[g].v);
-            sh[g].v.push_back(shear_args<double>(d, h->lws, h->s, db[0], db[1], db[2], db[3], db[4],
+            sh[g].v.push_back(shear_args<double, 3>(d, h->lws, h->s, db[0], db[1], db[2], db[3], db[4],
                                                (double *)nullptr));
             mid[g].v.push_back(mid_args<double, 3>(d, h->lws));
         }
-        un[g].v.push_back(unshear_args(d, h->lws, h->lws.dq, h->dq));
+        un[g].v.push_back(unshear_args(d, h->lws, h->dq));
         rp.v.push_back(residp_args(d, h->s, h->dj, h->w));
         rf.v.push_back(residf_args(d, 2, dp.beta, h->s, h->dj, h->w, h->st));   // nt > 1
         wk.v.push_back(wake_args(d, 3, h->wake, h->q, h->dq, h->s));
@@ -1333,7 +1312,6 @@ static smac_status build_tables(smac_batch *b)
     b->mean[1].members.clear();
     b->snap_mean.clear();
     b->snap_sa.clear();
-    int pf_sa = 0, pf_m[2] = {0, 0};
     for (size_t i = 0; i < b->cases.size(); ++i) {
         smac_handle *h = b->cases[i];
         b->snap_mean.push_back(h->lws);
@@ -1344,21 +1322,16 @@ static smac_status build_tables(smac_batch *b)
         const int g = h->p.precision == SMAC_FP32_LHS ? 1 : 0;
         b->mean[g].members.push_back((int)i);
         jm[g].push_back(BandJob{h->d, w, (int)i});
-        if (!pf_m[g]) pf_m[g] = w.ring ? -1 : w.pf3;
         if (has_sa(h)) {
             LusgsWs ws = h->lws_sa;
             ws.ev_fwd[0] = ws.ev_fwd[1] = nullptr;
             b->sa.members.push_back((int)i);
             jsa.push_back(BandJob{h->d, ws, (int)i});
-            if (!pf_sa) pf_sa = ws.pf1;
         }
     }
-    // the sweep form (LDS ring or register prefetch) and prefetch distance of a multi-case
-    // launch are those of its first case (every form and distance gives the same results)
-    B_TRY(build_group(b->sa, jsa, pf_sa ? pf_sa : 8));
-    // pf 0 selects the LDS-ring sweeps
-    B_TRY(build_group(b->mean[0], jm[0], pf_m[0] < 0 ? 0 : (pf_m[0] ? pf_m[0] : 4)));
-    B_TRY(build_group(b->mean[1], jm[1], pf_m[1] < 0 ? 0 : (pf_m[1] ? pf_m[1] : 4)));
+    B_TRY(build_group(b->sa, jsa));
+    B_TRY(build_group(b->mean[0], jm[0]));
+    B_TRY(build_group(b->mean[1], jm[1]));
     return build_multi(b);
 }
 
@@ -1412,9 +1385,9 @@ static smac_status enqueue_batch_pass_multi(smac_batch *b, bool time_band)
     multi_shear<double, 1>(ss, b->sa_shear);
     BandGroup &gs = b->sa;
     if (gs.nblk) {
-        lusgs_band_multi<double, 1>(ss, gs.jobs, gs.map, gs.nblk, gs.pf, true, b->active);
+        lusgs_band_multi<double, 1>(ss, gs.jobs, gs.map, gs.nblk, true, b->active);
         multi_mid<double, 1>(ss, b->sa_mid);
-        lusgs_band_multi<double, 1>(ss, gs.jobs, gs.map, gs.nblk, gs.pf, false, b->active);
+        lusgs_band_multi<double, 1>(ss, gs.jobs, gs.map, gs.nblk, false, b->active);
     }
     multi_unshear<double, 1>(ss, b->sa_unshear);
     multi_wake(ss, b->sa_wake);
@@ -1436,15 +1409,15 @@ static smac_status enqueue_batch_pass_multi(smac_batch *b, bool time_band)
         const bool rec = time_band && g == b->band_group;
         if (rec) HIP_TRY(hipEventRecord(b->ev_band[0], sm));
         if (g == 0)
-            lusgs_band_multi<double, 3>(sm, gm.jobs, gm.map, gm.nblk, gm.pf, true, b->active);
+            lusgs_band_multi<double, 3>(sm, gm.jobs, gm.map, gm.nblk, true, b->active);
         else
-            lusgs_band_multi<float, 3>(sm, gm.jobs, gm.map, gm.nblk, gm.pf, true, b->active);
+            lusgs_band_multi<float, 3>(sm, gm.jobs, gm.map, gm.nblk, true, b->active);
         if (rec) HIP_TRY(hipEventRecord(b->ev_band[1], sm));
         if (g == 0) {
             multi_mid<double, 3>(sm, b->mid[0]);
-            lusgs_band_multi<double, 3>(sm, gm.jobs, gm.map, gm.nblk, gm.pf, false, b->active);
+            lusgs_band_multi<double, 3>(sm, gm.jobs, gm.map, gm.nblk, false, b->active);
         } else {
-            lusgs_band_multi<float, 3>(sm, gm.jobs, gm.map, gm.nblk, gm.pf, false, b->active);
+            lusgs_band_multi<float, 3>(sm, gm.jobs, gm.map, gm.nblk, false, b->active);
         }
     }
     multi_unshear<double, 3>(sm, b->unshear[0]);
@@ -1500,7 +1473,7 @@ static smac_status enqueue_batch_pass(smac_batch *b, bool time_band,
     B_TRY(join_lanes(b));
     BandGroup &gs = b->sa;
     if (gs.nblk) {
-        lusgs_band_multi<double, 1>(sm, gs.jobs, gs.map, gs.nblk, gs.pf, true, act);
+        lusgs_band_multi<double, 1>(sm, gs.jobs, gs.map, gs.nblk, true, act);
         B_TRY(fork_lanes(b));
         for (size_t n = 0; n < gs.members.size(); ++n) {
             if (!runs(gs.members[n])) continue;
@@ -1508,7 +1481,7 @@ static smac_status enqueue_batch_pass(smac_batch *b, bool time_band,
             lusgs_mid<double, 1>(lane_of(gs.members[n]), h->d, h->lws_sa);
         }
         B_TRY(join_lanes(b));
-        lusgs_band_multi<double, 1>(sm, gs.jobs, gs.map, gs.nblk, gs.pf, false, act);
+        lusgs_band_multi<double, 1>(sm, gs.jobs, gs.map, gs.nblk, false, act);
     }
     // SA after its sweeps; mean flow up to its band sweeps (line relaxation: the whole solve)
     B_TRY(fork_lanes(b));
@@ -1520,7 +1493,7 @@ static smac_status enqueue_batch_pass(smac_batch *b, bool time_band,
         const DevParams &dp = h->dp;
         if (has_sa(h) && is_lusgs(h)) {
             SaArrays &a = h->sa;
-            lusgs_post<double, 1>(ls, d, h->lws_sa, h->wake, a.anut, a.ds, a.sf, false);
+            lusgs_post<double, 1>(ls, d, h->lws_sa, h->wake, a.anut, a.ds, a.sf);
             launch_sa_update(ls, d, dp, h->w, h->st, a);
         }
         double *btc = h->blk[0], *bjm = h->blk[1], *bjp = h->blk[2], *bkm = h->blk[3],
@@ -1553,9 +1526,9 @@ static smac_status enqueue_batch_pass(smac_batch *b, bool time_band,
         const bool rec = time_band && g == b->band_group;
         if (rec) HIP_TRY(hipEventRecord(b->ev_band[0], sm));
         if (g == 0)
-            lusgs_band_multi<double, 3>(sm, gm.jobs, gm.map, gm.nblk, gm.pf, true, act);
+            lusgs_band_multi<double, 3>(sm, gm.jobs, gm.map, gm.nblk, true, act);
         else
-            lusgs_band_multi<float, 3>(sm, gm.jobs, gm.map, gm.nblk, gm.pf, true, act);
+            lusgs_band_multi<float, 3>(sm, gm.jobs, gm.map, gm.nblk, true, act);
         if (rec) HIP_TRY(hipEventRecord(b->ev_band[1], sm));
         B_TRY(fork_lanes(b));
         for (int i : gm.members) {
@@ -1567,9 +1540,9 @@ static smac_status enqueue_batch_pass(smac_batch *b, bool time_band,
         }
         B_TRY(join_lanes(b));
         if (g == 0)
-            lusgs_band_multi<double, 3>(sm, gm.jobs, gm.map, gm.nblk, gm.pf, false, act);
+            lusgs_band_multi<double, 3>(sm, gm.jobs, gm.map, gm.nblk, false, act);
         else
-            lusgs_band_multi<float, 3>(sm, gm.jobs, gm.map, gm.nblk, gm.pf, false, act);
+            lusgs_band_multi<float, 3>(sm, gm.jobs, gm.map, gm.nblk, false, act);
     }
     B_TRY(fork_lanes(b));
     for (int i = 0; i < nc; ++i) {
@@ -1579,9 +1552,9 @@ static smac_status enqueue_batch_pass(smac_batch *b, bool time_band,
         const Dims &d = h->d;
         if (is_lusgs(h)) {
             if (h->p.precision == SMAC_FP32_LHS)
-                lusgs_post<float, 3>(ls, d, h->lws, h->wake, h->q, h->dq, h->s, false);
+                lusgs_post<float, 3>(ls, d, h->lws, h->wake, h->q, h->dq, h->s);
             else
-                lusgs_post<double, 3>(ls, d, h->lws, h->wake, h->q, h->dq, h->s, false);
+                lusgs_post<double, 3>(ls, d, h->lws, h->wake, h->q, h->dq, h->s);
         }
         launch_update_force(ls, d, h->dp, h->walls, h->x, h->y, h->met, h->dj, h->q, h->dq,
                             h->w, h->st);
@@ -1908,20 +1881,16 @@ smac_status smac_lusgs(const smac_params *p, int jmax, int kmax, int neqs, int n
     smac_status rc = wake_to_device(b, jmax, kmax, npair, wake, w);
     if (rc) return rc;
     LusgsWs ws{};
-    lusgs_ws_shape(jmax, kmax, 64, ws);
-    ws.ring = 1;
-    if (!lusgs_ws_fits(ws)) return fail(SMAC_ERR_SIZE, "grid too large for the LU-SGS workspace");
-    const long lb = lusgs_ws_lhs_bytes(ws, neqs), vb = lusgs_ws_vec_bytes(ws, neqs);
+    lusgs_ws_shape(jmax, kmax, 64, neqs, ws);
+    if (!lusgs_size_ok(jmax, kmax, 64))
+        return fail(SMAC_ERR_SIZE, "grid too large for the LU-SGS workspace");
+    const long lb = lusgs_ws_lhs_bytes(ws, neqs);
     ws.lhs = b.get<char>(lb);
-    ws.r = b.get<char>(vb);
-    ws.dq = b.get<char>(vb);
     ws.edge = b.get<unsigned long long>(ws.nedge);
     ws.stall = b.get<int>(1);
-    if (!ws.lhs || !ws.r || !ws.dq || !ws.edge || !ws.stall) return fail(SMAC_ERR_HIP, "hipMalloc failed");
-    // padding positions are read by idle lanes and must hold finite values
+    if (!ws.lhs || !ws.edge || !ws.stall) return fail(SMAC_ERR_HIP, "hipMalloc failed");
+    // padding positions are read by lanes without a row and must hold finite values
     HIP_TRY(hipMemset(ws.lhs, 0, lb));
-    HIP_TRY(hipMemset(ws.r, 0, vb));
-    HIP_TRY(hipMemset(ws.dq, 0, vb));
     HIP_TRY(hipMemset(ws.edge, 0, ws.nedge * 8));
     HIP_TRY(hipMemset(ws.stall, 0, sizeof(int)));
     HIP_TRY(hipMemcpy(q_, q, neqs * N * 8, hipMemcpyHostToDevice));

@@ -88,16 +88,20 @@ extern "C" smac_status smac_lusgs_noalloc(const smac_params *p, int jmax, int km
     smac_status rc = scratch_of(dev, &base);
     if (rc) return rc;
 
+    if (!lusgs_size_ok(jmax, kmax, 64))
+        return smac_fail_text(SMAC_ERR_SIZE, "grid too large for the LU-SGS workspace");
+    // The grids taken are those for which this bound on the workspace fits the scratch array:
+    // 464 (56) bytes per position, the hand-over slots of 64-row bands, and slack.  What the
+    // chunks and slots below take is less for every size.
+    const long pos = lusgs_positions(jmax, kmax, 64);
+    const long epitch = (jmax + 256L) * 4, nedge64 = (2L * ((kmax + 63) / 64) + 1) * epitch;
+    const long need = align256(pos * (neqs == 3 ? 400 : 40) + 256) +
+                      2 * align256(pos * (neqs == 3 ? 32 : 8) + 256) +
+                      align256(nedge64 * 8 + 256) + 256;
     LusgsWs ws{};
-    lusgs_ws_shape(jmax, kmax, 64, ws);
-    ws.ring = 1;
-    if (!lusgs_ws_fits(ws)) return smac_fail_text(SMAC_ERR_SIZE, "grid too large for the LU-SGS workspace");
-    // workspace regions, each with the 256 bytes of slack the kernels' buffers are given
-    const long lb = align256(lusgs_ws_lhs_bytes(ws, neqs) + 256);
-    const long vb = align256(lusgs_ws_vec_bytes(ws, neqs) + 256);
-    const long eb = align256(ws.nedge * 8 + 256);
-    const long need = lb + 2 * vb + eb + 256;
-    if (need > (long)SMAC_NOALLOC_SCRATCH_BYTES)
+    lusgs_ws_shape(jmax, kmax, 64, neqs, ws);
+    const long lb = align256(lusgs_ws_lhs_bytes(ws, neqs) + 256), eb = align256(ws.nedge * 8 + 256);
+    if (need > (long)SMAC_NOALLOC_SCRATCH_BYTES || lb + eb + 256 > (long)SMAC_NOALLOC_SCRATCH_BYTES)
         return smac_fail_text(SMAC_ERR_SIZE,
                               ("the LU-SGS workspace of a " + std::to_string(jmax) + "x" +
                                std::to_string(kmax) + " grid needs " + std::to_string(need) +
@@ -105,13 +109,11 @@ extern "C" smac_status smac_lusgs_noalloc(const smac_params *p, int jmax, int km
                                std::to_string((long)SMAC_NOALLOC_SCRATCH_BYTES))
                                   .c_str());
     ws.lhs = base;
-    ws.r = base + lb;
-    ws.dq = base + lb + vb;
-    ws.edge = (unsigned long long *)(base + lb + 2 * vb);
-    ws.stall = stall ? stall : (int *)(base + lb + 2 * vb + eb);
+    ws.edge = (unsigned long long *)(base + lb);
+    ws.stall = stall ? stall : (int *)(base + lb + eb);
 
     const hipStream_t sm = (hipStream_t)stream;
-    const long n16 = (lb + 2 * vb + eb) / 16;
+    const long n16 = (lb + eb) / 16;
     hipLaunchKernelGGL(k_noalloc_init, dim3(1024), dim3(256), 0, sm, (uint4 *)base, n16, ws.stall);
     const Dims d{jmax, kmax, (long)jmax * kmax};
     WakePairs w{npair, wake, 1};

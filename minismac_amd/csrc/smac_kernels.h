@@ -84,23 +84,17 @@ void launch_lrelax_scan_t(hipStream_t, const Dims &, int njsp, int nksp, double 
                           const double *in, double *out, const LrScan &wt, const LrTWork &v);
 
 // lusgs.hip: LU-SGS with hyperplane (j+k = const) sweeps (ref/lusgs.f, ref/ilusol.f).
-// Workspace in the sheared layout: point (j,k) at (j+k+16)*ks + k of every plane, planes
-// stored in pairs for the 3x3 system.
+// Workspace by hyperplanes: the operands of a few rows of one hyperplane are one chunk.
 struct LusgsWs {
-    int rows;                    // rows per band (one wavefront each), 1..64
+    int rows;                    // rows per band: 1..16 (3x3 system), 1..64 (scalar)
     int nband;                   // bands covering k = 0..km-1
-    int ks;                      // pitch of one hyperplane
+    int ks;                      // rows of one hyperplane, padded to whole chunks
     int H;                       // last hyperplane, jm + km - 2
-    long ns;                     // positions per plane, (H+33)*ks
     int epitch;                  // slots per band region: (jm + 2*128 padding)*4
-    long nedge;                  // (2*nband + 1)*epitch slots
-    void *lhs;                   // 5 block groups (factors, bjm, bkm, bjp, bkp), LT
-    void *r;                     // neqs planes: rhs, forward result, middle result
-    void *dq;                    // neqs planes (the solve's type: FP64, or FP32 for FP32-LHS)
+    long nedge;                  // 2*nband*epitch slots
+    void *lhs;                   // the forward chunks, then the backward chunks
     unsigned long long *edge;    // band hand-over slots (forward half, backward half)
     int *stall;                  // raised when a hand-over wait times out
-    int pf3, pf1;                // prefetch distance (steps) of the 3x3 and scalar sweeps
-    int ring;                    // 1: the 3x3 sweeps stream their operands through LDS
     hipEvent_t ev_fwd[2];        // when set: recorded around the forward band sweep
 };
 // one case's part of a multi-case band launch
@@ -119,17 +113,28 @@ template <typename LT, int NEQ>
 void lusgs_band(hipStream_t, const Dims &, const LusgsWs &, bool fwd);
 // jobs and map in device memory; map[i] = (job, band in dispatch order), nblk entries
 template <typename LT, int NEQ>
-void lusgs_band_multi(hipStream_t, const BandJob *jobs, const int2 *map, int nblk, int pf,
-                      bool fwd, const int *active);
+void lusgs_band_multi(hipStream_t, const BandJob *jobs, const int2 *map, int nblk, bool fwd,
+                      const int *active);
 template <typename LT, int NEQ>
 void lusgs_mid(hipStream_t, const Dims &, const LusgsWs &);
 template <typename LT, int NEQ>
 void lusgs_post(hipStream_t, const Dims &, const LusgsWs &, const WakePairs &, const double *q,
-                double *dq, double *rhs, bool rhs_out);
-void lusgs_ws_shape(int jm, int km, int rows, LusgsWs &);
-long lusgs_ws_lhs_bytes(const LusgsWs &, int neqs);   // the five block groups
-long lusgs_ws_vec_bytes(const LusgsWs &, int neqs);   // one vector (rhs or dq)
-bool lusgs_ws_fits(const LusgsWs &);                  // 32-bit buffer offsets suffice
+                double *dq, double *rhs);
+void lusgs_ws_shape(int jm, int km, int rows, int neqs, LusgsWs &);
+long lusgs_ws_lhs_bytes(const LusgsWs &, int neqs);   // all chunks
+// The grid sizes the LU-SGS entry points take, by a measure of the grid that does not depend on
+// the layout: its positions (hyperplanes with 32 padding ones, rows padded to the bands as
+// `rows` cuts them).
+inline long lusgs_positions(int jm, int km, int rows)
+{
+    rows = rows < 1 ? 1 : (rows > 64 ? 64 : rows);
+    const int need = ((km + rows - 1) / rows - 1) * rows + 64;
+    return (long)(jm + km - 1 + 32) * (((need < km + 1 ? km + 1 : need) + 63) / 64 * 64);
+}
+inline bool lusgs_size_ok(int jm, int km, int rows)
+{
+    return lusgs_positions(jm, km, rows) * 80 < (1L << 31);
+}
 // fac (nullable) receives the diagonal factors in the natural layout (the reference's scr1);
 // rhs_out also returns the middle-step rhs in the natural layout, as the reference leaves it
 template <typename LT>
@@ -345,7 +350,6 @@ struct UnshearArgs {  // k_unshear
     unsigned gx, gy;
     Dims d;
     LusgsWs w;
-    const void *src;  // the solve's type
     double *dst;
 };
 
@@ -356,12 +360,12 @@ AsmArgs asm_args(const Dims &, const DevParams &, const double *q, const double 
 ResidPArgs residp_args(const Dims &, const double *s, const double *dj, Scratch &);
 ResidFArgs residf_args(const Dims &, int nt, double beta, const double *s, const double *dj,
                        Scratch &, DevStats *);
-template <typename LT>
+template <typename LT, int NEQ>
 ShearArgs shear_args(const Dims &, const LusgsWs &, const double *rhs, const LT *btc,
                      const LT *bjm, const LT *bjp, const LT *bkm, const LT *bkp, LT *fac);
 template <typename LT, int NEQ>
 MidArgs mid_args(const Dims &, const LusgsWs &);   // gx = 0: no launch (scaled FP32 form)
-UnshearArgs unshear_args(const Dims &, const LusgsWs &, const void *src, double *dst);
+UnshearArgs unshear_args(const Dims &, const LusgsWs &, double *dst);
 WakeArgs wake_args(const Dims &, int neqs, const WakePairs &, const double *sq, double *ds,
                    double *rhs);          // gx = 0 when there are no pairs
 UpdArgs upd_args(const Dims &, double *q, const double *dq, Scratch &);
