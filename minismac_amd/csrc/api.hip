@@ -345,7 +345,8 @@ smac_status smac_create(const smac_params *p, int jmax, int kmax, const double *
     if (p->impsch == 2) TRY(alloc_lusgs_ws(h, h->lusgs_rows));
     if (p->impsch == 1) {
         char *lb = nullptr;
-        TRY(dalloc(h, &lb, (size_t)lr_scan_bytes(h->d)));
+        const long scan = lr_scan_bytes(h->d), ref = lr_ref_bytes(h->d);
+        TRY(dalloc(h, &lb, (size_t)(scan > ref ? scan : ref)));   // one form runs at a time
         h->lrs.opx = lb;
         h->lrs.ope = lb + 45 * N * 8 + 256;
         h->lrs.s_t = (double *)(lb + 2 * (45 * N * 8 + 256));
@@ -533,8 +534,8 @@ static void enqueue_lrelax(smac_handle *h, hipStream_t sm)
                         h->nt - h->lr_factored >= h->lr_refactor;
     h->lr_factored = !h->lr_solve ? -1 : (factor ? h->nt : h->lr_factored);
     if (!h->lr_solve)
-        launch_lrelax_ref<double>(sm, d, h->dp, h->p.njsp, h->p.nksp, h->p.nbcimp, h->wake, h->q,
-                                  h->dq, h->s, btc, bjm, bjp, bkm, bkp, h->lr_lines);
+        launch_lrelax_ref(sm, d, h->dp, h->p.njsp, h->p.nksp, h->p.nbcimp, h->wake, h->q, h->dq,
+                          h->s, btc, bjm, bjp, bkm, bkp, h->lrs.opx, h->lr_lines);
     else if (h->p.precision == SMAC_FP32_LHS)
         launch_lrelax_scan<float>(sm, d, h->dp, h->p.njsp, h->p.nksp, h->p.nbcimp, zebra, h->wake,
                                   h->q, h->dq, h->s, (const float *)btc, (const float *)bjm,
@@ -1827,7 +1828,8 @@ smac_status smac_lrelax(const smac_params *p, int jmax, int kmax, int npair, con
     double *bl[5];
     const double *hb[5] = {btc, bjm, bjp, bkm, bkp};
     for (int i = 0; i < 5; ++i) bl[i] = b.get<double>(9 * N);
-    if (!dq_ || !s_ || !q_ || !bl[0] || !bl[1] || !bl[2] || !bl[3] || !bl[4])
+    char *pack = b.get<char>(lr_ref_bytes(d));
+    if (!dq_ || !s_ || !q_ || !bl[0] || !bl[1] || !bl[2] || !bl[3] || !bl[4] || !pack)
         return fail(SMAC_ERR_HIP, "hipMalloc failed");
     WakePairs w;
     rc = wake_to_device(b, jmax, kmax, npair, wake, w);
@@ -1835,8 +1837,8 @@ smac_status smac_lrelax(const smac_params *p, int jmax, int kmax, int npair, con
     HIP_TRY(hipMemcpy(q_, q, 3 * N * 8, hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(s_, s, 3 * N * 8, hipMemcpyHostToDevice));
     for (int i = 0; i < 5; ++i) HIP_TRY(hipMemcpy(bl[i], hb[i], 9 * N * 8, hipMemcpyHostToDevice));
-    launch_lrelax_ref<double>(0, d, dp, p->njsp, p->nksp, p->nbcimp, w, q_, dq_, s_, bl[0], bl[1],
-                              bl[2], bl[3], bl[4]);
+    launch_lrelax_ref(0, d, dp, p->njsp, p->nksp, p->nbcimp, w, q_, dq_, s_, bl[0], bl[1], bl[2],
+                      bl[3], bl[4], pack);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipDeviceSynchronize());
     HIP_TRY(hipMemcpy(dq, dq_, 3 * N * 8, hipMemcpyDeviceToHost));

@@ -5,12 +5,13 @@
 //
 // Reference order ("parity mode"): the xi sweep visits k-lines in Gauss-Seidel order
 // (line k reads dq of line k-1 from the same sweep), so lines are strictly sequential.  One
-// workgroup walks the lines: its threads build the line's right-hand side in LDS in
-// parallel, one lane runs the block forward/back substitution with the factored blocks,
-// and the threads apply the under-relaxed update.  The factorisations are independent per
-// line: one thread per line, eta lines coalesced along j.
+// workgroup walks the lines: one wavefront runs the block forward/back substitution with the
+// factored blocks, the others form the updates and the next line's right-hand side behind it.
+// The factorisations are independent per line: one lane per line.
 #include "smac_dev.h"
 #include "smac_kernels.h"
+
+#include <type_traits>
 
 namespace smac {
 
@@ -110,222 +111,375 @@ SMAC_DEV void st9(LT *__restrict__ a, long N, long p, const LT r[9])
 }
 
 // ------------------------------------------------------------------------------------------
-// factorisation along lines: btlu3j (lines of constant k, walking j) and btlu3k.
-// `stride` is the point step along the line, `lstride` the step between lines.
+// the factored lines, packed: block b of line l (its points 16b .. 16b+15, q = point in the
+// block, c = equation) is one chunk of 4096 bytes, as the chain of a sweep reads it:
+//   [q][c][16 B]  (a_c0 a_c1), (a_c2 f8)       lower band of equation c
+//   [q][16 B]     (f0 f1) (f2 f3) (f4 f5) (f6 f7)   factored diagonal
+//   [q][c][16 B]  (C_c0 C_c1), (C_c2 -)        factored upper band
+// a is zero at a line's first point and C at its last, whose terms the reference does not form
+// (they meet a zero there); past the line's end everything is zero.
 
+typedef double v2d __attribute__((ext_vector_type(2)));
+constexpr int RB = 16, RCHUNK = 4096;
+constexpr int RA0 = 0, RA1 = 768, RD = 1536, RC0 = 2560, RC1 = 3328;
+
+SMAC_DEV int ref_blocks(int len) { return (len + RB - 1) / RB; }
+SMAC_DEV char *ref_point(char *pk, int len, int l, int i)   // + q*48 or q*16 by the caller
+{
+    return pk + ((long)l * ref_blocks(len) + i / RB) * RCHUNK;
+}
+
+long lr_ref_bytes(const Dims &d)
+{
+    const long xi = (long)d.km * ((d.jm + RB - 1) / RB), eta = (long)d.jm * ((d.km + RB - 1) / RB);
+    return (xi > eta ? xi : eta) * RCHUNK;
+}
+
+// factorisation along lines: btlu3j (lines of constant k, walking j) and btlu3k, one lane per
+// line, into the packed chunks.  `stride` is the point step along the line, `lstride` the step
+// between lines.  A point's recurrence takes about 0.4 us (three dependent divisions); its 27
+// values are loaded PF points ahead, since a load on the chain would cost three times that
+// (119x31, xi lines: 190 us without, 103 us with and a line per wave).
 template <typename LT>
 __global__ void __launch_bounds__(64) k_btlu3(long N, int nline, int len, long stride,
                                              long lstride, const LT *__restrict__ a,
-                                             LT *__restrict__ b, LT *__restrict__ c)
+                                             const LT *__restrict__ b, const LT *__restrict__ c,
+                                             char *__restrict__ pk)
 {
+    constexpr int PF = 4;
     const int l = blockIdx.x * blockDim.x + threadIdx.x;
     if (l >= nline) return;
-    LT cp[9];
-    for (int i = 0; i < len; ++i) {
-        const long p = lstride * l + stride * i;
-        LT bb[9];
-        ld9(b, N, p, bb);
-        if (i > 0) {
-            LT aa[9];
-            ld9(a, N, p, aa);
-            bminus3(bb, aa, cp);
-        }
-        lu3(bb);
-        if (i < len - 1) {
-            LT cc[9];
-            ld9(c, N, p, cc);
-            csolve3(bb, cc);
-            st9(c, N, p, cc);
+    LT la[PF][9], lb[PF][9], lc[PF][9];
+    auto load = [&](int u, int i) {
+        const long p = lstride * l + stride * (i < len ? i : len - 1);
+        ld9(b, N, p, lb[u]);
+        ld9(a, N, p, la[u]);
+        ld9(c, N, p, lc[u]);
+    };
 #pragma unroll
-            for (int e = 0; e < 9; ++e) cp[e] = cc[e];
+    for (int u = 0; u < PF; ++u) load(u, u);
+    LT cp[9];
+#pragma unroll
+    for (int e = 0; e < 9; ++e) cp[e] = (LT)0;
+    auto put = [&](int i, const LT *aa, const LT *bb, const LT *cc) {
+        const int q = i % RB;
+        char *ch = ref_point(pk, len, l, i);
+#pragma unroll
+        for (int m = 0; m < 3; ++m) {
+            char *lane = ch + q * 48 + m * 16;
+            *(v2d *)(lane + RA0) = v2d{aa[m], aa[m + 3]};
+            *(v2d *)(lane + RA1) = v2d{aa[m + 6], bb[8]};
+            *(v2d *)(lane + RC0) = v2d{cc[m], cc[m + 3]};
+            *(v2d *)(lane + RC1) = v2d{cc[m + 6], 0.};
         }
-        st9(b, N, p, bb);
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+            *(v2d *)(ch + RD + g * 256 + q * 16) = v2d{bb[2 * g], bb[2 * g + 1]};
+    };
+    for (int i0 = 0; i0 < len; i0 += PF) {
+#pragma unroll
+        for (int u = 0; u < PF; ++u) {
+            const int i = i0 + u;
+            if (i >= len) break;
+            if (i > 0) {
+                bminus3(lb[u], la[u], cp);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 9; ++e) la[u][e] = (LT)0;
+            }
+            lu3(lb[u]);
+            csolve3(lb[u], lc[u]);
+            if (i == len - 1) {
+#pragma unroll
+                for (int e = 0; e < 9; ++e) lc[u][e] = (LT)0;
+            }
+#pragma unroll
+            for (int e = 0; e < 9; ++e) cp[e] = lc[u][e];
+            put(i, la[u], lb[u], lc[u]);
+            load(u, i + PF);
+        }
     }
+#pragma unroll
+    for (int e = 0; e < 9; ++e) cp[e] = (LT)0;
+    for (int i = len; i < ref_blocks(len) * RB; ++i) put(i, cp, cp, cp);
 }
 
-// btund3j: recompose btc and bjp from their xi factors (ref/btlu3.f:628-838), walking each
-// line backwards so that c(i-1) is still factored when b(i) reads it
+// btund3j: recompose btc and bjp from their xi factors (ref/btlu3.f:628-838), one point per
+// thread (the factors are in the chunks, so a point does not wait for its neighbours)
 template <typename LT>
-__global__ void __launch_bounds__(64) k_btund3(long N, int nline, int len, long stride,
-                                              long lstride, const LT *__restrict__ a,
-                                              LT *__restrict__ b, LT *__restrict__ c)
+__global__ void __launch_bounds__(256) k_btund3(long N, int len, const LT *__restrict__ a,
+                                               LT *__restrict__ b, LT *__restrict__ c,
+                                               const char *__restrict__ pk)
 {
-    const int l = blockIdx.x * blockDim.x + threadIdx.x;
-    if (l >= nline) return;
-    for (int i = len - 1; i >= 0; --i) {
-        const long p = lstride * l + stride * i;
-        LT bb[9];
-        ld9(b, N, p, bb);
-        unlu3(bb);
-        if (i < len - 1) {
-            LT cc[9];
-            ld9(c, N, p, cc);
-            ctimes3(bb, cc);
-            st9(c, N, p, cc);
+    const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= N) return;
+    const int l = (int)(p / len), i = (int)(p % len);
+    auto band = [&](int ii, LT o[9]) {   // C of point ii
+        const char *ch = ref_point((char *)pk, len, l, ii) + ii % RB * 48;
+#pragma unroll
+        for (int m = 0; m < 3; ++m) {
+            const v2d t = *(const v2d *)(ch + m * 16 + RC0);
+            o[m] = t.x;
+            o[m + 3] = t.y;
+            o[m + 6] = *(const double *)(ch + m * 16 + RC1);
         }
-        if (i > 0) {
-            LT aa[9], cp[9];
-            ld9(a, N, p, aa);
-            ld9(c, N, p - stride, cp);
-            bplus3(bb, aa, cp);
+    };
+    LT bb[9];
+    {
+        const char *ch = ref_point((char *)pk, len, l, i);
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const v2d t = *(const v2d *)(ch + RD + g * 256 + i % RB * 16);
+            bb[2 * g] = t.x;
+            bb[2 * g + 1] = t.y;
         }
-        st9(b, N, p, bb);
+        bb[8] = ((const double *)(ch + i % RB * 48 + RA1))[1];
     }
+    unlu3(bb);
+    if (i < len - 1) {
+        LT cc[9];
+        band(i, cc);
+        ctimes3(bb, cc);
+        st9(c, N, p, cc);
+    }
+    if (i > 0) {
+        LT aa[9], cp[9];
+        ld9(a, N, p, aa);
+        band(i - 1, cp);
+        bplus3(bb, aa, cp);
+    }
+    st9(b, N, p, bb);
 }
 
 // ------------------------------------------------------------------------------------------
-// one sweep in reference line order (ljsweep / lksweep).  Lines run one after another in one
-// workgroup; `dir` chooses xi lines (lines of constant k) or eta lines (constant j).
+// one sweep in reference line order (ljsweep / lksweep): lines one after another in one
+// workgroup; `eta` chooses xi lines (lines of constant k) or eta lines (constant j).
+//
+// Wave 0 is the chain: forward substitution along the line, then back.  Lane 4q + c holds
+// equation c of point q of a block of 16 points (c = 3 repeats c = 2), so a block's operands
+// are six loads for the wave; the points are then solved one after another by all lanes, the
+// one whose turn it is for good, and its result goes to the next through scalar registers
+// (v_readlane).  A forward step is 21 FP64 operations (33 where one lane does all three
+// equations), a backward one 6, with no LDS access or load in either.
+// Waves 1..SW take segments of 64 points: as soon as the chain has passed a segment on its way
+// back, they form the under-relaxed update there and the next line's right-hand side, whose
+// operands they loaded while the chain was running.  The waves meet in LDS counters, each wait
+// for a wave that does not wait back: the chain for a segment's right-hand side of its line,
+// a segment for the chain's blocks of the line before.
+//
+// What bounds it: the chain, two dependent block steps per point, line after line: about 65 ns
+// each (21 and 6 FP64 operations and the passing on, at the 5 cycles a lone wavefront takes per
+// instruction).  At 119x31 a sweep takes 480 us; with one lane solving all three equations out
+// of LDS, and every line's operands staged and its right-hand side formed between the chains,
+// it took 1050 us (xi) and 1380 us (eta).
+constexpr int SW = 7;
 
-constexpr int SWEEP_THREADS = 256;
-constexpr int SWEEP_CHUNK = 256;   // points of the band staged per chunk (two chunks in LDS)
-
-template <typename LT>
-__global__ void __launch_bounds__(SWEEP_THREADS)
+__global__ void __launch_bounds__(64 * (SW + 1))
 k_sweep_ref(Dims d, int eta, int nsweep, double underr, double *__restrict__ dq,
-            const double *__restrict__ s, const LT *__restrict__ btc, const LT *__restrict__ lm,
-            const LT *__restrict__ lp, const LT *__restrict__ om, const LT *__restrict__ op)
+            const double *__restrict__ s, const char *__restrict__ pk,
+            const double *__restrict__ om, const double *__restrict__ op)
 {
-    // lm/lp: blocks along the line (bjm/bjp for xi, bkm/bkp for eta);
     // om/op: blocks to the neighbouring lines (bkm/bkp for xi, bjm/bjp for eta)
-    extern __shared__ double lds[];   // 3 * len rhs, then two chunks of 18 band planes
-    double *rhs = lds, *band = lds + 3 * (eta ? d.km : d.jm);
+    extern __shared__ double line[];   // per point 3: right-hand side, then y, then x
     const long N = d.N;
     const int nline = eta ? d.jm : d.km;
     const int len = eta ? d.km : d.jm;
     const long stride = eta ? d.jm : 1;          // along a line
     const long lstride = eta ? 1 : d.jm;         // between lines
     const bool rev = (nsweep / 2) * 2 == nsweep;
-    const double half = 0.5;
-    for (int ll = 0; ll < nline; ++ll) {
-        const int l = rev ? nline - 1 - ll : ll;
-        const int lmn = l - 1 > 0 ? l - 1 : 0;
-        const int lpl = l + 1 < nline - 1 ? l + 1 : nline - 1;
-        const double rkm = (double)(float)(l - lmn - 1);
-        const double rkp = (double)(float)(lpl - l - 1);
-        const double swm = half + copysign(half, rkm);
-        const double swp = half + copysign(half, rkp);
-        for (int i = threadIdx.x; i < len; i += SWEEP_THREADS) {
-            const long p = lstride * l + stride * i;
-            const long pm = lstride * lmn + stride * i, pp = lstride * lpl + stride * i;
-            double x1 = dq[pm], x2 = dq[N + pm], x3 = dq[2 * N + pm];
-            double y1 = dq[pp], y2 = dq[N + pp], y3 = dq[2 * N + pp];
-#pragma unroll
-            for (int m = 0; m < 3; ++m) {
-                double bm = (double)om[m * N + p] * x1 + (double)om[(m + 3) * N + p] * x2 +
-                            (double)om[(m + 6) * N + p] * x3;
-                double bp = (double)op[m * N + p] * y1 + (double)op[(m + 3) * N + p] * y2 +
-                            (double)op[(m + 6) * N + p] * y3;
-                rhs[3 * i + m] = s[m * N + p] - bm * swm - bp * swp;
+    const int nblk = ref_blocks(len), nseg = (len + 63) / 64;
+    int *back = (int *)(line + 3 * nblk * RB);   // backward blocks done, over all lines
+    int *ready = back + 1;                       // per segment: lines whose right-hand side is there
+    auto ld = [](const int *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); };
+    auto st = [](int *p, int v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); };
+    for (int i = 3 * len + threadIdx.x; i < 3 * nblk * RB; i += 64 * (SW + 1)) line[i] = 0.;
+    for (int i = threadIdx.x; i < 1 + nseg; i += 64 * (SW + 1)) back[i] = 0;
+    __syncthreads();
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    auto line_of = [&](int ll) { return rev ? nline - 1 - ll : ll; };
+
+    if (wave > 0) {
+        const double half = 0.5;
+        // the right-hand side of line l at point i, with dq of the line solved before it (lnew,
+        // -1: none) in xn
+        for (int ll = -1; ll < nline; ++ll) {
+            const int l = ll < 0 ? -1 : line_of(ll), ln = ll + 1 < nline ? line_of(ll + 1) : -1;
+            const int lmn = ln - 1 > 0 ? ln - 1 : 0;
+            const int lpl = ln + 1 < nline - 1 ? ln + 1 : nline - 1;
+            const double rkm = (double)(float)(ln - lmn - 1);
+            const double rkp = (double)(float)(lpl - ln - 1);
+            const double swm = half + copysign(half, rkm);
+            const double swp = half + copysign(half, rkp);
+            // bring the chunks of the line after next closer (the chain loads them from L2)
+            int warm = 0;
+            if (ll + 2 < nline) {
+                const char *w = pk + (long)line_of(ll + 2) * nblk * RCHUNK;
+                for (int o = ((wave - 1) * 64 + lane) * 128; o < nblk * RCHUNK; o += SW * 64 * 128)
+                    warm ^= *(const int *)(w + o);
             }
-        }
-        __syncthreads();
-        // The solve along the line is one dependent chain, run by thread 0 from LDS: the
-        // band is staged in chunks of SWEEP_CHUNK points (the reference copies it to /btri/,
-        // ref/lrelax.f:310-321), the next chunk loaded by waves 1.. while thread 0 works
-        // through the current one.
-        // forward with the factored diagonal blocks and the lower band (ref/lrelax.f:331-351)
-        {
-            const int nch = (len + SWEEP_CHUNK - 1) / SWEEP_CHUNK;
-            auto stage = [&](int c, double *buf) {
-                for (int ii = (int)threadIdx.x - 64; ii < SWEEP_CHUNK; ii += SWEEP_THREADS - 64) {
-                    if (ii < 0) continue;
-                    const int i = c * SWEEP_CHUNK + ii;
-                    if (i >= len) break;
-                    const long p = lstride * l + stride * i;
+            for (int sg = nseg - 1 - ((nseg - wave) % SW + SW) % SW; sg >= 0; sg -= SW) {
+                const int i = sg * 64 + lane;
+                const bool in = i < len;
+                const long po = stride * (in ? i : 0);
+                double dl[3], sn[3], x[3], y[3], bo[9], bp[9];
+                if (l >= 0) {
 #pragma unroll
-                    for (int e = 0; e < 9; ++e) {
-                        buf[e * SWEEP_CHUNK + ii] = (double)lm[e * N + p];
-                        buf[(9 + e) * SWEEP_CHUNK + ii] = (double)btc[e * N + p];
-                    }
+                    for (int n = 0; n < 3; ++n) dl[n] = dq[n * N + lstride * l + po];
                 }
-            };
-            if (threadIdx.x >= 64) stage(0, band);
-            __syncthreads();
-            double r1 = 0, r2 = 0, r3 = 0;
-            for (int c = 0; c < nch; ++c) {
-                double *cur = band + (c & 1) * 18 * SWEEP_CHUNK;
-                if (threadIdx.x >= 64) {
-                    if (c + 1 < nch) stage(c + 1, band + ((c + 1) & 1) * 18 * SWEEP_CHUNK);
-                } else if (threadIdx.x == 0) {
-                    const int i1 = (c + 1) * SWEEP_CHUNK < len ? (c + 1) * SWEEP_CHUNK : len;
-#pragma unroll 4
-                    for (int i = c * SWEEP_CHUNK; i < i1; ++i) {
-                        const int ii = i - c * SWEEP_CHUNK;
-                        double t1 = rhs[3 * i], t2 = rhs[3 * i + 1], t3 = rhs[3 * i + 2];
-                        if (i > 0) {
-                            const double *a = cur + ii;
-                            t1 = t1 - a[0] * r1 - a[3 * SWEEP_CHUNK] * r2 - a[6 * SWEEP_CHUNK] * r3;
-                            t2 = t2 - a[1 * SWEEP_CHUNK] * r1 - a[4 * SWEEP_CHUNK] * r2 -
-                                 a[7 * SWEEP_CHUNK] * r3;
-                            t3 = t3 - a[2 * SWEEP_CHUNK] * r1 - a[5 * SWEEP_CHUNK] * r2 -
-                                 a[8 * SWEEP_CHUNK] * r3;
+                if (ln >= 0) {
+                    const long p = lstride * ln + po;
+#pragma unroll
+                    for (int n = 0; n < 3; ++n) {
+                        sn[n] = s[n * N + p];
+                        x[n] = lmn == l ? 0. : dq[n * N + lstride * lmn + po];
+                        y[n] = lpl == l ? 0. : dq[n * N + lstride * lpl + po];
+                    }
+                    ld9(om, N, p, bo);
+                    ld9(op, N, p, bp);
+                }
+                if (l >= 0) {
+                    const int need = ll * nblk + nblk - 4 * sg;
+                    while (ld(back) < need) __builtin_amdgcn_s_sleep(1);
+                    asm volatile("" ::: "memory");
+                    if (in) {
+#pragma unroll
+                        for (int n = 0; n < 3; ++n) {
+                            const double v = dl[n] + underr * (line[3 * i + n] - dl[n]);
+                            dq[n * N + lstride * l + po] = v;
+                            x[n] = lmn == l ? v : x[n];
+                            y[n] = lpl == l ? v : y[n];
                         }
-                        const double *bb = cur + 9 * SWEEP_CHUNK + ii;
-                        double b0 = bb[0], b1 = bb[SWEEP_CHUNK], b2 = bb[2 * SWEEP_CHUNK],
-                               b3 = bb[3 * SWEEP_CHUNK], b4 = bb[4 * SWEEP_CHUNK],
-                               b5 = bb[5 * SWEEP_CHUNK], b6 = bb[6 * SWEEP_CHUNK],
-                               b7 = bb[7 * SWEEP_CHUNK], b8 = bb[8 * SWEEP_CHUNK];
-                        double d1 = b0 * t1;
-                        double d2 = b4 * (t2 - b1 * d1);
-                        double d3 = b8 * (t3 - b2 * d1 - b5 * d2);
-                        r3 = d3;
-                        r2 = d2 - b7 * r3;
-                        r1 = d1 - b6 * r3 - b3 * r2;
-                        rhs[3 * i] = r1;
-                        rhs[3 * i + 1] = r2;
-                        rhs[3 * i + 2] = r3;
                     }
                 }
-                __syncthreads();
-            }
-            // back substitution with the upper band (ref/lrelax.f:367-373), chunks from the end
-            auto stage_c = [&](int c, double *buf) {
-                for (int ii = (int)threadIdx.x - 64; ii < SWEEP_CHUNK; ii += SWEEP_THREADS - 64) {
-                    if (ii < 0) continue;
-                    const int i = c * SWEEP_CHUNK + ii;
-                    if (i > len - 2) break;
-                    const long p = lstride * l + stride * i;
+                if (ln >= 0) {
+                    if (in) {
 #pragma unroll
-                    for (int e = 0; e < 9; ++e) buf[e * SWEEP_CHUNK + ii] = (double)lp[e * N + p];
-                }
-            };
-            const int nb = len >= 2 ? (len - 2) / SWEEP_CHUNK + 1 : 0;   // chunks holding 0..len-2
-            if (nb > 0 && threadIdx.x >= 64) stage_c(nb - 1, band);
-            __syncthreads();
-            for (int q = 0; q < nb; ++q) {
-                const int c = nb - 1 - q;
-                double *cur = band + (q & 1) * 18 * SWEEP_CHUNK;
-                if (threadIdx.x >= 64) {
-                    if (c > 0) stage_c(c - 1, band + ((q + 1) & 1) * 18 * SWEEP_CHUNK);
-                } else if (threadIdx.x == 0) {
-                    const int ihi = (c + 1) * SWEEP_CHUNK - 1 < len - 2 ? (c + 1) * SWEEP_CHUNK - 1
-                                                                      : len - 2;
-#pragma unroll 4
-                    for (int i = ihi; i >= c * SWEEP_CHUNK; --i) {
-                        const double *cc = cur + (i - c * SWEEP_CHUNK);
-                        double t1 = rhs[3 * i] - cc[0] * r1 - cc[3 * SWEEP_CHUNK] * r2 -
-                                    cc[6 * SWEEP_CHUNK] * r3;
-                        double t2 = rhs[3 * i + 1] - cc[1 * SWEEP_CHUNK] * r1 -
-                                    cc[4 * SWEEP_CHUNK] * r2 - cc[7 * SWEEP_CHUNK] * r3;
-                        double t3 = rhs[3 * i + 2] - cc[2 * SWEEP_CHUNK] * r1 -
-                                    cc[5 * SWEEP_CHUNK] * r2 - cc[8 * SWEEP_CHUNK] * r3;
-                        r1 = t1; r2 = t2; r3 = t3;
-                        rhs[3 * i] = r1;
-                        rhs[3 * i + 1] = r2;
-                        rhs[3 * i + 2] = r3;
+                        for (int m = 0; m < 3; ++m) {
+                            double bm = bo[m] * x[0] + bo[m + 3] * x[1] + bo[m + 6] * x[2];
+                            double bq = bp[m] * y[0] + bp[m + 3] * y[1] + bp[m + 6] * y[2];
+                            line[3 * i + m] = sn[m] - bm * swm - bq * swp;
+                        }
                     }
+                    asm volatile("" ::: "memory");
+                    st(&ready[sg], ll + 2);
                 }
-                __syncthreads();
             }
+            asm volatile("" : : "v"(warm));
         }
-        for (int i = threadIdx.x; i < len; i += SWEEP_THREADS) {
-            const long p = lstride * l + stride * i;
+        return;
+    }
+
+    // ---- the chain
+    const int q = lane >> 2, c = (lane & 3) < 2 ? lane & 3 : 2;
+    const int o3 = q * 48 + c * 16, o1 = q * 16;
+    struct Fwd { v2d a0, a1, f[4]; } F[2];
+    struct Bck { v2d c0; double c2; } B[3];
+    auto ldf = [&](Fwd &t, const char *ch) {
+        t.a0 = *(const v2d *)(ch + RA0 + o3);
+        t.a1 = *(const v2d *)(ch + RA1 + o3);
 #pragma unroll
-            for (int m = 0; m < 3; ++m)
-                dq[m * N + p] = dq[m * N + p] + underr * (rhs[3 * i + m] - dq[m * N + p]);
+        for (int g = 0; g < 4; ++g) t.f[g] = *(const v2d *)(ch + RD + g * 256 + o1);
+    };
+    auto ldb = [&](Bck &t, const char *ch) {
+        t.c0 = *(const v2d *)(ch + RC0 + o3);
+        t.c2 = *(const double *)(ch + RC1 + o3);
+    };
+    auto chunk = [&](int l, int b) {
+        b = b < 0 ? 0 : (b < nblk ? b : nblk - 1);
+        return pk + ((long)l * nblk + b) * RCHUNK;
+    };
+    auto quad_value = [](double v, auto C) {   // v of lane C of the quad
+        const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+        constexpr int ctrl = decltype(C)::value * 0x55;
+        const int lo = __builtin_amdgcn_mov_dpp((int)(unsigned)u, ctrl, 0xf, 0xf, false);
+        const int hi = __builtin_amdgcn_mov_dpp((int)(unsigned)(u >> 32), ctrl, 0xf, 0xf, false);
+        return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) |
+                                                (unsigned long long)(unsigned)lo));
+    };
+    auto lane_value = [](double v, int from) {
+        const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+        const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)u, from);
+        const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(u >> 32), from);
+        return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+    };
+    ldf(F[0], chunk(line_of(0), 0));
+    ldf(F[1], chunk(line_of(0), 1));
+    for (int ll = 0; ll < nline; ++ll) {
+        const int l = line_of(ll);
+#pragma unroll
+        for (int u = 0; u < 3; ++u) ldb(B[u], chunk(l, nblk - 1 - u));
+        // forward with the factored diagonal blocks and the lower band (ref/lrelax.f:331-351)
+        double r1 = 0., r2 = 0., r3 = 0.;   // the point before, in every lane
+        auto forward = [&](const Fwd &t, int b) {
+            if (b % 4 == 0) {
+                while (ld(&ready[b / 4]) < ll + 1) {}
+                asm volatile("" ::: "memory");
+            }
+            double *slot = line + 3 * (b * RB + q) + c;
+            const double rhs = *slot;
+            const double b0 = t.f[0].x, b1 = t.f[0].y, b2 = t.f[1].x, b3 = t.f[1].y, b4 = t.f[2].x,
+                         b5 = t.f[2].y, b6 = t.f[3].x, b7 = t.f[3].y, b8 = t.a1.y;
+            double y1 = 0., y2 = 0., y3 = 0.;   // this lane's point, once its turn has come
+#pragma unroll
+            for (int g = 0; g < RB; ++g) {
+                const double tt = rhs - t.a0.x * r1 - t.a0.y * r2 - t.a1.x * r3;
+                const double t1 = quad_value(tt, std::integral_constant<int, 0>{}),
+                             t2 = quad_value(tt, std::integral_constant<int, 1>{}),
+                             t3 = quad_value(tt, std::integral_constant<int, 2>{});
+                if (q == g) {
+                    const double d1 = b0 * t1;
+                    const double d2 = b4 * (t2 - b1 * d1);
+                    const double d3 = b8 * (t3 - b2 * d1 - b5 * d2);
+                    y3 = d3;
+                    y2 = d2 - b7 * y3;
+                    y1 = d1 - b6 * y3 - b3 * y2;
+                }
+                r1 = lane_value(y1, 4 * g);
+                r2 = lane_value(y2, 4 * g);
+                r3 = lane_value(y3, 4 * g);
+            }
+            *slot = c == 0 ? y1 : c == 1 ? y2 : y3;
+        };
+        for (int b = 0;;) {
+            forward(F[0], b);
+            if (++b == nblk) break;
+            ldf(F[0], chunk(l, b + 1));
+            forward(F[1], b);
+            if (++b == nblk) break;
+            ldf(F[1], chunk(l, b + 1));
         }
-        __syncthreads();
+        if (ll + 1 < nline) {
+            ldf(F[0], chunk(line_of(ll + 1), 0));
+            ldf(F[1], chunk(line_of(ll + 1), 1));
+        }
+        // back substitution with the upper band (ref/lrelax.f:367-373)
+        double x1 = 0., x2 = 0., x3 = 0.;   // the point after, in every lane
+        auto backward = [&](const Bck &t, int b) {
+            double *slot = line + 3 * (b * RB + q) + c;
+            double v = *slot;
+#pragma unroll
+            for (int g = RB - 1; g >= 0; --g) {
+                const double tt = v - t.c0.x * x1 - t.c0.y * x2 - t.c2 * x3;
+                v = q == g ? tt : v;
+                x1 = lane_value(tt, 4 * g);
+                x2 = lane_value(tt, 4 * g + 1);
+                x3 = lane_value(tt, 4 * g + 2);
+            }
+            *slot = v;
+            asm volatile("" ::: "memory");
+            st(back, ll * nblk + nblk - b);
+        };
+        for (int b = nblk - 1;;) {
+            backward(B[0], b);
+            if (--b < 0) break;
+            ldb(B[0], chunk(l, b - 2));
+            backward(B[1], b);
+            if (--b < 0) break;
+            ldb(B[1], chunk(l, b - 2));
+            backward(B[2], b);
+            if (--b < 0) break;
+            ldb(B[2], chunk(l, b - 2));
+        }
     }
 }
 
@@ -392,41 +546,43 @@ void launch_wake(hipStream_t sm, const Dims &d, int neqs, const WakePairs &w, co
                        w.base, w.pairs, sq, ds, rhs);
 }
 
-template <typename LT>
 void launch_lrelax_ref(hipStream_t sm, const Dims &d, const DevParams &prm, int njsp, int nksp,
                        int nbcimp, const WakePairs &w, const double *q, double *dq, double *s,
-                       LT *btc, LT *bjm, LT *bjp, LT *bkm, LT *bkp, int lpb)
+                       double *btc, const double *bjm, double *bjp, const double *bkm,
+                       const double *bkp, void *pack, int lpb)
 {
     const long N = d.N;
-    // lines per workgroup of the factor kernels (one lane per line)
-    lpb = lpb < 1 ? 1 : (lpb > 64 ? 64 : lpb);
+    char *pk = (char *)pack;
+    // lines per workgroup of the factor kernels (one lane per line): as few as leave a wave per
+    // SIMD, at most lpb -- the lanes of a wave load from as many cache lines (31 lines of 119
+    // points: 160 us in one wave, 103 us in 31)
+    auto groups = [&](int nline) {
+        const int few = (nline + 1023) / 1024, n = lpb < 1 ? 1 : (lpb < few ? lpb : few);
+        return dim3((unsigned)((nline + n - 1) / n));
+    };
+    auto lines = [&](int nline) {
+        const int few = (nline + 1023) / 1024;
+        return dim3((unsigned)(lpb < 1 ? 1 : (lpb < few ? lpb : few)));
+    };
+    auto sweep = [&](int eta, int ns, const double *om, const double *op) {
+        const int len = eta ? d.km : d.jm;
+        const size_t lds = sizeof(double) * 3 * ((len + RB - 1) / RB * RB) + 4 * (1 + (len + 63) / 64);
+        hipLaunchKernelGGL(k_sweep_ref, dim3(1), dim3(64 * (SW + 1)), lds, sm, d, eta, ns, prm.underr,
+                           dq, s, pk, om, op);
+        if ((ns / nbcimp) * nbcimp == ns) launch_wake(sm, d, 3, w, q, dq, s);
+    };
     hipLaunchKernelGGL(k_fill, dim3(256), dim3(256), 0, sm, dq, 3 * N, 0.0);
     if (njsp > 0)
-        hipLaunchKernelGGL(k_btlu3<LT>, dim3((d.km + lpb - 1) / lpb), dim3(lpb), 0, sm, N, d.km, d.jm,
-                           1L, (long)d.jm, bjm, btc, bjp);
-    for (int nj = 1; nj <= njsp; ++nj) {
-        hipLaunchKernelGGL(k_sweep_ref<LT>, dim3(1), dim3(SWEEP_THREADS),
-                           sizeof(double) * (3 * d.jm + 36 * SWEEP_CHUNK), sm, d, 0, nj, prm.underr, dq, s, btc, bjm,
-                           bjp, bkm, bkp);
-        if ((nj / nbcimp) * nbcimp == nj) launch_wake(sm, d, 3, w, q, dq, s);
-    }
+        hipLaunchKernelGGL(k_btlu3<double>, groups(d.km), lines(d.km), 0, sm, N, d.km,
+                           d.jm, 1L, (long)d.jm, bjm, btc, bjp, pk);
+    for (int nj = 1; nj <= njsp; ++nj) sweep(0, nj, bkm, bkp);
     if (njsp > 0)
-        hipLaunchKernelGGL(k_btund3<LT>, dim3((d.km + lpb - 1) / lpb), dim3(lpb), 0, sm, N, d.km, d.jm,
-                           1L, (long)d.jm, bjm, btc, bjp);
+        hipLaunchKernelGGL(k_btund3<double>, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, sm, N,
+                           d.jm, bjm, btc, bjp, pk);
     if (nksp > 0)
-        hipLaunchKernelGGL(k_btlu3<LT>, dim3((d.jm + lpb - 1) / lpb), dim3(lpb), 0, sm, N, d.jm, d.km,
-                           (long)d.jm, 1L, bkm, btc, bkp);
-    for (int nk = 1; nk <= nksp; ++nk) {
-        hipLaunchKernelGGL(k_sweep_ref<LT>, dim3(1), dim3(SWEEP_THREADS),
-                           sizeof(double) * (3 * d.km + 36 * SWEEP_CHUNK), sm, d, 1, nk, prm.underr, dq, s, btc, bkm,
-                           bkp, bjm, bjp);
-        if ((nk / nbcimp) * nbcimp == nk) launch_wake(sm, d, 3, w, q, dq, s);
-    }
+        hipLaunchKernelGGL(k_btlu3<double>, groups(d.jm), lines(d.jm), 0, sm, N, d.jm,
+                           d.km, (long)d.jm, 1L, bkm, btc, bkp, pk);
+    for (int nk = 1; nk <= nksp; ++nk) sweep(1, nk, bjm, bjp);
 }
-
-template void launch_lrelax_ref<double>(hipStream_t, const Dims &, const DevParams &, int, int,
-                                        int, const WakePairs &, const double *, double *,
-                                        double *, double *, double *, double *, double *,
-                                        double *, int);
 
 }  // namespace smac

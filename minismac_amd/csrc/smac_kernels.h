@@ -45,10 +45,13 @@ void launch_resid(hipStream_t, const Dims &, int nt, double beta, const double *
                   const double *dj, Scratch &, DevStats *);
 
 // linerelax.hip: lrelax in the reference's line order (ref/lrelax.f:51-221)
-template <typename LT>
+// pack: lr_ref_bytes of device memory for the factored lines.  btc and bjp come back recomposed
+// from their xi factors, as the reference leaves them for the eta lines.
+long lr_ref_bytes(const Dims &);
 void launch_lrelax_ref(hipStream_t, const Dims &, const DevParams &, int njsp, int nksp,
                        int nbcimp, const WakePairs &, const double *q, double *dq, double *s,
-                       LT *btc, LT *bjm, LT *bjp, LT *bkm, LT *bkp, int lines_per_block = 64);
+                       double *btc, const double *bjm, double *bjp, const double *bkm,
+                       const double *bkp, void *pack, int lines_per_block = 64);
 void launch_wake(hipStream_t, const Dims &, int neqs, const WakePairs &, const double *sq,
                  double *ds, double *rhs);
 
