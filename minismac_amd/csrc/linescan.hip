@@ -5,7 +5,7 @@
 // block-tridiagonal system by block Thomas: the factorisation B_i = b_i - a_i C_(i-1),
 // C_i = B_i^-1 c_i, then y_i = B_i^-1 (r_i - a_i y_(i-1)) forward and x_i = y_i - C_i x_(i+1)
 // backward.  The factorisation does not depend on the right-hand side, so it is done once per
-// direction for all lines at once (k_lr_factor, one thread per line); it also forms
+// direction for all lines at once (k_lr_factor); it also forms
 // M_i = -B_i^-1 a_i, so that both substitutions are affine recurrences,
 //     y_i = M_i y_(i-1) + B_i^-1 r_i,        x_i = (-C_i) x_(i+1) + y_i,
 // and each is a prefix scan of affine maps (3x3 matrix, 3-vector) along the line.  One
@@ -97,21 +97,21 @@ SMAC_DEV void aff_shfl_down(Aff<T, NEQ> &o, const Aff<T, NEQ> &a, int d)
 
 // ------------------------------------------------------------------------------------------
 // factorisation: the block Thomas recurrence of btlu3j / btlu3k (ref/btlu3.f:52-624) and of
-// scatri (ref/lreltur.f:337-359), for every line of both directions in one launch, one
-// wavefront per line.  Waves [0, nx) take the xi lines (k = const: contiguous along the line),
-// waves [nx, nx + ne) the eta lines (j = const: stride jm).  The recurrence
+// scatri (ref/lreltur.f:337-359), for every line of both directions in one launch:
 //     T_i = b_i - a_i C_(i-1),   C_i = T_i^-1 c_i            (a_0 = 0, c_(len-1) = 0)
-// is sequential along the line, so the wave walks it in chunks of 64 points: lane u loads
-// point c0+u's blocks (coalesced for xi lines; for eta lines each lane reads its own cache
-// line, which the neighbouring lines' waves share through L2), the blocks are staged in LDS,
-// the next chunk's loads are issued, and then every lane steps through the chunk's points
-// reading each point's blocks from one LDS address (a broadcast) -- the recurrence runs
-// redundantly in all lanes, which costs nothing in a wave that has no other work.  A step
-// forms T_i^-1 c_i by the adjugate (one reciprocal on the chain) and writes C_i to LDS; after
-// the chunk lane u redoes its own point's pivot from C_(u-1), forms T_i^-1 and
-// M_i = -T_i^-1 a_i, and stores the operand planes line-major with coalesced stores.  The blocks to the neighbouring lines are copied
-// through unchanged.  (The reference keeps T_i as LU factors; the explicit inverse makes
-// the sweeps' T_i^-1 r_i a parallel product.)
+// Lane u of a group of CH lanes holds point c0+u of a line (the whole wave, or one of the four
+// 16-lane DPP rows of a wave that takes four lines).  In every step every lane forms T, adj(T),
+// det(T) and C of its own point from the C that the lane before it held (a DPP shift; the
+// group's first lane takes the one left by the chunk before): after u+1 steps lane u's value is
+// that of the recurrence, and forming it again in later steps leaves it as it is.  So a chunk
+// of CH points takes CH steps of about 110 instructions in registers alone, with no LDS access,
+// broadcast or capture, and T^-1 and M = -T^-1 a follow from what the lanes hold at its end.
+// The bound is the issue of those instructions, one per 5 cycles for a wave alone on its SIMD,
+// over half the longest line.  Broadcasting every point's blocks through LDS to a recurrence
+// that all lanes form alike took 238 us at 945x241 in FP64 and 116 at 705x173 in FP32; this
+// takes 160 and 92 (reference-order FP32 945x241, whole lines: 287 and 255).
+// (The reference keeps T_i as LU factors; the explicit inverse makes the sweeps' T_i^-1 r_i a
+// parallel product.)  The blocks to the neighbouring lines pass through to the operand planes.
 
 // 1/x: the hardware reciprocal refined by Newton-Raphson steps r <- r + r (1 - x r), each of
 // which doubles the number of correct bits (two for FP64, one for FP32)
@@ -160,8 +160,6 @@ SMAC_DEV void mm(const T *x, const T *y, T *out)
         }
 }
 
-constexpr int FW = 64;   // points per chunk = lanes of the wave
-
 // The line is split at m = len/2 and eliminated from both ends at once (a twisted
 // factorisation): wave 0 runs the recurrence forward over points 0..m-1,
 //     T_i = b_i - a_i C_(i-1),   C_i = T_i^-1 c_i,      M_i = -T_i^-1 a_i,
@@ -170,39 +168,62 @@ constexpr int FW = 64;   // points per chunk = lanes of the wave
 // and the middle point takes both: T_m = b_m - a_m C_(m-1) - c_m D_(m+1), with
 // Ma = -T_m^-1 a_m and Mc = -T_m^-1 c_m.  Each half's chain is half the line.  Planes per
 // point: T^-1; M (Ma at m); -C or -D (Mc at m); the blocks to the previous and next line.
-template <typename LT, int NEQ>
-__global__ void __launch_bounds__(2 * FW)
-k_lr_factor(Dims d, int nx, int twist, const LT *__restrict__ btc, const LT *__restrict__ bjm,
-            const LT *__restrict__ bjp, const LT *__restrict__ bkm, const LT *__restrict__ bkp,
-            LT *__restrict__ opx, LT *__restrict__ ope)
+// A workgroup takes LPW lines (1 or 4), wave 0 their first halves and wave 1 their second.
+constexpr int FW = 64;
+
+// another lane's value by a DPP move; zero where the move has no source lane
+template <int CTRL> SMAC_DEV float dpp_of(float v)
 {
-    constexpr int NB = NEQ * NEQ;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const bool eta = (int)blockIdx.x >= nx;
-    // the xi lines are the longer chains: their waves win issue slots on a shared SIMD
-    if (!eta) __builtin_amdgcn_s_setprio(2);
-    // eta lines: a point's nine planes are read by lanes jm apart, and the lines of
-    // neighbouring j share those cache lines; workgroups reach the 8 XCDs round-robin, so
-    // each XCD takes a contiguous run of j (its own L2 then holds the shared lines)
-    int l = (int)blockIdx.x;
-    if (eta) {
-        const int t = (int)blockIdx.x - nx, ne = (int)gridDim.x - nx;
-        const int r = t % 8, q = ne / 8, rem = ne % 8;
-        l = r * q + (r < rem ? r : rem) + t / 8;
-    }
-    const int len = eta ? d.km : d.jm;
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL,
+                                                                 0xf, 0xf, true));
+}
+template <int CTRL> SMAC_DEV double dpp_of(double v)
+{
+    const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)u, CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(u >> 32), CTRL, 0xf, 0xf, true);
+    return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) |
+                                            (unsigned long long)(unsigned)lo));
+}
+
+// t -= x C, and for T = t - x C:  det(T) and adj(T) (T^-1 = adj / det)
+template <typename LT, int NEQ>
+SMAC_DEV void lr_less(const LT *x, LT *t, const LT *C)
+{
+#pragma unroll
+    for (int cc = 0; cc < NEQ; ++cc)
+#pragma unroll
+        for (int r = 0; r < NEQ; ++r)
+#pragma unroll
+            for (int k = 0; k < NEQ; ++k)
+                t[r + NEQ * cc] = t[r + NEQ * cc] - x[r + NEQ * k] * C[k + NEQ * cc];
+}
+template <typename LT, int NEQ>
+SMAC_DEV LT lr_pivot(const LT *x, LT *t, const LT *C, LT *ad)
+{
+    lr_less<LT, NEQ>(x, t, C);
+    if constexpr (NEQ == 3) return adj3(t, ad);
+    ad[0] = (LT)1;
+    return t[0];
+}
+
+template <typename LT, int NEQ, int LPW>
+SMAC_DEV void lr_factor(const Dims &d, bool eta, int grp, int twist, const LT *__restrict__ btc,
+                        const LT *__restrict__ lm, const LT *__restrict__ lp,
+                        const LT *__restrict__ om, const LT *__restrict__ opn,
+                        LT *__restrict__ out, LT (*edge)[4][NEQ * NEQ])
+{
+    constexpr int NB = NEQ * NEQ, CH = FW / LPW;
+    constexpr int SHR = LPW == 1 ? 0x138 : 0x111, ROR = LPW == 1 ? 0x13c : 0x121;   // wave / row
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, u = lane % CH, row = lane / CH;
+    const int nline = eta ? d.jm : d.km, len = eta ? d.km : d.jm;
+    const int l = grp * LPW + row;
+    const bool on = l < nline;
     // twist = 0: the plain (one-sided) factorisation, forward over the whole line (wave 0;
     // launched with one wave)
     const int mid = twist ? len / 2 : len;
     const long N = d.N;
     const long stride = eta ? d.jm : 1, base = eta ? (long)l : (long)l * d.jm;
-    const LT *lm = eta ? bkm : bjm, *lp = eta ? bkp : bjp, *om = eta ? bjm : bkm,
-             *opn = eta ? bjp : bkp;
-    LT *out = eta ? ope : opx;
-    __shared__ LT sh[2][FW][3 * NB + 1];   // per wave: carried-side, b, solve-side blocks
-    __shared__ LT res[2][FW][NB + 1];      // per wave: C (or D) of the chunk's points
-    __shared__ LT cinl[2][NB];             // per wave: the C entering the chunk
-    __shared__ LT edge[2][NB];             // C_(m-1) and D_(m+1)
     // wave 0 walks points 0, 1, .., mid-1; wave 1 walks len-1, len-2, .., mid+1
     const bool fwd = wv == 0;
     const int first = fwd ? 0 : len - 1, count = fwd ? mid : (len - 1 - mid > 0 ? len - 1 - mid : 0),
@@ -210,148 +231,106 @@ k_lr_factor(Dims d, int nx, int twist, const LT *__restrict__ btc, const LT *__r
     // forward: the carried side is a (times C of the point before), the solved side c;
     // backward the other way round
     const LT *carried = fwd ? lm : lp, *solved = fwd ? lp : lm;
-    LT rcar[NB], rb[NB], rsol[NB], rom[NB], rop[NB];
-    // a chunk's blocks of this direction (prefetched over the previous chunk's recurrence) ...
-    auto load = [&](int c0) {
-        const int u = c0 + lane;
-        if (u < count) {
-            const int i = first + step * u;
+    struct Pt { LT car[NB], b[NB], sol[NB]; } cur, nxt;
+    auto load = [&](Pt &t, int c0) {
+        const int v = c0 + u;
+        if (on && v < count) {
+            const int i = first + step * v;
             const long p = base + stride * i;
             const bool has_a = i > 0, has_c = i < len - 1;
             const bool has_car = fwd ? has_a : has_c, has_sol = fwd ? has_c : has_a;
 #pragma unroll
             for (int e = 0; e < NB; ++e) {
-                rb[e] = btc[e * N + p];
-                rcar[e] = has_car ? carried[e * N + p] : (LT)0;
-                rsol[e] = has_sol ? solved[e * N + p] : (LT)0;
+                t.b[e] = btc[e * N + p];
+                t.car[e] = has_car ? carried[e * N + p] : (LT)0;
+                t.sol[e] = has_sol ? solved[e * N + p] : (LT)0;
             }
         }
     };
-    // ... and the other direction's two blocks, which pass through to the operand planes
-    // (loaded after the recurrence, so that they hold no registers during it)
-    auto load_o = [&](int c0) {
-        const int u = c0 + lane;
-        if (u < count) {
-            const long p = base + stride * (first + step * u);
+    LT C[NB], carry[NB], ad[NB], rd = (LT)0;
+#pragma unroll
+    for (int e = 0; e < NB; ++e) {
+        C[e] = carry[e] = ad[e] = (LT)0;
+        cur.b[e] = cur.car[e] = cur.sol[e] = nxt.b[e] = nxt.car[e] = nxt.sol[e] = (LT)0;
+    }
+    load(cur, 0);
+    for (int c0 = 0; c0 < count; c0 += CH) {
+        const int v = c0 + u;
+        const bool act = on && v < count;
+        const long p = base + stride * (first + step * v);
+        const long o = (long)l * len + (first + step * v);
+        if (c0 + CH < count) load(nxt, c0 + CH);
+        LT rom[NB], rop[NB];
+        if (act) {
 #pragma unroll
             for (int e = 0; e < NB; ++e) {
                 rom[e] = om[e * N + p];
                 rop[e] = opn[e * N + p];
             }
         }
-    };
-    // T = b - x C;  det(T) and adj(T) (T^-1 = adj / det)
-    auto pivot = [&](const LT *x, LT *t, const LT *C, LT *ad) -> LT {
+        const int nv = count - c0 < CH ? count - c0 : CH;
+        // the group's first lane takes its product with the carried value here, and nothing
+        // from a neighbour in the steps
+        LT car[NB];
+        {
+            LT t[NB];
 #pragma unroll
-        for (int cc = 0; cc < NEQ; ++cc)
-#pragma unroll
-            for (int r = 0; r < NEQ; ++r)
-#pragma unroll
-                for (int k = 0; k < NEQ; ++k)
-                    t[r + NEQ * cc] = t[r + NEQ * cc] - x[r + NEQ * k] * C[k + NEQ * cc];
-        if constexpr (NEQ == 3) return adj3(t, ad);
-        ad[0] = (LT)1;
-        return t[0];
-    };
-    LT C[NB];
-#pragma unroll
-    for (int e = 0; e < NB; ++e) C[e] = (LT)0;
-    load(0);
-    load_o(0);
-    // both waves make the same number of chunk steps (their barriers pair up); the shorter
-    // half idles through its last one
-    const int nchunk = twist && len - 1 - mid > mid ? len - 1 - mid : mid;
-    for (int c0 = 0; c0 < nchunk; c0 += FW) {
-        const int u0 = c0 + lane;
-        const long o = (long)l * len + (first + step * u0);
-        if (lane == 0) {
-#pragma unroll
-            for (int e = 0; e < NB; ++e) cinl[wv][e] = C[e];
-        }
-        if (u0 < count) {
+            for (int e = 0; e < NB; ++e) t[e] = cur.b[e];
+            lr_less<LT, NEQ>(cur.car, t, carry);
 #pragma unroll
             for (int e = 0; e < NB; ++e) {
-                sh[wv][lane][e] = rcar[e];
-                sh[wv][lane][NB + e] = rb[e];
-                sh[wv][lane][2 * NB + e] = rsol[e];
-                out[(3 * NB + e) * N + o] = rom[e];
-                out[(4 * NB + e) * N + o] = rop[e];
+                cur.b[e] = u == 0 ? t[e] : cur.b[e];
+                car[e] = u == 0 ? (LT)0 : cur.car[e];
             }
         }
-        __syncthreads();
-        if (c0 + FW < count) load(c0 + FW);
-        const int nv = count - c0 < FW ? (count - c0 > 0 ? count - c0 : 0) : FW;
-        // the recurrence, in every lane of the wave: only C goes on to the next point.  Two
-        // register sets alternate: the next point's blocks are read from LDS while this
-        // one's are used, so that their latency is off the chain; one lane keeps C for the
-        // per-lane pass below.
-        LT xa[NB], ta[NB], ca[NB], xb[NB], tb[NB], cb[NB];
-        auto rd3 = [&](int u, LT *x, LT *t, LT *c) {
-            const int q = u < FW ? u : FW - 1;   // past the chunk: read, never used
+        for (int s = 0; s < nv; ++s) {
+            LT x[NB], t[NB], ac[NB];
 #pragma unroll
             for (int e = 0; e < NB; ++e) {
-                x[e] = sh[wv][q][e];
-                t[e] = sh[wv][q][NB + e];
-                c[e] = sh[wv][q][2 * NB + e];
+                x[e] = dpp_of<SHR>(C[e]);
+                t[e] = cur.b[e];
             }
-        };
-        auto rec = [&](const LT *x, LT *t, const LT *c, int u) {
-            LT ad[NB], ac[NB];
-            const LT det = pivot(x, t, C, ad);
-            mm<LT, NEQ>(ad, c, ac);
-            const LT rd = rcp_nr(det);
+            const LT det = lr_pivot<LT, NEQ>(car, t, x, ad);
+            mm<LT, NEQ>(ad, cur.sol, ac);
+            rd = rcp_nr(det);
 #pragma unroll
             for (int e = 0; e < NB; ++e) C[e] = ac[e] * rd;
-            if (lane == 0) {
-#pragma unroll
-                for (int e = 0; e < NB; ++e) res[wv][u][e] = C[e];
-            }
-        };
-        rd3(0, xa, ta, ca);
-        for (int u = 0; u < nv; u += 2) {
-            rd3(u + 1, xb, tb, cb);
-            rec(xa, ta, ca, u);
-            if (u + 1 < nv) {
-                rd3(u + 2, xa, ta, ca);
-                rec(xb, tb, cb, u + 1);
-            }
         }
-        __syncthreads();
-        if (c0 + FW < count) load_o(c0 + FW);
-        // each lane redoes its own point's pivot from the C entering it (the same operations
-        // as the recurrence, so the same values) and forms T^-1 and M = -T^-1 x; its blocks
-        // are still in the chunk's LDS
-        if (u0 < count) {
-            LT cp[NB], ad[NB], bi[NB], m[NB], ocar[NB], ob[NB];
-#pragma unroll
-            for (int e = 0; e < NB; ++e) {
-                cp[e] = lane > 0 ? res[wv][lane - 1][e] : cinl[wv][e];
-                ocar[e] = sh[wv][lane][e];
-                ob[e] = sh[wv][lane][NB + e];
-            }
-            const LT rd = rcp_nr(pivot(ocar, ob, cp, ad));
+        if (act) {
+            LT bi[NB], m[NB];
 #pragma unroll
             for (int e = 0; e < NB; ++e) bi[e] = ad[e] * rd;
-            mm<LT, NEQ>(bi, ocar, m);
+            mm<LT, NEQ>(bi, cur.car, m);
 #pragma unroll
             for (int e = 0; e < NB; ++e) {
                 out[e * N + o] = bi[e];
                 out[(NB + e) * N + o] = -m[e];
-                out[(2 * NB + e) * N + o] = -res[wv][lane][e];
+                out[(2 * NB + e) * N + o] = -C[e];
+                out[(3 * NB + e) * N + o] = rom[e];
+                out[(4 * NB + e) * N + o] = rop[e];
             }
         }
-        __syncthreads();
+        if (c0 + CH >= count) {
+            if (u == nv - 1) {
+#pragma unroll
+                for (int e = 0; e < NB; ++e) edge[wv][row][e] = C[e];   // C_(m-1) / D_(m+1)
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < NB; ++e) carry[e] = dpp_of<ROR>(C[e]);
+            cur = nxt;
+        }
     }
     if (!twist) return;
-    if (lane == 0) {
+    if (count == 0 && u == 0) {
 #pragma unroll
-        for (int e = 0; e < NB; ++e) edge[wv][e] = C[e];   // C_(m-1) / D_(m+1) (0 if empty)
+        for (int e = 0; e < NB; ++e) edge[wv][row][e] = (LT)0;
     }
     __syncthreads();
     // the middle point
-    if (threadIdx.x == 0) {
+    if (wv == 0 && u == 0 && on) {
         const long p = base + stride * mid, o = (long)l * len + mid;
-        LT a[NB], b[NB], c[NB], t[NB], ad[NB], u[NB];
+        LT a[NB], b[NB], c[NB], t[NB], am[NB], w[NB];
 #pragma unroll
         for (int e = 0; e < NB; ++e) {
             b[e] = btc[e * N + p];
@@ -361,23 +340,62 @@ k_lr_factor(Dims d, int nx, int twist, const LT *__restrict__ btc, const LT *__r
             out[(4 * NB + e) * N + o] = opn[e * N + p];
             t[e] = b[e];
         }
-        pivot(a, t, edge[0], ad);        // b - a C_(m-1)
-        const LT det = pivot(c, t, edge[1], ad);   // - c D_(m+1)
-        const LT rd = rcp_nr(det);
+        lr_pivot<LT, NEQ>(a, t, edge[0][row], am);              // b - a C_(m-1)
+        const LT det = lr_pivot<LT, NEQ>(c, t, edge[1][row], am);   // - c D_(m+1)
+        const LT rm = rcp_nr(det);
         LT bi[NB];
 #pragma unroll
-        for (int e = 0; e < NB; ++e) bi[e] = ad[e] * rd;
-        mm<LT, NEQ>(bi, a, u);
+        for (int e = 0; e < NB; ++e) bi[e] = am[e] * rm;
+        mm<LT, NEQ>(bi, a, w);
 #pragma unroll
         for (int e = 0; e < NB; ++e) {
             out[e * N + o] = bi[e];
-            out[(NB + e) * N + o] = -u[e];
+            out[(NB + e) * N + o] = -w[e];
         }
-        mm<LT, NEQ>(bi, c, u);
+        mm<LT, NEQ>(bi, c, w);
 #pragma unroll
-        for (int e = 0; e < NB; ++e) out[(2 * NB + e) * N + o] = -u[e];
+        for (int e = 0; e < NB; ++e) out[(2 * NB + e) * N + o] = -w[e];
     }
 }
+
+// workgroups [0, nx) take the xi lines (k = const: contiguous along the line), the rest the eta
+// lines (j = const: stride jm); lpx, lpe: lines per workgroup of each
+template <typename LT, int NEQ>
+__global__ void __launch_bounds__(2 * FW)
+k_lr_factor(Dims d, int nx, int lpx, int lpe, int twist, const LT *__restrict__ btc,
+            const LT *__restrict__ bjm, const LT *__restrict__ bjp, const LT *__restrict__ bkm,
+            const LT *__restrict__ bkp, LT *__restrict__ opx, LT *__restrict__ ope)
+{
+    __shared__ LT edge[2][4][NEQ * NEQ];   // per half and line of the workgroup
+    if ((int)blockIdx.x < nx) {
+        // the xi lines are the longer chains: their waves win issue slots on a shared SIMD
+        __builtin_amdgcn_s_setprio(2);
+        if (lpx == 1)
+            lr_factor<LT, NEQ, 1>(d, false, (int)blockIdx.x, twist, btc, bjm, bjp, bkm, bkp, opx, edge);
+        else
+            lr_factor<LT, NEQ, 4>(d, false, (int)blockIdx.x, twist, btc, bjm, bjp, bkm, bkp, opx, edge);
+        return;
+    }
+    // eta lines: a point's planes are read by lanes jm apart, and the lines of neighbouring j
+    // share those cache lines; workgroups reach the 8 XCDs round-robin, so each XCD takes a
+    // contiguous run of j (its own L2 then holds the shared lines)
+    const int t = (int)blockIdx.x - nx, ne = (int)gridDim.x - nx;
+    const int r = t % 8, q = ne / 8, rem = ne % 8;
+    const int g = r * q + (r < rem ? r : rem) + t / 8;
+    if (lpe == 1)
+        lr_factor<LT, NEQ, 1>(d, true, g, twist, btc, bkm, bkp, bjm, bjp, ope, edge);
+    else
+        lr_factor<LT, NEQ, 4>(d, true, g, twist, btc, bkm, bkp, bjm, bjp, ope, edge);
+}
+
+// Lines per workgroup.  One where the direction's waves (two per line when twisted) find a SIMD
+// each: a chunk of 64 points loads and stores coalesced and pays its ends once per 64 steps.
+// Four where they do not: two waves on a SIMD halve each other's rate, and four lines in one
+// wave take the steps of one.  Twisted FP64 945x241 (241 xi lines, 945 eta lines): one line
+// everywhere 212 us, four everywhere 202, the xi lines singly and the eta lines by four 160;
+// FP32 705x173 101, 109, 92.  Below the line one per workgroup stays the better: 203x47 FP64
+// 36 us against 42, the plain FP32 factorisation of 945x241 255 against 289.
+static int lines_per_group(int nline, bool twist) { return nline * (twist ? 2 : 1) <= 1024 ? 1 : 4; }
 
 // ------------------------------------------------------------------------------------------
 // the sweep: lines count of them, line l = (first + idx*step) mod nline.  SEQ: one
@@ -787,10 +805,11 @@ void launch_lr_factor3(hipStream_t sm, const Dims &d, bool xi, bool eta, bool tw
                        const LT *btc, const LT *bjm, const LT *bjp, const LT *bkm, const LT *bkp,
                        LT *opx, LT *ope)
 {
-    const int nx = xi ? d.km : 0, ne = eta ? d.jm : 0;
+    const int lpx = lines_per_group(d.km, twist), lpe = lines_per_group(d.jm, twist);
+    const int nx = xi ? (d.km + lpx - 1) / lpx : 0, ne = eta ? (d.jm + lpe - 1) / lpe : 0;
     if (nx + ne > 0)
         hipLaunchKernelGGL((k_lr_factor<LT, 3>), dim3(nx + ne), dim3(twist ? 2 * FW : FW), 0, sm, d,
-                           nx, twist ? 1 : 0, btc, bjm, bjp, bkm, bkp, opx, ope);
+                           nx, lpx, lpe, twist ? 1 : 0, btc, bjm, bjp, bkm, bkp, opx, ope);
 }
 
 template <typename LT>
@@ -925,9 +944,10 @@ void launch_sa_lreltur_scan(hipStream_t sm, const Dims &d, int ntjsp, const Wake
     // the zebra order (that of the mean flow) a pass takes the even lines, the odd lines, and
     // then line k = 1 again.
     hipLaunchKernelGGL(k_zero, dim3(256), dim3(256), 0, sm, a.ds, d.N);
-    hipLaunchKernelGGL((k_lr_factor<double, 1>), dim3(d.km), dim3(ws.zebra ? 2 * FW : FW), 0, sm, d,
-                       d.km, ws.zebra ? 1 : 0, a.stc,
-                       a.sjm, a.sjp, a.skm, a.skp, ws.sa_op, (double *)nullptr);
+    const int lpx = lines_per_group(d.km, ws.zebra), nx = (d.km + lpx - 1) / lpx;
+    hipLaunchKernelGGL((k_lr_factor<double, 1>), dim3(nx), dim3(ws.zebra ? 2 * FW : FW), 0, sm, d, nx,
+                       lpx, lpx, ws.zebra ? 1 : 0, a.stc, a.sjm, a.sjp, a.skm, a.skp, ws.sa_op,
+                       (double *)nullptr);
     for (int pass = 1; pass <= ntjsp; ++pass) {
         if (ws.zebra) {
             sweep_launch<double, 1, false>(sm, d.km, d.jm, d.N, (d.km + 1) / 2, 0, 2, 1.0, 1,
