@@ -885,8 +885,9 @@ static smac_status adj_prepare(smac_handle *h, int m)
         if (c.lr) {
             // the factored lines of M and M^T (FP64) and the transposed sweeps' vectors
             char *f = nullptr, *t = nullptr;
-            if ((rc = dalloc(h, &f, 2 * 45 * N * 8)) || (rc = dalloc(h, &t, 2 * 45 * N * 8)))
-                return rc;
+            // and 256 bytes, as the sweeps' last pair may read past the last line
+            const size_t fb = (size_t)2 * 45 * N * 8 + 256;
+            if ((rc = dalloc(h, &f, fb)) || (rc = dalloc(h, &t, fb))) return rc;
             c.lr_f.opx = f;
             c.lr_f.ope = f + 45 * N * 8;
             c.lr_t.opx = t;

@@ -77,22 +77,43 @@ SMAC_DEV void aff_apply(const T *m, const T *v, const T *x, T *out)
     }
 }
 
-template <typename T, int NEQ>
-SMAC_DEV void aff_shfl_up(Aff<T, NEQ> &o, const Aff<T, NEQ> &a, int d)
+// another lane's value by a DPP move; zero where the move has no source lane
+template <int CTRL> SMAC_DEV float dpp_of(float v)
 {
-#pragma unroll
-    for (int e = 0; e < NEQ * NEQ; ++e) o.m[e] = __shfl_up(a.m[e], d, 64);
-#pragma unroll
-    for (int e = 0; e < NEQ; ++e) o.v[e] = __shfl_up(a.v[e], d, 64);
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL,
+                                                                 0xf, 0xf, true));
+}
+template <int CTRL> SMAC_DEV double dpp_of(double v)
+{
+    const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)u, CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(u >> 32), CTRL, 0xf, 0xf, true);
+    return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) |
+                                            (unsigned long long)(unsigned)lo));
 }
 
-template <typename T, int NEQ>
-SMAC_DEV void aff_shfl_down(Aff<T, NEQ> &o, const Aff<T, NEQ> &a, int d)
+// the value OFF lanes below (UP) or above; lanes that have none get anything.  One lane is a
+// DPP move and half a wave a swap of halves; the distances between go through the LDS crossbar,
+// whose latency of about 120 cycles a wave alone on its SIMD has nothing to fill with.
+template <int OFF, bool UP> SMAC_DEV int lane_shift(int v, int lane)
 {
-#pragma unroll
-    for (int e = 0; e < NEQ * NEQ; ++e) o.m[e] = __shfl_down(a.m[e], d, 64);
-#pragma unroll
-    for (int e = 0; e < NEQ; ++e) o.v[e] = __shfl_down(a.v[e], d, 64);
+    if constexpr (OFF == 1)
+        return __builtin_amdgcn_update_dpp(0, v, UP ? 0x138 : 0x130, 0xf, 0xf, true);
+    else if constexpr (OFF == 32)
+        return __builtin_amdgcn_permlane32_swap(v, v, false, false)[UP ? 0 : 1];
+    else
+        return __builtin_amdgcn_ds_bpermute(4 * (UP ? lane - OFF : lane + OFF), v);
+}
+template <int OFF, bool UP> SMAC_DEV float lane_shift(float v, int lane)
+{
+    return __builtin_bit_cast(float, lane_shift<OFF, UP>(__builtin_bit_cast(int, v), lane));
+}
+template <int OFF, bool UP> SMAC_DEV double lane_shift(double v, int lane)
+{
+    const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+    const unsigned lo = (unsigned)lane_shift<OFF, UP>((int)(unsigned)u, lane);
+    const unsigned hi = (unsigned)lane_shift<OFF, UP>((int)(unsigned)(u >> 32), lane);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
 // ------------------------------------------------------------------------------------------
@@ -167,24 +188,11 @@ SMAC_DEV void mm(const T *x, const T *y, T *out)
 //     T_i = b_i - c_i D_(i+1),   D_i = T_i^-1 a_i,      M_i = -T_i^-1 c_i,
 // and the middle point takes both: T_m = b_m - a_m C_(m-1) - c_m D_(m+1), with
 // Ma = -T_m^-1 a_m and Mc = -T_m^-1 c_m.  Each half's chain is half the line.  Planes per
-// point: T^-1; M (Ma at m); -C or -D (Mc at m); the blocks to the previous and next line.
+// point: T^-1; M (Ma at m); -C or -D (Mc at m); the blocks to the previous and next line.  In
+// the planes a line's points stand in the order of the sweeps' scans: the first half, the
+// second from its end, the middle point.
 // A workgroup takes LPW lines (1 or 4), wave 0 their first halves and wave 1 their second.
 constexpr int FW = 64;
-
-// another lane's value by a DPP move; zero where the move has no source lane
-template <int CTRL> SMAC_DEV float dpp_of(float v)
-{
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL,
-                                                                 0xf, 0xf, true));
-}
-template <int CTRL> SMAC_DEV double dpp_of(double v)
-{
-    const unsigned long long u = (unsigned long long)__double_as_longlong(v);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)u, CTRL, 0xf, 0xf, true);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(u >> 32), CTRL, 0xf, 0xf, true);
-    return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) |
-                                            (unsigned long long)(unsigned)lo));
-}
 
 // t -= x C, and for T = t - x C:  det(T) and adj(T) (T^-1 = adj / det)
 template <typename LT, int NEQ>
@@ -258,7 +266,7 @@ SMAC_DEV void lr_factor(const Dims &d, bool eta, int grp, int twist, const LT *_
         const int v = c0 + u;
         const bool act = on && v < count;
         const long p = base + stride * (first + step * v);
-        const long o = (long)l * len + (first + step * v);
+        const long o = (long)l * len + (fwd ? v : mid + v);
         if (c0 + CH < count) load(nxt, c0 + CH);
         LT rom[NB], rop[NB];
         if (act) {
@@ -329,7 +337,7 @@ SMAC_DEV void lr_factor(const Dims &d, bool eta, int grp, int twist, const LT *_
     __syncthreads();
     // the middle point
     if (wv == 0 && u == 0 && on) {
-        const long p = base + stride * mid, o = (long)l * len + mid;
+        const long p = base + stride * mid, o = (long)l * len + len - 1;
         LT a[NB], b[NB], c[NB], t[NB], am[NB], w[NB];
 #pragma unroll
         for (int e = 0; e < NB; ++e) {
@@ -398,8 +406,8 @@ k_lr_factor(Dims d, int nx, int lpx, int lpe, int twist, const LT *__restrict__ 
 static int lines_per_group(int nline, bool twist) { return nline * (twist ? 2 : 1) <= 1024 ? 1 : 4; }
 
 // ------------------------------------------------------------------------------------------
-// the sweep: lines count of them, line l = (first + idx*step) mod nline.  SEQ: one
-// workgroup walks them in order; otherwise one workgroup per line (lines of one colour).
+// the sweep: lines count of them, line l = (first + idx*step) mod nline, one workgroup per line
+// (lines of one colour); k_lr_walk below takes them in order in one workgroup.
 // s, dq: NEQ planes, line-major; op: the factor kernel's planes.  assign: dq = x (the SA's
 // lreltur); otherwise dq += underr (x - dq) (ref/lrelax.f:377-381).  couple = 0 leaves out
 // the neighbouring lines' terms: a plain solve of each line (the transposed sweeps).
@@ -412,6 +420,61 @@ static int lines_per_group(int nline, bool twist) { return nline * (twist ? 2 : 
 //   phase 2  x_i = -C_i x_(i+1) + y_i  backward over i < mid, and
 //            x_i = -D_i x_(i-1) + z_i  forward over i > mid, the point mid entering both
 //            scans as the constant map x_mid.
+//
+// What bounds a sweep of one colour is how fast the few workgroups (121 of 945 points) can draw
+// their operands, then the latency of the scan's exchanges.  With every load in flight before
+// the first wait, pairs of points in one load, the scan without branches, and its distances 1
+// and 32 as DPP move and half-wave swap instead of crossbar reads, a 945x241 FP64 xi colour
+// takes 18.6 us (28.6 before) and an eta colour 16.4 (17.9); FP32 at 705x173 11.7 (14.1) and 9.2
+// (10.1); one colour of the 203x47 transposed sweeps 7.7 (8.5).
+
+// one doubling step: the lane's map after that of OFF lanes before
+template <typename AT, int NEQ, bool FWD, int OFF>
+SMAC_DEV void scan_level(Aff<AT, NEQ> &agg, int lane)
+{
+    Aff<AT, NEQ> o, n = agg;
+#pragma unroll
+    for (int e = 0; e < NEQ * NEQ; ++e) o.m[e] = lane_shift<OFF, FWD>(agg.m[e], lane);
+#pragma unroll
+    for (int e = 0; e < NEQ; ++e) o.v[e] = lane_shift<OFF, FWD>(agg.v[e], lane);
+    aff_after(n, o);
+    const bool has = FWD ? lane >= OFF : lane + OFF < 64;
+#pragma unroll
+    for (int e = 0; e < NEQ * NEQ; ++e) agg.m[e] = has ? n.m[e] : agg.m[e];
+#pragma unroll
+    for (int e = 0; e < NEQ; ++e) agg.v[e] = has ? n.v[e] : agg.v[e];
+}
+
+// the value entering wave wv: the maps of the waves before it, one after the other, from zero.
+// Their totals are read from LDS four at a time ahead of the products, where the registers
+// hold them (8 waves of FP64 3x3 maps: one at a time).
+template <typename AT, int NEQ, int NW, bool FWD>
+SMAC_DEV void wave_entry(const AT (*tot)[NEQ * NEQ + NEQ], int wv, AT *Y)
+{
+    constexpr int NB = NEQ * NEQ, G = sizeof(AT) * NEQ * NW > 96 ? 1 : 4;
+    const int before = __builtin_amdgcn_readfirstlane(FWD ? wv : NW - 1 - wv);
+#pragma unroll
+    for (int n = 0; n < NEQ; ++n) Y[n] = (AT)0;
+#pragma unroll
+    for (int k0 = 0; k0 < NW - 1; k0 += G) {
+        if (k0 >= before) break;
+        AT a[G][NB + NEQ];
+#pragma unroll
+        for (int i = 0; i < G; ++i)
+            if (k0 + i < NW - 1)
+#pragma unroll
+                for (int e = 0; e < NB + NEQ; ++e)
+                    a[i][e] = tot[FWD ? k0 + i : NW - 1 - k0 - i][e];
+#pragma unroll
+        for (int i = 0; i < G; ++i)
+            if (k0 + i < NW - 1 && k0 + i < before) {
+                AT nY[NEQ];
+                aff_apply<AT, NEQ>(a[i], a[i] + NB, Y, nY);
+#pragma unroll
+                for (int n = 0; n < NEQ; ++n) Y[n] = nY[n];
+            }
+    }
+}
 
 // one scan of the thread's PP points along the line (FWD: ascending, else descending) with
 // the value 0 entering the line: get(u, a) gives point u's map, put(u, x) receives the value
@@ -433,17 +496,12 @@ SMAC_DEV void line_scan(Get get, Put put, AT (*tot)[NEQ * NEQ + NEQ], int lane, 
             agg = a;
         }
     }
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        Aff<AT, NEQ> o;
-        if constexpr (FWD) {
-            aff_shfl_up(o, agg, off);
-            if (lane >= off) aff_after(agg, o);
-        } else {
-            aff_shfl_down(o, agg, off);
-            if (lane + off < 64) aff_after(agg, o);
-        }
-    }
+    scan_level<AT, NEQ, FWD, 1>(agg, lane);
+    scan_level<AT, NEQ, FWD, 2>(agg, lane);
+    scan_level<AT, NEQ, FWD, 4>(agg, lane);
+    scan_level<AT, NEQ, FWD, 8>(agg, lane);
+    scan_level<AT, NEQ, FWD, 16>(agg, lane);
+    scan_level<AT, NEQ, FWD, 32>(agg, lane);
     if (lane == (FWD ? 63 : 0)) {
 #pragma unroll
         for (int e = 0; e < NB; ++e) tot[wv][e] = agg.m[e];
@@ -452,21 +510,13 @@ SMAC_DEV void line_scan(Get get, Put put, AT (*tot)[NEQ * NEQ + NEQ], int lane, 
     }
     __syncthreads();
     // the value entering this wave, then this thread
-    AT Y[NEQ], cur[NEQ];
-#pragma unroll
-    for (int n = 0; n < NEQ; ++n) Y[n] = (AT)0;
-    for (int k = 0; k < (FWD ? wv : NW - 1 - wv); ++k) {
-        const int w = FWD ? k : NW - 1 - k;
-        AT nY[NEQ];
-        aff_apply<AT, NEQ>(tot[w], tot[w] + NB, Y, nY);
-#pragma unroll
-        for (int n = 0; n < NEQ; ++n) Y[n] = nY[n];
-    }
-    AT ye[NEQ];
+    AT Y[NEQ];
+    wave_entry<AT, NEQ, NW, FWD>(tot, wv, Y);
+    AT ye[NEQ], cur[NEQ];
     aff_apply<AT, NEQ>(agg.m, agg.v, Y, ye);
 #pragma unroll
     for (int n = 0; n < NEQ; ++n) {
-        const AT nb = FWD ? __shfl_up(ye[n], 1, 64) : __shfl_down(ye[n], 1, 64);
+        const AT nb = lane_shift<1, FWD>(ye[n], lane);
         cur[n] = lane == (FWD ? 0 : 63) ? Y[n] : nb;
     }
 #pragma unroll
@@ -493,7 +543,27 @@ SMAC_DEV void aff_identity(Aff<AT, NEQ> &a)
     }
 }
 
-template <typename LT, int NEQ, int NT, int PP, bool SEQ, bool TWIST>
+// a thread's PP points of NB planes from p on, a pair in one load (of element alignment): with
+// an odd length the last pair reaches one element past the line, which nothing uses; past the
+// last line of the last plane lie the operands' 256 bytes of padding
+template <typename T, int NB, int PP>
+SMAC_DEV void load_planes(T (&x)[PP][NB], const T *p, long N)
+{
+    static_assert(PP == 1 || PP == 2, "one point or a pair");
+    typedef T Pair __attribute__((ext_vector_type(2), aligned(sizeof(T))));
+#pragma unroll
+    for (int e = 0; e < NB; ++e) {
+        if constexpr (PP == 2) {
+            const Pair y = *(const Pair *)(p + e * N);
+            x[0][e] = y.x;
+            x[1][e] = y.y;
+        } else {
+            x[0][e] = p[e * N];
+        }
+    }
+}
+
+template <typename LT, int NEQ, int NT, int PP, bool TWIST>
 __global__ void __launch_bounds__(NT)
 k_lr_sweep(int nline, int len, long N, int count, int first, int step, double underr,
            int assign, int couple, double *__restrict__ dq, const double *__restrict__ s,
@@ -514,69 +584,71 @@ k_lr_sweep(int nline, int len, long N, int count, int first, int step, double un
     auto phys = [&](int v) { return (!TWIST || v < mid) ? v : (v < len - 1 ? len - 1 - v + mid : mid); };
     const LT *pB = op, *pM = op + NB * N, *pC = op + 2 * NB * N, *pOm = op + 3 * NB * N,
              *pOp = op + 4 * NB * N;
-    double dqprev[PP][NEQ];
-    int lprev = -2;
-    for (int idx = SEQ ? 0 : (int)blockIdx.x; idx < count; idx += SEQ ? 1 : (int)gridDim.x) {
-        int l = (first + idx * step) % nline;
-        if (l < 0) l += nline;
+    // point u's place in the natural planes
+    auto nat = [&](int l, int u) {
+        const int v = t * PP + u;
+        return (long)l * len + phys(v < len ? v : len - 1);
+    };
+    for (int idx = (int)blockIdx.x; idx < count; idx += (int)gridDim.x) {
+        const int l = (first + idx * step) % nline;
         const bool hm = couple && l > 0, hp = couple && l < nline - 1;
-        const bool regm = SEQ && lprev == l - 1, regp = SEQ && lprev == l + 1;
         AT mmat[PP][NB];               // M (Ma at mid)
         AT bv[PP][NEQ];                // T^-1 r
         AT w[PP][NEQ];                 // y (i < mid) or z (i > mid); z_(mid+1), then x_mid, at
                                        // the middle point; then x
-        // ---- this thread's points: T^-1 r, M, -C / -D
+        // ---- this thread's points: T^-1 r, M, -C / -D.  Past the line's end (and beyond the
+        // first and last line) stand in-range addresses whose values are not used: without
+        // branches every load is in flight before the first is waited for.
+        const long lo = (long)l * len + (t * PP < len ? t * PP : len - 1);
+        AT bi[PP][NB];
+        double r[PP][NEQ];
+        load_planes(bi, pB + lo, N);
+        load_planes(mmat, pM + lo, N);
 #pragma unroll
-        for (int u = 0; u < PP; ++u) {
-            const int v = t * PP + u;
-            if (v < len) {
-                const long o = (long)l * len + phys(v);
-                double r[NEQ];
+        for (int u = 0; u < PP; ++u)
 #pragma unroll
-                for (int n = 0; n < NEQ; ++n) r[n] = s[n * N + o];
-                if (hm) {
-                    double x[NEQ];
+            for (int n = 0; n < NEQ; ++n) r[u][n] = s[n * N + nat(l, u)];
+        if (couple) {
+            AT om[PP][NB], op_[PP][NB];
+            double xm[PP][NEQ], xp[PP][NEQ];
+            load_planes(om, pOm + lo, N);
+            load_planes(op_, pOp + lo, N);
 #pragma unroll
-                    for (int n = 0; n < NEQ; ++n) x[n] = regm ? dqprev[u][n] : dq[n * N + o - len];
+            for (int u = 0; u < PP; ++u)
 #pragma unroll
-                    for (int m = 0; m < NEQ; ++m) {
-                        double b = (double)pOm[m * N + o] * x[0];
-#pragma unroll
-                        for (int n = 1; n < NEQ; ++n) b = b + (double)pOm[(m + NEQ * n) * N + o] * x[n];
-                        r[m] = r[m] - b;
-                    }
+                for (int n = 0; n < NEQ; ++n) {
+                    xm[u][n] = dq[n * N + nat(hm ? l - 1 : l, u)];
+                    xp[u][n] = dq[n * N + nat(hp ? l + 1 : l, u)];
                 }
-                if (hp) {
-                    double x[NEQ];
 #pragma unroll
-                    for (int n = 0; n < NEQ; ++n) x[n] = regp ? dqprev[u][n] : dq[n * N + o + len];
-#pragma unroll
-                    for (int m = 0; m < NEQ; ++m) {
-                        double b = (double)pOp[m * N + o] * x[0];
-#pragma unroll
-                        for (int n = 1; n < NEQ; ++n) b = b + (double)pOp[(m + NEQ * n) * N + o] * x[n];
-                        r[m] = r[m] - b;
-                    }
-                }
-                AT bi[NB], rr[NEQ];
-#pragma unroll
-                for (int e = 0; e < NB; ++e) bi[e] = pB[e * N + o];
-#pragma unroll
-                for (int n = 0; n < NEQ; ++n) rr[n] = (AT)r[n];
+            for (int u = 0; u < PP; ++u) {
 #pragma unroll
                 for (int m = 0; m < NEQ; ++m) {
-                    AT acc = bi[m] * rr[0];
+                    double b = (double)om[u][m] * xm[u][0];
 #pragma unroll
-                    for (int n = 1; n < NEQ; ++n) acc = acc + bi[m + NEQ * n] * rr[n];
-                    bv[u][m] = acc;
+                    for (int n = 1; n < NEQ; ++n) b = b + (double)om[u][m + NEQ * n] * xm[u][n];
+                    r[u][m] = hm ? r[u][m] - b : r[u][m];
                 }
 #pragma unroll
-                for (int e = 0; e < NB; ++e) mmat[u][e] = pM[e * N + o];
-            } else {
+                for (int m = 0; m < NEQ; ++m) {
+                    double b = (double)op_[u][m] * xp[u][0];
 #pragma unroll
-                for (int e = 0; e < NB; ++e) mmat[u][e] = (AT)0;
+                    for (int n = 1; n < NEQ; ++n) b = b + (double)op_[u][m + NEQ * n] * xp[u][n];
+                    r[u][m] = hp ? r[u][m] - b : r[u][m];
+                }
+            }
+        }
 #pragma unroll
-                for (int n = 0; n < NEQ; ++n) bv[u][n] = (AT)0;
+        for (int u = 0; u < PP; ++u) {
+            AT rr[NEQ];
+#pragma unroll
+            for (int n = 0; n < NEQ; ++n) rr[n] = (AT)r[u][n];
+#pragma unroll
+            for (int m = 0; m < NEQ; ++m) {
+                AT acc = bi[u][m] * rr[0];
+#pragma unroll
+                for (int n = 1; n < NEQ; ++n) acc = acc + bi[u][m + NEQ * n] * rr[n];
+                bv[u][m] = acc;
             }
         }
         // ---- phase 1: y forward over i < mid, z backward over i > mid, in one forward scan
@@ -608,13 +680,7 @@ k_lr_sweep(int nline, int len, long N, int count, int first, int step, double un
             lf, lane, wv);
         // the -C / -D planes (Mc at mid), read only now: phase 1 does not need them
         AT cm[PP][NB];
-#pragma unroll
-        for (int u = 0; u < PP; ++u) {
-            const int v = t * PP + u;
-#pragma unroll
-            for (int e = 0; e < NB; ++e)
-                cm[u][e] = v < len ? pC[e * N + (long)l * len + phys(v)] : (AT)0;
-        }
+        load_planes(cm, pC + lo, N);
         __syncthreads();   // phase 1's wave totals have been read; y_(mid-1) is in xch
         // ---- the middle point: x_mid = T^-1 r + Ma y_(mid-1) + Mc z_(mid+1) (the plain
         // factorisation has none: there mid = len, past the line)
@@ -684,11 +750,167 @@ k_lr_sweep(int nline, int len, long N, int count, int first, int step, double un
                     const double dold = assign ? 0.0 : dq[n * N + o];
                     const double nv = assign ? xd : dold + underr * (xd - dold);
                     dq[n * N + o] = nv;
-                    dqprev[u][n] = nv;
                 }
             }
         }
         __syncthreads();   // phase 2's wave totals and xch have been read before the next line
+    }
+}
+
+// The reference's line order (the plain factorisation): one workgroup walks the lines, line l
+// taking the dq of the line before it from registers (a thread owns the same points of every
+// line) and that of the line after it, not yet updated, from memory.  The walk is one chain, bound
+// by the instructions and exchanges of a line's two scans on one compute unit: the next line's
+// operands are loaded during the present one's scans (AHEAD; where a line takes 1024 threads,
+// their 128 registers do not hold them, and each line loads its own: FP64 1201x241 31 ms a pass
+// against 53 with the spilled prefetch).  FP32-LHS 945x241: an eta line (241 points) 3.2 us, 5.7
+// without prefetch and with crossbar scans, a xi line (945 points) 6.6, before 12.1; FP64 passes
+// 20.0 ms, before 24.9.
+template <typename LT, int NEQ, int NT, int PP>
+__global__ void __launch_bounds__(NT)
+k_lr_walk(int nline, int len, long N, int count, int first, int step, double underr, int assign,
+          double *__restrict__ dq, const double *__restrict__ s, const LT *__restrict__ op)
+{
+    using AT = LT;
+    constexpr int NB = NEQ * NEQ, NW = NT / 64;
+    __shared__ AT lf[NW][NB + NEQ], lb[NW][NB + NEQ];
+    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+    const bool up = step > 0;
+    // planes of the block to the line before (near) and after (far) in the walk
+    const LT *pB = op, *pM = op + NB * N, *pC = op + 2 * NB * N,
+             *pNear = op + (up ? 3 : 4) * NB * N, *pFar = op + (up ? 4 : 3) * NB * N;
+    LT B[PP][NB], M[PP][NB], C[PP][NB], near[PP][NB], far[PP][NB];
+    double rhs[PP][NEQ], fx[PP][NEQ], own[PP][NEQ], done[PP][NEQ];
+    auto line = [&](int idx) {
+        const int l = (first + idx * step) % nline;
+        return l < 0 ? l + nline : l;
+    };
+    // past the line's end in-range addresses stand, whose values nothing uses
+    const int at0 = t * PP < len ? t * PP : len - 1;
+    auto load = [&](LT (&x)[PP][NB], const LT *pl, int l) {
+        load_planes(x, pl + (long)l * len + at0, N);
+    };
+    auto loadv = [&](double (&x)[PP][NEQ], const double *pl, int l) {
+#pragma unroll
+        for (int n = 0; n < NEQ; ++n)
+#pragma unroll
+            for (int u = 0; u < PP; ++u) x[u][n] = pl[n * N + (long)l * len + (t * PP + u < len ? t * PP + u : len - 1)];
+    };
+    // what a line needs before its scans
+    auto fetch = [&](int l) {
+        const int beyond = up ? l + 1 : l - 1;
+        load(B, pB, l);
+        load(near, pNear, l);
+        load(far, pFar, l);
+        loadv(rhs, s, l);
+        loadv(fx, dq, beyond >= 0 && beyond < nline ? beyond : l);
+    };
+    constexpr bool AHEAD = NT < 1024;
+    if (AHEAD) {
+        fetch(line(0));
+        load(M, pM, line(0));
+        load(C, pC, line(0));
+    }
+    int lprev = -2;
+    for (int idx = 0; idx < count; ++idx) {
+        const int l = line(idx), ln = line(idx + 1 < count ? idx + 1 : idx);
+        const bool hm = l > 0, hp = l < nline - 1;
+        const bool regm = lprev == l - 1, regp = lprev == l + 1;
+        AT w[PP][NEQ], bv[PP][NEQ];
+        if (!AHEAD) {
+            fetch(l);
+            load(M, pM, l);
+        }
+#pragma unroll
+        for (int u = 0; u < PP; ++u) {
+            double r[NEQ];
+#pragma unroll
+            for (int n = 0; n < NEQ; ++n) r[n] = rhs[u][n];
+            if (hm) {
+#pragma unroll
+                for (int m = 0; m < NEQ; ++m) {
+                    double x[NEQ];
+#pragma unroll
+                    for (int n = 0; n < NEQ; ++n) x[n] = regm ? done[u][n] : fx[u][n];
+                    double b = (double)(up ? near : far)[u][m] * x[0];
+#pragma unroll
+                    for (int n = 1; n < NEQ; ++n)
+                        b = b + (double)(up ? near : far)[u][m + NEQ * n] * x[n];
+                    r[m] = r[m] - b;
+                }
+            }
+            if (hp) {
+#pragma unroll
+                for (int m = 0; m < NEQ; ++m) {
+                    double x[NEQ];
+#pragma unroll
+                    for (int n = 0; n < NEQ; ++n) x[n] = regp ? done[u][n] : fx[u][n];
+                    double b = (double)(up ? far : near)[u][m] * x[0];
+#pragma unroll
+                    for (int n = 1; n < NEQ; ++n)
+                        b = b + (double)(up ? far : near)[u][m + NEQ * n] * x[n];
+                    r[m] = r[m] - b;
+                }
+            }
+            AT rr[NEQ];
+#pragma unroll
+            for (int n = 0; n < NEQ; ++n) rr[n] = (AT)r[n];
+#pragma unroll
+            for (int m = 0; m < NEQ; ++m) {
+                AT acc = B[u][m] * rr[0];
+#pragma unroll
+                for (int n = 1; n < NEQ; ++n) acc = acc + B[u][m + NEQ * n] * rr[n];
+                bv[u][m] = acc;
+            }
+        }
+        loadv(own, dq, l);
+        if (AHEAD) fetch(ln);
+        line_scan<AT, NEQ, NT, PP, true>(
+            [&](int u, Aff<AT, NEQ> &a) {
+                const bool pass = t * PP + u >= len;
+#pragma unroll
+                for (int r = 0; r < NEQ; ++r) {
+#pragma unroll
+                    for (int c = 0; c < NEQ; ++c)
+                        a.m[r + NEQ * c] = pass ? (r == c ? (AT)1 : (AT)0) : M[u][r + NEQ * c];
+                    a.v[r] = pass ? (AT)0 : bv[u][r];
+                }
+            },
+            [&](int u, const AT *x) {
+#pragma unroll
+                for (int n = 0; n < NEQ; ++n) w[u][n] = x[n];
+            },
+            lf, lane, wv);
+        if (AHEAD) load(M, pM, ln);
+        else load(C, pC, l);
+        line_scan<AT, NEQ, NT, PP, false>(
+            [&](int u, Aff<AT, NEQ> &a) {
+                const bool past = t * PP + u >= len;
+#pragma unroll
+                for (int r = 0; r < NEQ; ++r) {
+#pragma unroll
+                    for (int c = 0; c < NEQ; ++c)
+                        a.m[r + NEQ * c] = past ? (r == c ? (AT)1 : (AT)0) : C[u][r + NEQ * c];
+                    a.v[r] = past ? (AT)0 : w[u][r];
+                }
+            },
+            [&](int u, const AT *x) {
+#pragma unroll
+                for (int n = 0; n < NEQ; ++n) w[u][n] = x[n];
+            },
+            lb, lane, wv);
+        if (AHEAD) load(C, pC, ln);
+#pragma unroll
+        for (int u = 0; u < PP; ++u) {
+            const int v = t * PP + u;
+#pragma unroll
+            for (int n = 0; n < NEQ; ++n) {
+                const double xd = (double)w[u][n];
+                const double nv = assign ? xd : own[u][n] + underr * (xd - own[u][n]);
+                if (v < len) dq[n * N + (long)l * len + v] = nv;
+                done[u][n] = nv;
+            }
+        }
         lprev = l;
     }
 }
@@ -758,22 +980,29 @@ static void sweep_launch(hipStream_t sm, int nline, int len, long N, int count, 
                          int step, double underr, int assign, double *dq, const double *s,
                          const LT *op, int couple, bool twist)
 {
-    const dim3 g(SEQ ? 1 : count);
-#define SW(NT, PPV, TW)                                                                         \
-    hipLaunchKernelGGL((k_lr_sweep<LT, NEQ, NT, PPV, SEQ, TW>), g, dim3(NT), 0, sm, nline, len, \
-                       N, count, first, step, underr, assign, couple, dq, s, op)
-#define SWT(TW)                                                                                 \
+#define SWT(LAUNCH)                                                                             \
     do {                                                                                       \
-        if (len <= 256) SW(256, 1, TW);                                                        \
-        else if (len <= 512) SW(512, 1, TW);                                                   \
-        else if (len <= 1024) SW(512, 2, TW);                                                  \
-        else SW(1024, 2, TW);                                                                  \
+        if (len <= 256) LAUNCH(256, 1);                                                        \
+        else if (len <= 512) LAUNCH(512, 1);                                                   \
+        else if (len <= 1024) LAUNCH(512, 2);                                                  \
+        else LAUNCH(1024, 2);                                                                  \
     } while (0)
-    if constexpr (SEQ) SWT(false);
-    else if (twist) SWT(true);
-    else SWT(false);
+#define WALK(NT, PPV)                                                                           \
+    hipLaunchKernelGGL((k_lr_walk<LT, NEQ, NT, PPV>), dim3(1), dim3(NT), 0, sm, nline, len, N,  \
+                       count, first, step, underr, assign, dq, s, op)
+#define TWISTED(NT, PPV)                                                                        \
+    hipLaunchKernelGGL((k_lr_sweep<LT, NEQ, NT, PPV, true>), dim3(count), dim3(NT), 0, sm,      \
+                       nline, len, N, count, first, step, underr, assign, couple, dq, s, op)
+#define PLAIN(NT, PPV)                                                                          \
+    hipLaunchKernelGGL((k_lr_sweep<LT, NEQ, NT, PPV, false>), dim3(count), dim3(NT), 0, sm,     \
+                       nline, len, N, count, first, step, underr, assign, couple, dq, s, op)
+    if constexpr (SEQ) SWT(WALK);
+    else if (twist) SWT(TWISTED);
+    else SWT(PLAIN);
+#undef PLAIN
+#undef TWISTED
+#undef WALK
 #undef SWT
-#undef SW
 }
 
 // one sweep of lines (reference order: odd sweeps ascending, even descending, as
