@@ -18,8 +18,8 @@
 //    (k-2..k+2), each evaluated once per stencil point with the point's three variables
 //    seeded (the same expressions as the assembly kernel, FP32 islands rounded in value);
 //    BC rows are written directly.
-//  - k_adj_jtv + k_adj_wake_t: lambda -> F_q^T lambda, a gather over the 9 offsets plus the
-//    wake cut's far partner (jb,2).
+//  - k_adj_op: lambda -> F_q^T lambda, a gather over the 9 offsets plus the wake cut's far
+//    partner (jb,2), and the operator's rank-one term.
 //  - the preconditioner: the transpose of the primal iteration's own solve
 //    P = W M^-1 (on non-target rows) + identity (on targets).  For LU-SGS (impsch 2),
 //    M = (D+L) D^-1 (D+U) of the converged state; M^T = (D+U)^T D^-T (D+L)^T is again an
@@ -378,7 +378,7 @@ k_adj_jac(Dims d, AdjParams prm, const signed char *__restrict__ rtype,
         put(od, 0, 1, -b12.v);
         put(od, 0, 2, -b13.v);
     } else if (t == RT_WAKE) {
-        // (q(jt,2) + q(jb,2)) / 2 - q(jt,1); the (jb,2) part is applied by k_adj_wake_t
+        // (q(jt,2) + q(jb,2)) / 2 - q(jt,1); the (jb,2) part is applied by k_adj_op
         for (int m = 0; m < 3; ++m) {
             put(0, m, m, -1.0);
             put(off_index(0, 1), m, m, 0.5);
@@ -387,57 +387,120 @@ k_adj_jac(Dims d, AdjParams prm, const signed char *__restrict__ rtype,
 }
 
 
-// out = F_q^T lam over the 9 offsets (the wake cut's far partner is added by k_adj_wake_t)
-__global__ void __launch_bounds__(256)
-k_adj_jtv(Dims d, const double *__restrict__ jac, const double *__restrict__ lam,
-          double *__restrict__ out)
+// the sum of the ADJ_DOT_BLOCKS partials of a product, in every lane (the order of k_adj_msum)
+constexpr int ADJ_DOT_BLOCKS = 512;
+
+SMAC_DEV double wave_sum(double v)
+{
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    return v;
+}
+SMAC_DEV double part_sum(const double *__restrict__ part)
+{
+    double a = 0.0;
+#pragma unroll
+    for (int b = 0; b < ADJ_DOT_BLOCKS; b += 64) a += part[b + (int)(threadIdx.x & 63)];
+    return wave_sum(a);
+}
+
+// out = F_q^T lam: the 9 offsets and the wake rows' dependence on their partner across the cut
+// ((jb,2) receives lam(jt,1)/2; every point of the cut is the partner of exactly one pair).
+// With part (the partials of fc . lam) out = -F_q^T lam - (fc . lam) g, and with b then
+// out = b - that.  Bound by latency at the sizes in use (a launch per factor of the operator
+// cost 2-4 us each, and the 9 offsets' loads waited for one another): a block of one wave per
+// 64 points of a row, three offsets' loads in flight together.
+__global__ void __launch_bounds__(64)
+k_adj_op(Dims d, const double *__restrict__ jac, const int *__restrict__ across,
+         const double *__restrict__ lam, const double *__restrict__ part,
+         const double *__restrict__ g, const double *__restrict__ b, double *__restrict__ out)
 {
     const Blk bk = xcd_blk();   // the rows of the 9 offsets in this XCD's L2
-    const int j = bk.x * blockDim.x + threadIdx.x, k = bk.y;
-    if (j >= d.jm || k >= d.km) return;
+    const int j = bk.x * 64 + threadIdx.x, k = bk.y;
+    const double c = part ? part_sum(part) : 0.0;
+    if (j >= d.jm) return;
     const long N = d.N, p = P(d, j, k);
+    const int jt = k == 1 ? across[j] : -1;
     double acc[3] = {0.0, 0.0, 0.0};
-    for (int o = 0; o < 9; ++o) {
-        const int jr = j - c_off[o][0], kr = k - c_off[o][1];   // the row whose offset o hits p
-        if (jr < 0 || jr >= d.jm || kr < 0 || kr >= d.km) continue;
-        const long r = P(d, jr, kr);
-        const double l0 = lam[r], l1 = lam[N + r], l2 = lam[2 * N + r];
 #pragma unroll
-        for (int n = 0; n < 3; ++n) {
-            const long b = (long)(o * 9 + 3 * n) * N + r;
-            acc[n] += jac[b] * l0 + jac[b + N] * l1 + jac[b + 2 * N] * l2;
+    for (int o0 = 0; o0 < 9; o0 += 3) {
+        double l[3][3], a[3][9];
+        bool in[3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const int o = o0 + i;
+            // the row whose offset o hits p; past an edge p itself stands in and is not used
+            const int jr = j - c_off[o][0], kr = k - c_off[o][1];
+            in[i] = jr >= 0 && jr < d.jm && kr >= 0 && kr < d.km;
+            const long r = in[i] ? P(d, jr, kr) : p;
+#pragma unroll
+            for (int m = 0; m < 3; ++m) l[i][m] = lam[m * N + r];
+#pragma unroll
+            for (int e = 0; e < 9; ++e) a[i][e] = jac[(long)(o * 9 + e) * N + r];
         }
-    }
 #pragma unroll
-    for (int n = 0; n < 3; ++n) out[n * N + p] = acc[n];
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int n = 0; n < 3; ++n) {
+                const double t = acc[n] + (a[i][3 * n] * l[i][0] + a[i][3 * n + 1] * l[i][1] +
+                                           a[i][3 * n + 2] * l[i][2]);
+                acc[n] = in[i] ? t : acc[n];
+            }
+    }
+    if (jt >= 0)
+#pragma unroll
+        for (int n = 0; n < 3; ++n) acc[n] += 0.5 * lam[n * N + jt];
+#pragma unroll
+    for (int n = 0; n < 3; ++n) {
+        double v = acc[n];
+        if (part) v = -v - c * g[n * N + p];
+        if (b) v = -v + b[n * N + p];
+        out[n * N + p] = v;
+    }
 }
 
-// the wake rows' dependence on their partner across the cut: out(jb,2) += lam(jt,1)/2.  Every
-// point of the cut is the partner of exactly one pair, so no two threads write one entry.
-__global__ void k_adj_wake_t(Dims d, int npair, const int *__restrict__ pairs,
-                             const double *__restrict__ lam, double *__restrict__ out)
+// entry (n, p) of W^T r on the rows that are no targets (zero on those): a target's entry
+// moves, halved, to (jt,2) and (jb,2), so that point (j,2) of the cut gathers both halves
+SMAC_DEV double wake_in(long N, int jm, const signed char *rtype, const int *across,
+                        const double *r, int n, long p)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= npair) return;
-    const long jt = pairs[2 * i], jb = pairs[2 * i + 1];
-    const long N = d.N;
-    if (jt < 0 || jt >= d.jm || jb < 0 || jb >= d.jm) return;
-    for (int n = 0; n < 3; ++n) out[n * N + jb + d.jm] += 0.5 * lam[n * N + jt];
+    double v = rtype[p] == RT_WAKE ? 0.0 : r[n * N + p];
+    if (p >= jm && p < 2 * jm) {
+        const long j = p - jm, jo = across[j];
+        if (jo >= 0) v += 0.5 * r[n * N + j] + 0.5 * r[n * N + jo];
+    }
+    return v;
 }
 
-// W^T r, given v = r with the targets cleared: a target's entry moves, halved, to (jt,2) and
-// (jb,2).  Every cut point is the target of one pair and the partner of one other (inv[i]:
-// the pair whose partner is jt of pair i), so thread i gathers both halves for (jt_i, 2).
-__global__ void k_adj_wake_wt(Dims d, int npair, const int *__restrict__ pairs,
-                              const int *__restrict__ inv, const double *__restrict__ r,
-                              double *__restrict__ v)
+__global__ void __launch_bounds__(256)
+k_adj_wake_in(long N, int jm, const signed char *__restrict__ rtype,
+              const int *__restrict__ across, const double *__restrict__ r,
+              double *__restrict__ v)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= npair) return;
-    const long jt = pairs[2 * i], jo = pairs[2 * inv[i]];
-    const long N = d.N;
-    for (int n = 0; n < 3; ++n)
-        v[n * N + jt + d.jm] += 0.5 * r[n * N + jt] + 0.5 * r[n * N + jo];
+    for (long p = (long)blockIdx.x * blockDim.x + threadIdx.x; p < N;
+         p += (long)gridDim.x * blockDim.x)
+#pragma unroll
+        for (int n = 0; n < 3; ++n) v[n * N + p] = wake_in(N, jm, rtype, across, r, n, p);
+}
+
+// the same in the eta-major layout
+__global__ void __launch_bounds__(256)
+k_adj_wake_in_t(Dims d, const signed char *__restrict__ rtype, const int *__restrict__ across,
+                const double *__restrict__ r, double *__restrict__ v)
+{
+    constexpr int TT = 32;
+    __shared__ double tile[TT][TT + 1];
+    const int n = blockIdx.z, j0 = blockIdx.x * TT, k0 = blockIdx.y * TT;
+    for (int kk = threadIdx.y; kk < TT; kk += 8) {
+        const int k = k0 + kk, j = j0 + threadIdx.x;
+        if (k < d.km && j < d.jm)
+            tile[kk][threadIdx.x] = wake_in(d.N, d.jm, rtype, across, r, n, P(d, j, k));
+    }
+    __syncthreads();
+    for (int jj = threadIdx.y; jj < TT; jj += 8) {
+        const int j = j0 + jj, k = k0 + threadIdx.x;
+        if (k < d.km && j < d.jm) v[n * d.N + (long)j * d.km + k] = tile[threadIdx.x][jj];
+    }
 }
 
 // P's wake rows: out(target) = (z(jt,2) + z(jb,2)) / 2 + u(target), z elsewhere
@@ -480,24 +543,52 @@ __global__ void k_adj_fc(Dims d, double alpha, const signed char *__restrict__ r
     }
 }
 
-// out = -out - s[0] * z  (the rank-one clift coupling of the adjoint operator)
-__global__ void k_adj_negate_rank1(long len, const double *__restrict__ s,
-                                   const double *__restrict__ z, double *__restrict__ out)
+// the block's share of a product into part[blockIdx.x]
+SMAC_DEV void block_part(double acc, double *sh, double *__restrict__ part)
 {
-    const double c = s[0];
-    for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < len;
-         e += (long)gridDim.x * blockDim.x)
-        out[e] = -out[e] - c * z[e];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    acc = wave_sum(acc);
+    if (lane == 0) sh[wv] = acc;
+    __syncthreads();
+    if (threadIdx.x == 0) part[blockIdx.x] = sh[0] + sh[1] + sh[2] + sh[3];
 }
 
-// out = target ? u : z
-__global__ void k_adj_merge_targets(long N, const signed char *__restrict__ rtype,
-                                    const double *__restrict__ u, const double *__restrict__ z,
-                                    double *__restrict__ out)
+// out = target ? u : z, and the partials of fc . out
+__global__ void __launch_bounds__(256)
+k_adj_merge(long N, const signed char *__restrict__ rtype, const double *__restrict__ u,
+            const double *__restrict__ z, double *__restrict__ out,
+            const double *__restrict__ fc, double *__restrict__ part)
 {
+    __shared__ double sh[4];
+    double acc = 0.0;
     for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < 3 * N;
-         e += (long)gridDim.x * blockDim.x)
-        out[e] = rtype[e % N] == RT_WAKE ? u[e] : z[e];
+         e += (long)gridDim.x * blockDim.x) {
+        const double v = rtype[e % N] == RT_WAKE ? u[e] : z[e];
+        out[e] = v;
+        acc += fc[e] * v;
+    }
+    block_part(acc, sh, part);
+}
+
+// x + smu (fc . x) binv (pin: the partials of fc . x; left out without smu) into x, or added to
+// y; pout: the partials of fc with what was stored
+__global__ void __launch_bounds__(256)
+k_adj_rank1(long len, const double *__restrict__ pin, double binv, const double *__restrict__ smu,
+            double *__restrict__ x, double *__restrict__ y, const double *__restrict__ fc,
+            double *__restrict__ pout)
+{
+    __shared__ double sh[4];
+    const double a = smu ? part_sum(pin) * binv : 0.0;
+    double acc = 0.0;
+    for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < len;
+         e += (long)gridDim.x * blockDim.x) {
+        double v = x[e];
+        if (smu) v += a * smu[e];
+        if (y) v = y[e] + v;
+        (y ? y : x)[e] = v;
+        acc += fc[e] * v;
+    }
+    block_part(acc, sh, pout);
 }
 
 // the block arrays of M^T's LU-SGS form (see the file header)
@@ -761,13 +852,6 @@ __global__ void k_adj_force_tangent(Dims d, int ivis, double vnu, Walls wl,
 // the plain one-vector form.
 constexpr int MDG = 8;
 
-SMAC_DEV double wave_sum(double v)
-{
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
-
 __global__ void __launch_bounds__(256)
 k_adj_mdot(long len, int nv, const double *__restrict__ V, const double *__restrict__ w,
            double *__restrict__ part, const int *__restrict__ gate)
@@ -815,15 +899,11 @@ k_adj_dot1(long len, const double *__restrict__ v, const double *__restrict__ w,
            double *__restrict__ part)
 {
     __shared__ double sh[4];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     double acc = 0.0;
     for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < len;
          e += (long)gridDim.x * blockDim.x)
         acc += v[e] * w[e];
-    acc = wave_sum(acc);
-    if (lane == 0) sh[wv] = acc;
-    __syncthreads();
-    if (threadIdx.x == 0) part[blockIdx.x] = sh[0] + sh[1] + sh[2] + sh[3];
+    block_part(acc, sh, part);
 }
 
 // out[i] = the sum of product i's nblk partials, one wavefront per product (four per block)
@@ -845,15 +925,80 @@ k_adj_msum(int nv, int nblk, const double *__restrict__ part, double *__restrict
 
 __global__ void __launch_bounds__(256)
 k_adj_maxpy(long len, int nv, double a, double cs, const double *__restrict__ V,
-            const double *__restrict__ c, double *__restrict__ w, const int *__restrict__ gate)
+            const double *__restrict__ c, double *__restrict__ w)
 {
-    if (gate && *gate == 0) return;
     for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < len;
          e += (long)gridDim.x * blockDim.x) {
         double acc = 0.0;
         for (int i = 0; i < nv; ++i) acc += c[i] * V[(long)i * len + e];
         w[e] = a * w[e] + cs * acc;
     }
+}
+
+// w -= sum_i red[i] V_i, and gate = 1 when less than the fraction keep of w's square norm
+// red[nv] survives the projections red[0..nv-1] (then it is projected a second time; keep = 1/2
+// is the DGKS test, 0 never projects twice)
+__global__ void __launch_bounds__(256)
+k_adj_project(long len, int nv, const double *__restrict__ V, const double *__restrict__ red,
+              double keep, double *__restrict__ w, int *__restrict__ gate)
+{
+    if (blockIdx.x == 0 && threadIdx.x < 64) {
+        double s2 = 0.0;
+        for (int i = threadIdx.x; i < nv; i += 64) s2 += red[i] * red[i];
+        s2 = wave_sum(s2);
+        if (threadIdx.x == 0) *gate = (red[nv] - s2 < keep * red[nv]) ? 1 : 0;
+    }
+    for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < len;
+         e += (long)gridDim.x * blockDim.x) {
+        double acc = 0.0;
+        for (int i = 0; i < nv; ++i) acc += red[i] * V[(long)i * len + e];
+        w[e] = w[e] - acc;
+    }
+}
+
+// the second projection, where the gate asks for it, and the partials of w . w
+__global__ void __launch_bounds__(256)
+k_adj_project2(long len, int nv, const double *__restrict__ V, const double *__restrict__ red2,
+               const int *__restrict__ gate, double *__restrict__ w, double *__restrict__ part)
+{
+    __shared__ double sh[4];
+    const bool twice = *gate != 0;
+    double a2 = 0.0;
+    for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < len;
+         e += (long)gridDim.x * blockDim.x) {
+        double v = w[e];
+        if (twice) {
+            double acc = 0.0;
+            for (int i = 0; i < nv; ++i) acc += red2[i] * V[(long)i * len + e];
+            v = v - acc;
+            w[e] = v;
+        }
+        a2 += v * v;
+    }
+    block_part(a2, sh, part);
+}
+
+// w /= its norm (part: the partials of w . w), and the column to the host: the nv products of
+// both projections and the square norm
+__global__ void __launch_bounds__(256)
+k_adj_column(long len, int nv, int m, const double *__restrict__ part,
+             const double *__restrict__ red, const double *__restrict__ red2,
+             double *__restrict__ w, double *__restrict__ host)
+{
+    const double n2 = part_sum(part);
+    if (blockIdx.x == 0) {
+        for (int i = threadIdx.x; i < nv; i += blockDim.x) {
+            host[i] = red[i];
+            host[m + 2 + i] = red2[i];
+        }
+        if (threadIdx.x == 0) host[2 * (m + 2)] = n2;
+    }
+    const double hn = sqrt(n2);
+    if (!(hn > 0.0)) return;
+    const double sc = 1.0 / hn;
+    for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < len;
+         e += (long)gridDim.x * blockDim.x)
+        w[e] = sc * w[e];
 }
 
 // y = a*x + b*y + g*z (any of x, z may be null)
@@ -890,8 +1035,6 @@ static unsigned nblk(long n, long cap = 2048)
     long b = (n + 255) / 256;
     return (unsigned)(b > cap ? cap : b);
 }
-
-constexpr int ADJ_DOT_BLOCKS = 512;
 
 // nv dot products of w with V[0..nv-1] into out[0..nv-1] (device); with a gate, nothing is
 // computed (and zeros are written) when *gate == 0
@@ -950,50 +1093,57 @@ void adj_build(AdjCtx &c)
     c.sm_binv = c.sm_on ? 1.0 / beta : 0.0;
 }
 
+static void op_launch(AdjCtx &c, const double *in, const double *part, const double *b,
+                      double *out)
+{
+    hipLaunchKernelGGL(k_adj_op, dim3((c.d.jm + 63) / 64, c.d.km), dim3(64), 0, c.sm, c.d, c.jac,
+                       c.across, in, part, (const double *)c.g[0], b, out);
+}
+
 // out = F_q^T in
 void adj_apply_jt(AdjCtx &c, const double *in, double *out)
 {
-    const Dims &d = c.d;
-    hipLaunchKernelGGL(k_adj_jtv, dim3((d.jm + 255) / 256, d.km), dim3(256), 0, c.sm, d, c.jac,
-                       in, out);
-    if (c.npair > 0)
-        hipLaunchKernelGGL(k_adj_wake_t, dim3((c.npair + 63) / 64), dim3(64), 0, c.sm, d, c.npair,
-                           c.pairs, in, out);
+    op_launch(c, in, nullptr, nullptr, out);
 }
 
-// out = -F_q^T in - (in . F_c) CL_q
+// out = -F_q^T in - (in . F_c) CL_q, or b less that; part: the partials of in . F_c, if they
+// are there already
+static void apply_op(AdjCtx &c, const double *in, const double *part, const double *b, double *out)
+{
+    if (!part) {
+        hipLaunchKernelGGL(k_adj_dot1, dim3(ADJ_DOT_BLOCKS), dim3(256), 0, c.sm, 3 * c.d.N,
+                           (const double *)c.fc, in, c.part);
+        part = c.part;
+    }
+    op_launch(c, in, part, b, out);
+}
+
 void adj_apply_op(AdjCtx &c, const double *in, double *out)
 {
-    const Dims &d = c.d;
-    hipLaunchKernelGGL(k_adj_jtv, dim3((d.jm + 255) / 256, d.km), dim3(256), 0, c.sm, d, c.jac,
-                       in, out);
-    if (c.npair > 0)
-        hipLaunchKernelGGL(k_adj_wake_t, dim3((c.npair + 63) / 64), dim3(64), 0, c.sm, d, c.npair,
-                           c.pairs, in, out);
-    mdot(c, c.fc, 1, in, c.red);
-    hipLaunchKernelGGL(k_adj_negate_rank1, dim3(nblk(3 * d.N)), dim3(256), 0, c.sm, 3 * d.N,
-                       (const double *)c.red, (const double *)c.g[0], out);
+    apply_op(c, in, nullptr, nullptr, out);
 }
 
-// out = P^T in = (targets cleared) M^-T W^T in  +  (targets only) in
+// out = P^T in = (targets cleared) M^-T W^T in  +  (targets only) in; leaves the partials of
+// F_c . out in c.part
 void adj_apply_prec_t(AdjCtx &c, const double *in, double *out)
 {
     const Dims &d = c.d;
     const long N = d.N;
-    hipLaunchKernelGGL(k_adj_mask_targets, dim3(nblk(3 * N)), dim3(256), 0, c.sm, N, c.rtype, 0,
-                       in, c.t1);
-    if (c.npair > 0)
-        hipLaunchKernelGGL(k_adj_wake_wt, dim3((c.npair + 63) / 64), dim3(64), 0, c.sm, d,
-                           c.npair, c.pairs, c.inv, in, c.t1);
+    const bool turned = c.lr && c.nksp > 0;   // the eta sweeps' transposes come first
+    if (turned)
+        hipLaunchKernelGGL(k_adj_wake_in_t, dim3((d.jm + 31) / 32, (d.km + 31) / 32, 3),
+                           dim3(32, 8), 0, c.sm, d, c.rtype, c.across, in, c.lrv.at);
+    else
+        hipLaunchKernelGGL(k_adj_wake_in, dim3(nblk(N)), dim3(256), 0, c.sm, N, d.jm, c.rtype,
+                           c.across, in, c.lr ? c.lrv.a : c.t1);
     const WakePairs none{0, nullptr};
     if (c.lr)
-        launch_lrelax_scan_t<double>(c.sm, d, c.njsp, c.nksp, c.dp.underr, c.t1, c.t2, c.lr_t,
-                                     c.lrv);
+        launch_lrelax_scan_t<double>(c.sm, d, c.njsp, c.nksp, c.dp.underr, c.t2, c.lr_t, c.lrv);
     else
         launch_lusgs3<double>(c.sm, d, c.ws, none, c.q, c.t2, c.t1, c.tb[0], c.tb[1], c.tb[2],
                               c.tb[3], c.tb[4], nullptr, false);
-    hipLaunchKernelGGL(k_adj_merge_targets, dim3(nblk(3 * N)), dim3(256), 0, c.sm, N, c.rtype,
-                       in, c.t2, out);
+    hipLaunchKernelGGL(k_adj_merge, dim3(ADJ_DOT_BLOCKS), dim3(256), 0, c.sm, N, c.rtype, in,
+                       (const double *)c.t2, out, (const double *)c.fc, c.part);
 }
 
 // out = P in = W M^-1 (targets cleared) in  +  (targets only) in: the primal's own update
@@ -1016,38 +1166,18 @@ void adj_apply_prec(AdjCtx &c, const double *in, double *out)
                            c.pairs, out, in, out);
 }
 
-// gate = 1 when less than the fraction keep of the square norm red[n] of the vector survives
-// the projections red[0..n-1] (then it is projected a second time; keep = 1/2 is the DGKS
-// test, 0 never projects twice)
-__global__ void k_adj_dgks(int n, const double *__restrict__ red, double keep, int *__restrict__ gate)
-{
-    double s2 = 0.0;
-    for (int i = threadIdx.x; i < n; i += 64) s2 += red[i] * red[i];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) s2 += __shfl_xor(s2, off, 64);
-    if (threadIdx.x == 0) *gate = (red[n] - s2 < keep * red[n]) ? 1 : 0;
-}
-
-// out += u * red[0] * binv
-__global__ void __launch_bounds__(256)
-k_adj_sm_add(long len, const double *__restrict__ red, double binv, const double *__restrict__ u,
-             double *__restrict__ out)
-{
-    const double a = red[0] * binv;
-    for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < len;
-         e += (long)gridDim.x * blockDim.x)
-        out[e] += a * u[e];
-}
-
-// the preconditioner GMRES uses: P^T with the rank-one correction (see the file header)
-static void adj_apply_prec_gm(AdjCtx &c, const double *in, double *out)
+// the preconditioner GMRES uses: P^T with the rank-one correction (see the file header), into
+// out or, with sum, added to it (out is scratch then); returns the partials of F_c . result
+static const double *prec_gm(AdjCtx &c, const double *in, double *out, double *sum)
 {
     adj_apply_prec_t(c, in, out);
-    if (!c.sm_on) return;
-    const long len = 3 * c.d.N;
-    mdot(c, c.fc, 1, out, c.red);
-    hipLaunchKernelGGL(k_adj_sm_add, dim3(nblk(len)), dim3(256), 0, c.sm, len,
-                       (const double *)c.red, c.sm_binv, (const double *)c.smu, out);
+    if (!c.sm_on && !sum) return c.part;
+    double *pout = c.part + ADJ_DOT_BLOCKS;
+    hipLaunchKernelGGL(k_adj_rank1, dim3(ADJ_DOT_BLOCKS), dim3(256), 0, c.sm, 3 * c.d.N,
+                       (const double *)c.part, c.sm_binv,
+                       c.sm_on ? (const double *)c.smu : nullptr, out, sum, (const double *)c.fc,
+                       pout);
+    return pout;
 }
 
 // The GMRES preconditioner: psteps steps of the transposed update Q as a stationary
@@ -1055,18 +1185,15 @@ static void adj_apply_prec_gm(AdjCtx &c, const double *in, double *out)
 // sum_i (I - Q Op)^i Q, a fixed linear operator.  Each step costs one more Q and Op and cuts
 // the GMRES iterations about as much (945x241: 4140 / 3455 with one step, 1961 / 1761 with
 // two, 1301 / 1254 with three).
-static void adj_apply_prec_poly(AdjCtx &c, const double *in, double *out)
+// Returns the partials of F_c . out.
+static const double *prec_poly(AdjCtx &c, const double *in, double *out)
 {
-    adj_apply_prec_gm(c, in, out);
-    const long len = 3 * c.d.N;
+    const double *part = prec_gm(c, in, out, nullptr);
     for (int st = 1; st < c.psteps; ++st) {
-        adj_apply_op(c, out, c.pk1);
-        hipLaunchKernelGGL(k_adj_axpby, dim3(nblk(len)), dim3(256), 0, c.sm, len, 1.0, in, -1.0,
-                           c.pk1, 0.0, (const double *)nullptr);
-        adj_apply_prec_gm(c, c.pk1, c.pk2);
-        hipLaunchKernelGGL(k_adj_axpby, dim3(nblk(len)), dim3(256), 0, c.sm, len, 1.0, c.pk2, 1.0,
-                           out, 0.0, (const double *)nullptr);
+        apply_op(c, out, part, in, c.pk1);
+        part = prec_gm(c, c.pk1, c.pk2, out);
     }
+    return part;
 }
 
 // ||v||_2 on the host
@@ -1098,7 +1225,7 @@ int adj_gmres(AdjCtx &c, const double *b, double *x, int maxit, double tol, doub
                        (const double *)nullptr);
     int it = 0;
     double res = bn;
-    std::vector<double> H((m + 1) * m), cs(m), sn(m), gv(m + 1), h(m + 1), h2(m + 1), y(m);
+    std::vector<double> H((m + 1) * m), cs(m), sn(m), gv(m + 1), h(m + 1), y(m);
     while (it < maxit) {
         res = norm2(c, c.w);
         if (res <= tol * bn) break;
@@ -1110,29 +1237,24 @@ int adj_gmres(AdjCtx &c, const double *b, double *x, int maxit, double tol, doub
         int jl = -1;
         for (int j = 0; j < m && it < maxit; ++j) {
             double *vj = c.V + (long)j * len, *vn = c.V + (long)(j + 1) * len;
-            adj_apply_prec_poly(c, vj, c.z);
-            adj_apply_op(c, c.z, vn);
+            apply_op(c, c.z, prec_poly(c, vj, c.z), nullptr, vn);
             // classical Gram-Schmidt; its products with the basis and vn . vn in one pass (vn
             // is V_(j+1)), then a second pass only where the first cancelled more than half of
             // vn's square norm (the DGKS test, decided on the device)
             mdot(c, c.V, j + 2, vn, c.red);
-            hipLaunchKernelGGL(k_adj_dgks, dim3(1), dim3(64), 0, c.sm, j + 1,
-                               (const double *)c.red, c.reorth, c.gate);
-            hipLaunchKernelGGL(k_adj_maxpy, dim3(nb), dim3(256), 0, c.sm, len, j + 1, 1.0, -1.0,
-                               (const double *)c.V, (const double *)c.red, vn,
-                               (const int *)nullptr);
-            (void)hipMemcpyAsync(h.data(), c.red, sizeof(double) * (j + 1), hipMemcpyDeviceToHost, c.sm);
+            hipLaunchKernelGGL(k_adj_project, dim3(nb), dim3(256), 0, c.sm, len, j + 1,
+                               (const double *)c.V, (const double *)c.red, c.reorth, vn, c.gate);
             mdot(c, c.V, j + 1, vn, c.red2, c.gate);
-            hipLaunchKernelGGL(k_adj_maxpy, dim3(nb), dim3(256), 0, c.sm, len, j + 1, 1.0, -1.0,
-                               (const double *)c.V, (const double *)c.red2, vn,
-                               (const int *)c.gate);
-            (void)hipMemcpyAsync(h2.data(), c.red2, sizeof(double) * (j + 1), hipMemcpyDeviceToHost, c.sm);
-            const double hn = norm2(c, vn);   // synchronises
-            for (int i = 0; i <= j; ++i) h[i] += h2[i];
+            hipLaunchKernelGGL(k_adj_project2, dim3(ADJ_DOT_BLOCKS), dim3(256), 0, c.sm, len,
+                               j + 1, (const double *)c.V, (const double *)c.red2,
+                               (const int *)c.gate, vn, c.part);
+            hipLaunchKernelGGL(k_adj_column, dim3(nb), dim3(256), 0, c.sm, len, j + 1, m,
+                               (const double *)c.part, (const double *)c.red,
+                               (const double *)c.red2, vn, c.pin_dev);
+            (void)hipStreamSynchronize(c.sm);
+            const double hn = std::sqrt(c.pin[2 * (m + 2)]);
+            for (int i = 0; i <= j; ++i) h[i] = c.pin[i] + c.pin[m + 2 + i];
             h[j + 1] = hn;
-            if (hn > 0.0)
-                hipLaunchKernelGGL(k_adj_axpby, dim3(nb), dim3(256), 0, c.sm, len, 0.0,
-                                   (const double *)nullptr, 1.0 / hn, vn, 0.0, (const double *)nullptr);
             // Givens rotations of the new column
             for (int i = 0; i < j; ++i) {
                 const double t = cs[i] * h[i] + sn[i] * h[i + 1];
@@ -1160,15 +1282,12 @@ int adj_gmres(AdjCtx &c, const double *b, double *x, int maxit, double tol, doub
         }
         (void)hipMemcpyAsync(c.red, y.data(), sizeof(double) * (jl + 1), hipMemcpyHostToDevice, c.sm);
         hipLaunchKernelGGL(k_adj_maxpy, dim3(nb), dim3(256), 0, c.sm, len, jl + 1, 0.0, 1.0,
-                           (const double *)c.V, (const double *)c.red, c.t1b,
-                           (const int *)nullptr);
-        adj_apply_prec_poly(c, c.t1b, c.z);
+                           (const double *)c.V, (const double *)c.red, c.t1b);
+        (void)prec_poly(c, c.t1b, c.z);
         hipLaunchKernelGGL(k_adj_axpby, dim3(nb), dim3(256), 0, c.sm, len, 1.0, c.z, 1.0, x, 0.0,
                            (const double *)nullptr);
         // true residual r = b - Op x
-        adj_apply_op(c, x, c.w);
-        hipLaunchKernelGGL(k_adj_axpby, dim3(nb), dim3(256), 0, c.sm, len, 1.0, b, -1.0, c.w, 0.0,
-                           (const double *)nullptr);
+        apply_op(c, x, nullptr, b, c.w);
     }
     res = norm2(c, c.w);
     if (rel) *rel = res / bn;

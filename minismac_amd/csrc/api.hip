@@ -83,6 +83,7 @@ struct smac_handle {
     AdjCtx adj = {};
     LusgsWs adj_ws = {};
     LusgsWs adj_ws2 = {};      // the second adjoint solve's (LU-SGS preconditioner)
+    double *adj_pin = nullptr; // host memory: the two solves' GMRES columns
     AdjCtx adj2 = {};          // the second adjoint solve's work vectors (the rest is adj's)
     std::vector<void *> lws_allocs;
     Walls walls = {};
@@ -197,6 +198,7 @@ static void free_handle(smac_handle *h)
     for (hipEvent_t e : {h->ev_q, h->ev_sa_read, h->ev_sa_done, h->ev_force})
         if (e) (void)hipEventDestroy(e);
     if (h->pin) (void)hipHostFree(h->pin);
+    if (h->adj_pin) (void)hipHostFree(h->adj_pin);
     delete h;
 }
 
@@ -808,7 +810,7 @@ smac_status smac_get_array(smac_handle *h, const char *name, double *out)
 
 // row types of the steady equations (the BC rows in file order, then the wake-cut targets)
 static smac_status adj_row_types(smac_handle *h, std::vector<signed char> &rt,
-                                 std::vector<int> &inv)
+                                 std::vector<int> &across)
 {
     const int jm = h->d.jm, km = h->d.km;
     rt.assign(h->d.N, (signed char)-1);
@@ -826,15 +828,15 @@ static smac_status adj_row_types(smac_handle *h, std::vector<signed char> &rt,
     std::vector<int> pr(2 * np);
     if (np > 0 && hipMemcpy(pr.data(), h->pairs, 2 * np * sizeof(int), hipMemcpyDeviceToHost) != hipSuccess)
         return fail(SMAC_ERR_HIP, "reading the wake pairs failed");
-    inv.assign(np, -1);
+    across.assign(jm, -1);
     for (int i = 0; i < np; ++i) {
         const long p = pr[2 * i];
         if (rt[p] != -1)
             return fail(SMAC_ERR_BC, "a wake-cut point also carries a BC row: not a steady system the adjoint covers");
         rt[p] = 5;
         for (int i2 = 0; i2 < np; ++i2)
-            if (pr[2 * i2 + 1] == pr[2 * i]) inv[i] = i2;
-        if (inv[i] < 0) return fail(SMAC_ERR_BC, "wake cut: a target that is no pair's partner");
+            if (pr[2 * i2 + 1] == pr[2 * i]) across[p] = pr[2 * i2];
+        if (across[p] < 0) return fail(SMAC_ERR_BC, "wake cut: a target that is no pair's partner");
     }
     for (long p = 0; p < h->d.N; ++p)
         if (rt[p] < 0) return fail(SMAC_ERR_BC, "a boundary point without a BC row or wake-cut relation");
@@ -848,16 +850,16 @@ static smac_status adj_prepare(smac_handle *h, int m)
         AdjCtx &c = h->adj;
         c = AdjCtx{};
         std::vector<signed char> rt;
-        std::vector<int> inv;
-        smac_status rc = adj_row_types(h, rt, inv);
+        std::vector<int> across;
+        smac_status rc = adj_row_types(h, rt, across);
         if (rc) return rc;
         signed char *rtd = nullptr;
-        int *invd = nullptr;
-        if ((rc = dalloc(h, &rtd, N)) || (rc = dalloc(h, &invd, inv.size() + 1))) return rc;
+        int *acd = nullptr;
+        if ((rc = dalloc(h, &rtd, N)) || (rc = dalloc(h, &acd, across.size()))) return rc;
         HIP_TRY(hipMemcpy(rtd, rt.data(), N, hipMemcpyHostToDevice));
-        if (!inv.empty()) HIP_TRY(hipMemcpy(invd, inv.data(), inv.size() * sizeof(int), hipMemcpyHostToDevice));
+        HIP_TRY(hipMemcpy(acd, across.data(), across.size() * sizeof(int), hipMemcpyHostToDevice));
         c.rtype = rtd;
-        c.inv = invd;
+        c.across = acd;
         double **v3[] = {&c.lam[0], &c.lam[1], &c.g[0], &c.g[1], &c.fc, &c.fa, &c.w, &c.z,
                          &c.t1, &c.t2, &c.t1b, &c.fb, &c.smu, &c.pk1, &c.pk2};
         if ((rc = dalloc(h, &c.jac, 81 * N))) return rc;
@@ -901,6 +903,18 @@ static smac_status adj_prepare(smac_handle *h, int m)
             for (double **pp : lv)
                 if ((rc = dalloc(h, pp, 3 * N))) return rc;
         }
+        if (h->adj_pin) (void)hipHostFree(h->adj_pin);
+        h->adj_pin = nullptr;
+        const size_t col = 2 * (m + 2) + 1;
+        double *dev = nullptr;
+        if (hipHostMalloc((void **)&h->adj_pin, 2 * col * 8, hipHostMallocCoherent | hipHostMallocMapped) !=
+                hipSuccess ||
+            hipHostGetDevicePointer((void **)&dev, h->adj_pin, 0) != hipSuccess)
+            return fail(SMAC_ERR_HIP, "hipHostMalloc / hipHostGetDevicePointer failed (adjoint)");
+        c.pin = h->adj_pin;
+        c.pin_dev = dev;
+        c2.pin = h->adj_pin + col;
+        c2.pin_dev = dev + col;
         h->adj_m = m;
         h->adj_ready = true;
     }
@@ -976,6 +990,7 @@ smac_status smac_adjoint(smac_handle *h, int nshape, const double *dx, const dou
         c2.V = b2.V; c2.w = b2.w; c2.z = b2.z; c2.t1 = b2.t1; c2.t2 = b2.t2; c2.t1b = b2.t1b;
         c2.pk1 = b2.pk1; c2.pk2 = b2.pk2; c2.part = b2.part; c2.red = b2.red;
         c2.red2 = b2.red2; c2.gate = b2.gate; c2.lrv = b2.lrv;
+        c2.pin = b2.pin; c2.pin_dev = b2.pin_dev;
         c2.ws = h->adj_ws2;
     }
     HIP_TRY(hipStreamSynchronize(h->stream));   // the operator and factors are built

@@ -426,7 +426,7 @@ static int lines_per_group(int nline, bool twist) { return nline * (twist ? 2 : 
 // the first wait, pairs of points in one load, the scan without branches, and its distances 1
 // and 32 as DPP move and half-wave swap instead of crossbar reads, a 945x241 FP64 xi colour
 // takes 18.6 us (28.6 before) and an eta colour 16.4 (17.9); FP32 at 705x173 11.7 (14.1) and 9.2
-// (10.1); one colour of the 203x47 transposed sweeps 7.7 (8.5).
+// (10.1).
 
 // one doubling step: the lane's map after that of OFF lanes before
 template <typename AT, int NEQ, bool FWD, int OFF>
@@ -563,11 +563,32 @@ SMAC_DEV void load_planes(T (&x)[PP][NB], const T *p, long N)
     }
 }
 
-template <typename LT, int NEQ, int NT, int PP, bool TWIST>
+// acc += block x, where there is such a line
+template <typename LT, int NEQ>
+SMAC_DEV void lr_terms(double *acc, bool has, const LT *b, const double *x)
+{
+#pragma unroll
+    for (int m = 0; m < NEQ; ++m) {
+        double t = acc[m];
+#pragma unroll
+        for (int k = 0; k < NEQ; ++k) t += (double)b[m + NEQ * k] * x[k];
+        acc[m] = has ? t : acc[m];
+    }
+}
+
+// A colour step of the transposed sweeps (TRANS; see below): dq is z, s is not read
+struct LrTStep {
+    double *a, *sbar;
+    double w;
+    int spread;   // the other colour's z belongs to the step before: a takes its terms first
+    int begin;    // the colour's first step: sbar starts from zero
+};
+
+template <typename LT, int NEQ, int NT, int PP, bool TWIST, bool TRANS>
 __global__ void __launch_bounds__(NT)
 k_lr_sweep(int nline, int len, long N, int count, int first, int step, double underr,
            int assign, int couple, double *__restrict__ dq, const double *__restrict__ s,
-           const LT *__restrict__ op)
+           const LT *__restrict__ op, LrTStep ts)
 {
     using AT = LT;
     constexpr int NB = NEQ * NEQ, NW = NT / 64;
@@ -591,7 +612,7 @@ k_lr_sweep(int nline, int len, long N, int count, int first, int step, double un
     };
     for (int idx = (int)blockIdx.x; idx < count; idx += (int)gridDim.x) {
         const int l = (first + idx * step) % nline;
-        const bool hm = couple && l > 0, hp = couple && l < nline - 1;
+        const bool hm = (TRANS || couple) && l > 0, hp = (TRANS || couple) && l < nline - 1;
         AT mmat[PP][NB];               // M (Ma at mid)
         AT bv[PP][NEQ];                // T^-1 r
         AT w[PP][NEQ];                 // y (i < mid) or z (i > mid); z_(mid+1), then x_mid, at
@@ -601,14 +622,17 @@ k_lr_sweep(int nline, int len, long N, int count, int first, int step, double un
         // branches every load is in flight before the first is waited for.
         const long lo = (long)l * len + (t * PP < len ? t * PP : len - 1);
         AT bi[PP][NB];
-        double r[PP][NEQ];
+        double r[PP][NEQ], sb[PP][NEQ];
         load_planes(bi, pB + lo, N);
         load_planes(mmat, pM + lo, N);
 #pragma unroll
         for (int u = 0; u < PP; ++u)
 #pragma unroll
-            for (int n = 0; n < NEQ; ++n) r[u][n] = s[n * N + nat(l, u)];
-        if (couple) {
+            for (int n = 0; n < NEQ; ++n) {
+                r[u][n] = (TRANS ? ts.a : s)[n * N + nat(l, u)];
+                if constexpr (TRANS) sb[u][n] = ts.begin ? 0.0 : ts.sbar[n * N + nat(l, u)];
+            }
+        if (TRANS ? ts.spread : couple) {
             AT om[PP][NB], op_[PP][NB];
             double xm[PP][NEQ], xp[PP][NEQ];
             load_planes(om, pOm + lo, N);
@@ -620,21 +644,32 @@ k_lr_sweep(int nline, int len, long N, int count, int first, int step, double un
                     xm[u][n] = dq[n * N + nat(hm ? l - 1 : l, u)];
                     xp[u][n] = dq[n * N + nat(hp ? l + 1 : l, u)];
                 }
+            if constexpr (TRANS) {
 #pragma unroll
-            for (int u = 0; u < PP; ++u) {
+                for (int u = 0; u < PP; ++u) {
+                    double acc[NEQ] = {};
+                    lr_terms<LT, NEQ>(acc, hm, om[u], xm[u]);
+                    lr_terms<LT, NEQ>(acc, hp, op_[u], xp[u]);
 #pragma unroll
-                for (int m = 0; m < NEQ; ++m) {
-                    double b = (double)om[u][m] * xm[u][0];
-#pragma unroll
-                    for (int n = 1; n < NEQ; ++n) b = b + (double)om[u][m + NEQ * n] * xm[u][n];
-                    r[u][m] = hm ? r[u][m] - b : r[u][m];
+                    for (int m = 0; m < NEQ; ++m) r[u][m] -= ts.w * acc[m];
                 }
+            } else {
 #pragma unroll
-                for (int m = 0; m < NEQ; ++m) {
-                    double b = (double)op_[u][m] * xp[u][0];
+                for (int u = 0; u < PP; ++u) {
 #pragma unroll
-                    for (int n = 1; n < NEQ; ++n) b = b + (double)op_[u][m + NEQ * n] * xp[u][n];
-                    r[u][m] = hp ? r[u][m] - b : r[u][m];
+                    for (int m = 0; m < NEQ; ++m) {
+                        double b = (double)om[u][m] * xm[u][0];
+#pragma unroll
+                        for (int n = 1; n < NEQ; ++n) b = b + (double)om[u][m + NEQ * n] * xm[u][n];
+                        r[u][m] = hm ? r[u][m] - b : r[u][m];
+                    }
+#pragma unroll
+                    for (int m = 0; m < NEQ; ++m) {
+                        double b = (double)op_[u][m] * xp[u][0];
+#pragma unroll
+                        for (int n = 1; n < NEQ; ++n) b = b + (double)op_[u][m + NEQ * n] * xp[u][n];
+                        r[u][m] = hp ? r[u][m] - b : r[u][m];
+                    }
                 }
             }
         }
@@ -678,7 +713,8 @@ k_lr_sweep(int nline, int len, long N, int count, int first, int step, double un
                 }
             },
             lf, lane, wv);
-        // the -C / -D planes (Mc at mid), read only now: phase 1 does not need them
+        // the -C / -D planes (Mc at mid), read only now: phase 1 does not need them (loaded with
+        // the others, 945x241 FP64 colours take 19.2 and 17.0 us instead of 18.6 and 16.4)
         AT cm[PP][NB];
         load_planes(cm, pC + lo, N);
         __syncthreads();   // phase 1's wave totals have been read; y_(mid-1) is in xch
@@ -747,6 +783,12 @@ k_lr_sweep(int nline, int len, long N, int count, int first, int step, double un
 #pragma unroll
                 for (int n = 0; n < NEQ; ++n) {
                     const double xd = (double)w[u][n];
+                    if constexpr (TRANS) {
+                        dq[n * N + o] = xd;
+                        ts.sbar[n * N + o] = sb[u][n] + ts.w * xd;
+                        ts.a[n * N + o] = r[u][n] * (1.0 - ts.w);
+                        continue;
+                    }
                     const double dold = assign ? 0.0 : dq[n * N + o];
                     const double nv = assign ? xd : dold + underr * (xd - dold);
                     dq[n * N + o] = nv;
@@ -973,16 +1015,22 @@ __global__ void k_zero(double *__restrict__ a, long n)
 
 // ------------------------------------------------------------------------------------------
 
+// Threads and points per line: a line of up to 64 points stays within one wave, which has no
+// waves to wait for or chain (47 points FP64: 6.4 us a transposed step against 7.8 in 256
+// threads); pairs of points keep lines of up to 1024 at two waves per SIMD.
 // twist: the operand planes hold the twisted factorisation (the reference-order walk always
 // takes the plain one)
-template <typename LT, int NEQ, bool SEQ>
+enum SweepForm { SWEEP_COLOUR, SWEEP_WALK, SWEEP_TRANSPOSED };
+
+template <typename LT, int NEQ, SweepForm FORM>
 static void sweep_launch(hipStream_t sm, int nline, int len, long N, int count, int first,
                          int step, double underr, int assign, double *dq, const double *s,
-                         const LT *op, int couple, bool twist)
+                         const LT *op, int couple, bool twist, const LrTStep &ts = {})
 {
 #define SWT(LAUNCH)                                                                             \
     do {                                                                                       \
-        if (len <= 256) LAUNCH(256, 1);                                                        \
+        if (len <= 64) LAUNCH(64, 1);                                                          \
+        else if (len <= 256) LAUNCH(256, 1);                                                   \
         else if (len <= 512) LAUNCH(512, 1);                                                   \
         else if (len <= 1024) LAUNCH(512, 2);                                                  \
         else LAUNCH(1024, 2);                                                                  \
@@ -990,17 +1038,20 @@ static void sweep_launch(hipStream_t sm, int nline, int len, long N, int count, 
 #define WALK(NT, PPV)                                                                           \
     hipLaunchKernelGGL((k_lr_walk<LT, NEQ, NT, PPV>), dim3(1), dim3(NT), 0, sm, nline, len, N,  \
                        count, first, step, underr, assign, dq, s, op)
-#define TWISTED(NT, PPV)                                                                        \
-    hipLaunchKernelGGL((k_lr_sweep<LT, NEQ, NT, PPV, true>), dim3(count), dim3(NT), 0, sm,      \
-                       nline, len, N, count, first, step, underr, assign, couple, dq, s, op)
-#define PLAIN(NT, PPV)                                                                          \
-    hipLaunchKernelGGL((k_lr_sweep<LT, NEQ, NT, PPV, false>), dim3(count), dim3(NT), 0, sm,     \
-                       nline, len, N, count, first, step, underr, assign, couple, dq, s, op)
-    if constexpr (SEQ) SWT(WALK);
+#define COLOUR(NT, PPV, TW, TR)                                                                 \
+    hipLaunchKernelGGL((k_lr_sweep<LT, NEQ, NT, PPV, TW, TR>), dim3(count), dim3(NT), 0, sm,    \
+                       nline, len, N, count, first, step, underr, assign, couple, dq, s, op, ts)
+#define TWISTED(NT, PPV) COLOUR(NT, PPV, true, false)
+#define PLAIN(NT, PPV) COLOUR(NT, PPV, false, false)
+#define TRANSPOSED(NT, PPV) COLOUR(NT, PPV, false, true)
+    if constexpr (FORM == SWEEP_WALK) SWT(WALK);
+    else if constexpr (FORM == SWEEP_TRANSPOSED) SWT(TRANSPOSED);
     else if (twist) SWT(TWISTED);
     else SWT(PLAIN);
+#undef TRANSPOSED
 #undef PLAIN
 #undef TWISTED
+#undef COLOUR
 #undef WALK
 #undef SWT
 }
@@ -1012,14 +1063,14 @@ static void sweep(hipStream_t sm, int nline, int len, long N, int nsweep, bool z
                   double underr, double *dq, const double *s, const LT *op)
 {
     if (zebra) {
-        sweep_launch<LT, NEQ, false>(sm, nline, len, N, (nline + 1) / 2, 0, 2, underr, 0, dq, s,
+        sweep_launch<LT, NEQ, SWEEP_COLOUR>(sm, nline, len, N, (nline + 1) / 2, 0, 2, underr, 0, dq, s,
                                      op, 1, twist);
-        sweep_launch<LT, NEQ, false>(sm, nline, len, N, nline / 2, 1, 2, underr, 0, dq, s, op, 1,
+        sweep_launch<LT, NEQ, SWEEP_COLOUR>(sm, nline, len, N, nline / 2, 1, 2, underr, 0, dq, s, op, 1,
                                      twist);
         return;
     }
     const bool rev = (nsweep / 2) * 2 == nsweep;
-    sweep_launch<LT, NEQ, true>(sm, nline, len, N, nline, rev ? nline - 1 : 0, rev ? -1 : 1,
+    sweep_launch<LT, NEQ, SWEEP_WALK>(sm, nline, len, N, nline, rev ? nline - 1 : 0, rev ? -1 : 1,
                                 underr, 0, dq, s, op, 1, false);
 }
 
@@ -1086,83 +1137,84 @@ void launch_lrelax_scan(hipStream_t sm, const Dims &d, const DevParams &prm, int
 // where Om'_m = (Op_(m-1))^T and Op'_m = (Om_(m+1))^T are again the transposed system's
 // blocks to the neighbouring lines at the point.
 
+//
+// A step's line solves are one launch: a line first takes the terms of the z that the step
+// before left on its neighbours (LrTStep::spread), is solved, and adds to its sbar and scales
+// its a from what the workgroup holds.  The terms that the last step leaves to the other
+// colour are taken on the way back to the natural layout (k_lr_tback).  A pair of kernels per
+// step, solve and spread, took 7.7 + 4.9 us at 203x47; a xi step takes 8.3, an eta step 6.4.
+
+// after the last eta step: out = sbar and, with planes 3..5, a = at less the terms of z on the
+// lines of odd index, eta-major to natural
 template <typename LT>
 __global__ void __launch_bounds__(256)
-k_lr_tspread(int nline, int len, long N, int par, double w, double *__restrict__ a,
-             double *__restrict__ sbar, const double *__restrict__ z, const LT *__restrict__ op)
+k_lr_tback(int nline, int len, long N, double w, const double *__restrict__ at,
+           const double *__restrict__ sbar, const double *__restrict__ z,
+           const LT *__restrict__ op, double *__restrict__ a, double *__restrict__ out)
 {
+    __shared__ double tile[TT][TT + 1];
     const LT *pOm = op + 27 * N, *pOp = op + 36 * N;
-    for (long o = (long)blockIdx.x * blockDim.x + threadIdx.x; o < N;
-         o += (long)gridDim.x * blockDim.x) {
-        const int l = (int)o / len;   // o < N < 2^31: a 32-bit division
-        if ((l & 1) == par) {
+    const int m = blockIdx.z % 3;
+    const bool second = blockIdx.z >= 3;
+    const int c0 = blockIdx.x * TT, r0 = blockIdx.y * TT;
+    for (int rr = threadIdx.y; rr < TT; rr += 8) {
+        const int l = r0 + rr, c = c0 + threadIdx.x;
+        if (l >= nline || c >= len) continue;
+        const long o = (long)l * len + c;
+        double v = (second ? at : sbar)[m * N + o];
+        if (second && (l & 1)) {
+            double acc = 0.0;
 #pragma unroll
-            for (int n = 0; n < 3; ++n) {
-                sbar[n * N + o] += w * z[n * N + o];
-                a[n * N + o] *= 1.0 - w;
+            for (int k = 0; k < 3; ++k) acc += (double)pOm[(m + 3 * k) * N + o] * z[k * N + o - len];
+            if (l < nline - 1) {
+#pragma unroll
+                for (int k = 0; k < 3; ++k)
+                    acc += (double)pOp[(m + 3 * k) * N + o] * z[k * N + o + len];
             }
-            continue;
+            v -= w * acc;
         }
-        double acc[3] = {0.0, 0.0, 0.0};
-        if (l > 0) {
-#pragma unroll
-            for (int m = 0; m < 3; ++m)
-#pragma unroll
-                for (int k = 0; k < 3; ++k)
-                    acc[m] += (double)pOm[(m + 3 * k) * N + o] * z[k * N + o - len];
-        }
-        if (l < nline - 1) {
-#pragma unroll
-            for (int m = 0; m < 3; ++m)
-#pragma unroll
-                for (int k = 0; k < 3; ++k)
-                    acc[m] += (double)pOp[(m + 3 * k) * N + o] * z[k * N + o + len];
-        }
-#pragma unroll
-        for (int m = 0; m < 3; ++m) a[m * N + o] -= w * acc[m];
+        tile[rr][threadIdx.x] = v;
+    }
+    __syncthreads();
+    for (int cc = threadIdx.y; cc < TT; cc += 8) {
+        const int c = c0 + cc, l = r0 + threadIdx.x;
+        if (l < nline && c < len)
+            (second ? a : out)[m * N + (long)c * nline + l] = tile[threadIdx.x][cc];
     }
 }
 
-__global__ void k_copy(const double *__restrict__ src, double *__restrict__ dst, long n)
-{
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (long)gridDim.x * blockDim.x)
-        dst[i] = src[i];
-}
-
+// begin: sbar starts from zero with each colour's first step
 template <typename LT>
 static void tsweep(hipStream_t sm, int nline, int len, long N, int nsweep, double w, double *a,
-                   double *sbar, double *z, const LT *op)
+                   double *sbar, double *z, const LT *op, bool begin)
 {
-    const unsigned g = (unsigned)((N + 255) / 256 < 2048 ? (N + 255) / 256 : 2048);
     for (int sw = 0; sw < nsweep; ++sw)
         for (int par = 1; par >= 0; --par) {
+            const LrTStep ts{a, sbar, w, sw > 0 || par == 0, begin && sw == 0};
             const int count = par ? nline / 2 : (nline + 1) / 2;
             if (count > 0)
-                sweep_launch<LT, 3, false>(sm, nline, len, N, count, par, 2, 1.0, 1, z, a, op, 0,
-                                           false);
-            hipLaunchKernelGGL(k_lr_tspread<LT>, dim3(g), dim3(256), 0, sm, nline, len, N, par, w,
-                               a, sbar, (const double *)z, op);
+                sweep_launch<LT, 3, SWEEP_TRANSPOSED>(sm, nline, len, N, count, par, 2, 1.0, 1, z,
+                                                      nullptr, op, 0, false, ts);
         }
 }
 
 template <typename LT>
 void launch_lrelax_scan_t(hipStream_t sm, const Dims &d, int njsp, int nksp, double underr,
-                          const double *in, double *out, const LrScan &wt, const LrTWork &v)
+                          double *out, const LrScan &wt, const LrTWork &v)
 {
     const long N = d.N;
-    const unsigned g = (unsigned)((3 * N + 255) / 256 < 2048 ? (3 * N + 255) / 256 : 2048);
-    hipLaunchKernelGGL(k_copy, dim3(g), dim3(256), 0, sm, in, v.a, 3 * N);
-    hipLaunchKernelGGL(k_zero, dim3(256), dim3(256), 0, sm, out, 3 * N);
     // the eta sweeps came last in the primal: their transposes come first
     if (nksp > 0) {
-        transpose(sm, v.a, v.at, d.km, d.jm, N, 3);
-        hipLaunchKernelGGL(k_zero, dim3(256), dim3(256), 0, sm, v.st, 3 * N);
-        tsweep<LT>(sm, d.jm, d.km, N, nksp, underr, v.at, v.st, v.zt, (const LT *)wt.ope);
-        transpose(sm, v.st, out, d.jm, d.km, N, 3);
-        transpose(sm, v.at, v.a, d.jm, d.km, N, 3);
+        const LT *op = (const LT *)wt.ope;
+        tsweep<LT>(sm, d.jm, d.km, N, nksp, underr, v.at, v.st, v.zt, op, true);
+        const dim3 g((d.km + TT - 1) / TT, (d.jm + TT - 1) / TT, njsp > 0 ? 6 : 3);
+        hipLaunchKernelGGL(k_lr_tback<LT>, g, dim3(TT, 8), 0, sm, d.jm, d.km, N, underr, v.at,
+                           v.st, v.zt, op, v.a, out);
+    } else if (njsp == 0) {
+        hipLaunchKernelGGL(k_zero, dim3(256), dim3(256), 0, sm, out, 3 * N);
     }
-    if (njsp > 0) tsweep<LT>(sm, d.km, d.jm, N, njsp, underr, v.a, out, v.z, (const LT *)wt.opx);
+    if (njsp > 0)
+        tsweep<LT>(sm, d.km, d.jm, N, njsp, underr, v.a, out, v.z, (const LT *)wt.opx, nksp == 0);
 }
 
 void launch_sa_lreltur_scan(hipStream_t sm, const Dims &d, int ntjsp, const WakePairs &w,
@@ -1179,14 +1231,14 @@ void launch_sa_lreltur_scan(hipStream_t sm, const Dims &d, int ntjsp, const Wake
                        (double *)nullptr);
     for (int pass = 1; pass <= ntjsp; ++pass) {
         if (ws.zebra) {
-            sweep_launch<double, 1, false>(sm, d.km, d.jm, d.N, (d.km + 1) / 2, 0, 2, 1.0, 1,
+            sweep_launch<double, 1, SWEEP_COLOUR>(sm, d.km, d.jm, d.N, (d.km + 1) / 2, 0, 2, 1.0, 1,
                                            a.ds, a.sf, ws.sa_op, 1, true);
-            sweep_launch<double, 1, false>(sm, d.km, d.jm, d.N, d.km / 2, 1, 2, 1.0, 1, a.ds,
+            sweep_launch<double, 1, SWEEP_COLOUR>(sm, d.km, d.jm, d.N, d.km / 2, 1, 2, 1.0, 1, a.ds,
                                            a.sf, ws.sa_op, 1, true);
-            sweep_launch<double, 1, false>(sm, d.km, d.jm, d.N, 1, 0, 1, 1.0, 1, a.ds, a.sf,
+            sweep_launch<double, 1, SWEEP_COLOUR>(sm, d.km, d.jm, d.N, 1, 0, 1, 1.0, 1, a.ds, a.sf,
                                            ws.sa_op, 1, true);
         } else {
-            sweep_launch<double, 1, true>(sm, d.km, d.jm, d.N, d.km + 1, 0, 1, 1.0, 1, a.ds, a.sf,
+            sweep_launch<double, 1, SWEEP_WALK>(sm, d.km, d.jm, d.N, d.km + 1, 0, 1, 1.0, 1, a.ds, a.sf,
                                           ws.sa_op, 1, false);
         }
         launch_wake(sm, d, 1, w, a.anut, a.ds, a.sf);
@@ -1196,9 +1248,8 @@ void launch_sa_lreltur_scan(hipStream_t sm, const Dims &d, int ntjsp, const Wake
 template void launch_lr_factor3<double>(hipStream_t, const Dims &, bool, bool, bool, const double *,
                                         const double *, const double *, const double *,
                                         const double *, double *, double *);
-template void launch_lrelax_scan_t<double>(hipStream_t, const Dims &, int, int, double,
-                                           const double *, double *, const LrScan &,
-                                           const LrTWork &);
+template void launch_lrelax_scan_t<double>(hipStream_t, const Dims &, int, int, double, double *,
+                                           const LrScan &, const LrTWork &);
 template void launch_lrelax_scan<double>(hipStream_t, const Dims &, const DevParams &, int, int,
                                          int, bool, const WakePairs &, const double *, double *,
                                          double *, const double *, const double *,

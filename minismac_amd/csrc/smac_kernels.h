@@ -84,7 +84,7 @@ struct LrTWork {
 };
 template <typename LT>
 void launch_lrelax_scan_t(hipStream_t, const Dims &, int njsp, int nksp, double underr,
-                          const double *in, double *out, const LrScan &wt, const LrTWork &v);
+                          double *out, const LrScan &wt, const LrTWork &v);
 
 // lusgs.hip: LU-SGS with hyperplane (j+k = const) sweeps (ref/lusgs.f, ref/ilusol.f).
 // Workspace by hyperplanes: the operands of a few rows of one hyperplane are one chunk.
@@ -199,8 +199,8 @@ struct AdjCtx {
     double *pk1, *pk2;           // its work vectors (3 planes each)
     const signed char *rtype;    // row type per point
     int npair;
-    const int *pairs, *inv;      // wake pairs (0-based) and, per pair, the pair whose partner
-                                 // is its target
+    const int *pairs;            // wake pairs (0-based)
+    const int *across;           // per j: the target of the pair whose partner is (j,1), or -1
     int lr;                      // preconditioner: 1 the zebra line relaxation, 0 LU-SGS
     int njsp, nksp;
     DevParams dp;
@@ -211,6 +211,8 @@ struct AdjCtx {
     int sm_on;
     double *dmet, *ddj, *dxy, *fb, *fpart;
     double *part, *red, *red2;
+    volatile double *pin;        // host memory: a GMRES column (m + 2 products with the basis, as
+    double *pin_dev;             // many of the second pass, the square norm), and its device view
     int *gate;                   // second Gram-Schmidt pass wanted (device flag)
 };
 void adj_build(AdjCtx &);
