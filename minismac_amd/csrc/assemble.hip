@@ -4,15 +4,18 @@
 // the BC rows of bcmain (ref/bc.f:60-224 and the routines it calls), and resid + rhsnorm
 // (ref/step.f:613-756, 513-519).
 //
-// One thread per grid point computes everything its point needs: the flux-split face
-// Jacobians A+/A- of its four xi faces and four eta faces (the third-order flux of a face
-// reads dfp/dfm of the faces either side), the point Jacobians of its neighbours, and the
-// constant-viscosity face coefficients, then writes s (3 planes) and the five 3x3 blocks
-// (45 planes) once.  Faces are recomputed by neighbouring threads instead of being staged
-// through memory: the kernel is store-bound (48 words out per point against 8 in), so the
-// extra FP64 work is cheaper than a second pass over HBM.
+// A point needs the flux-split face Jacobians A+/A- of its four xi faces and four eta faces
+// (the third-order flux of a face reads dfp/dfm of the faces either side), the point Jacobians
+// of its neighbours and the constant-viscosity face coefficients, and writes s (3 planes) and
+// the five 3x3 blocks (45 planes) once: 448 bytes a point in FP64, which the memory takes in
+// 21 us at 945x241 and 83 at 1889x481.  A face is 230 FP64 instructions with five divisions and
+// a root.  With every point computing its eight faces the kernel was bound by those (41 and
+// 197 us, FP32-LHS batch of 1.2 M points 242); b_assemble below computes each face about once
+// (30, 117 and 169).
 #include "smac_dev.h"
 #include "smac_kernels.h"
+
+#include <type_traits>
 
 namespace smac {
 
@@ -90,244 +93,341 @@ SMAC_DEV void point_flux(double p, double u, double v, double rx, double ry, dou
     fv[2] = v * cvel + ry * p;
 }
 
-// One direction of the stencil of point c (index t = 0 in a line of n points whose local
-// index is `i`): values of the 5 points i-2..i+2 that exist.
-struct Line5 {
-    double p[5], u[5], v[5], rx[5], ry[5], dj[5];
+// what a point's stencil needs of it
+struct Pt {
+    double p, u, v, dj, xix, xiy, etx, ety;
 };
 
-SMAC_DEV void load_line(const double *__restrict__ q, const double *__restrict__ mx,
-                        const double *__restrict__ my, const double *__restrict__ dj, long N,
-                        long base, long stride, int i, int n, Line5 &L)
+// element j of the row at `row`, the same for all lanes: a 32-bit byte offset to a scalar base
+template <typename T> SMAC_DEV T &at_lane(T *row, unsigned j)
 {
-#pragma unroll
-    for (int t = 0; t < 5; ++t) {
-        int ii = i + t - 2;
-        ii = ii < 0 ? 0 : (ii > n - 1 ? n - 1 : ii);   // clamped copies are never used
-        long a = base + stride * ii;
-        L.p[t] = q[a];
-        L.u[t] = q[N + a];
-        L.v[t] = q[2 * N + a];
-        L.rx[t] = mx[a];
-        L.ry[t] = my[a];
-        L.dj[t] = dj[a];
-    }
+    using C = typename std::conditional<std::is_const<T>::value, const char, char>::type;
+    return *(T *)((C *)row + j * (unsigned)sizeof(T));
 }
 
-// The convective part of one direction at interior point i of its line (flux.f + conup.f):
-// returns the flux difference f(i) - f(i-1) and the three blocks m (i-1), p (i+1), c.
-SMAC_DEV void convect_dir(const Line5 &L, int i, int n, double beta, double cdis, double dflux[3],
-                          double bm[9], double bp[9], double bc[9])
+// point j of the row that starts at point o
+SMAC_DEV void load_pt(const double *__restrict__ q, const double *__restrict__ met,
+                      const double *__restrict__ dj, long N, long o, unsigned j, Pt &t)
 {
-    // faces i-2 .. i+1 (face f lies between points f and f+1); index s = f - (i-2).  The
-    // blocks are formed as faces i-1 and i appear (same expressions, same order), so only
-    // face i-1's split is held until face i's.
-    double dfp[4][3], dfm[4][3];
-    double ap0[9], am0[9];   // face i-1
+    t.p = at_lane(q + o, j);
+    t.u = at_lane(q + o + N, j);
+    t.v = at_lane(q + o + 2 * N, j);
+    t.dj = at_lane(dj + o, j);
+    t.xix = at_lane(met + o, j);
+    t.xiy = at_lane(met + o + N, j);
+    t.etx = at_lane(met + o + 2 * N, j);
+    t.ety = at_lane(met + o + 3 * N, j);
+}
+
+// one face of one direction, between points a and b (a first): the split Jacobians, the
+// differences they take (d: dfp, then dfm), and the viscous coefficients, default REAL
+// (ref/visc.f:95-113)
+struct FaceVals {
+    Face F;
+    double d[6];
+};
+SMAC_DEV void face_vals(const Pt &a, const Pt &b, double rxa, double rya, double rxb, double ryb,
+                        double beta, FaceVals &f)
+{
+    const double rx = 0.5 * (rxb + rxa);
+    const double ry = 0.5 * (ryb + rya);
+    const double q2 = 0.5 * (b.u + a.u);
+    const double q3 = 0.5 * (b.v + a.v);
+    face_split(rx, ry, q2, q3, beta, f.F);
+    const double dq1 = b.p - a.p;
+    const double dq2 = b.u - a.u;
+    const double dq3 = b.v - a.v;
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-        int f = i - 2 + s;
-        bool exists = f >= 0 && f <= n - 2;
-        if (!exists) {
-            // a face the reference reads only as 0*stale (cp = 0 or cm = 0)
-            dfp[s][0] = dfp[s][1] = dfp[s][2] = 0.0;
-            dfm[s][0] = dfm[s][1] = dfm[s][2] = 0.0;
-            continue;
-        }
-        int a = s, b = s + 1;   // local points of the face
-        double rx = 0.5 * (L.rx[b] + L.rx[a]);
-        double ry = 0.5 * (L.ry[b] + L.ry[a]);
-        double q2 = 0.5 * (L.u[b] + L.u[a]);
-        double q3 = 0.5 * (L.v[b] + L.v[a]);
-        Face F;
-        face_split(rx, ry, q2, q3, beta, F);
-        double dq1 = L.p[b] - L.p[a];
-        double dq2 = L.u[b] - L.u[a];
-        double dq3 = L.v[b] - L.v[a];
-#pragma unroll
-        for (int m = 0; m < 3; ++m) {
-            dfp[s][m] = F.ap[m] * dq1 + F.ap[m + 3] * dq2 + F.ap[m + 6] * dq3;
-            dfm[s][m] = F.am[m] * dq1 + F.am[m + 3] * dq2 + F.am[m + 6] * dq3;
-        }
-        if (s == 1) {
-            double atm[9];
-            point_jac(L.rx[1], L.ry[1], L.u[1], L.v[1], beta, atm);
-#pragma unroll
-            for (int e = 0; e < 9; ++e) {
-                ap0[e] = F.ap[e];
-                am0[e] = F.am[e];
-                bm[e] = 0.5 * (-atm[e] - F.ap[e] + F.am[e]);
-            }
-        }
-        if (s == 2) {
-            double atp[9];
-            point_jac(L.rx[3], L.ry[3], L.u[3], L.v[3], beta, atp);
-#pragma unroll
-            for (int e = 0; e < 9; ++e) {
-                bp[e] = 0.5 * (atp[e] - F.ap[e] + F.am[e]);
-                bc[e] = 0.5 * (F.ap[e] + ap0[e] - F.am[e] - am0[e]);
-            }
-        }
+    for (int m = 0; m < 3; ++m) {
+        f.d[m] = f.F.ap[m] * dq1 + f.F.ap[m + 3] * dq2 + f.F.ap[m + 6] * dq3;
+        f.d[3 + m] = f.F.am[m] * dq1 + f.F.am[m + 3] * dq2 + f.F.am[m + 6] * dq3;
     }
+}
+struct Visc {
+    float vf, ud, vd;
+};
+SMAC_DEV Visc face_visc(const Pt &a, const Pt &b, double rxa, double rya, double rxb, double ryb,
+                        double vnu)
+{
+    const double djv = 0.5 * (a.dj * vnu + b.dj * vnu);
+    const double rx = 0.5 * (rxa + rxb);
+    const double ry = 0.5 * (rya + ryb);
+    return Visc{(float)(djv * (rx * rx + ry * ry)), (float)(b.u - a.u), (float)(b.v - a.v)};
+}
+
+// the numerical flux of face f of a line of n points (flux.f): fv0, fv1 the physical fluxes of
+// its two points, dm, dc, dp the differences of faces f-1, f and f+1.  The reference clamps
+// the neighbour faces' indices; the coefficients cp, cm vanish where it does (face 0's own
+// differences stand for face -1's, zeros for those of the face past the last).
+SMAC_DEV void face_flux(int f, int n, double cdis, const double fv0[3], const double fv1[3],
+                        const double dm[6], const double dc[6], const double dp[6], double ff[3])
+{
     const double r6 = (double)(1.0f / 6.0f);   // a default-REAL quotient in the reference
-    double ff[2][3];
-    // Point i is interior (1 <= i <= n-2), so for faces f = i-1 and i the neighbour faces
-    // f+1 and f+2 (clamped at n-1) and the points f, f+1 are the local entries sc = 1+w,
-    // sp = 2+w (no clamp reaches them), and face f-1, clamped at 0, is entry w except for
-    // i = 1, w = 0, where it is face 0 itself (entry 1).  Constant indices keep dfp/dfm in
-    // registers.
+    const int fm = f - 1 > 0 ? f - 1 : 0;
+    const int fp = f + 1 < n - 1 ? f + 1 : n - 1;
+    const int fpp = f + 2 < n - 1 ? f + 2 : n - 1;
+    const float cp = (float)(fpp - fp);
+    const float cm = (float)(f - fm);
 #pragma unroll
-    for (int w = 0; w < 2; ++w) {
-        int f = i - 1 + w;             // face index; its neighbours are faces f-1 (clamped) and f+1
-        int fm = f - 1 > 0 ? f - 1 : 0;
-        int fp = f + 1 < n - 1 ? f + 1 : n - 1;
-        int fpp = f + 2 < n - 1 ? f + 2 : n - 1;
-        float cp = (float)(fpp - fp);
-        float cm = (float)(f - fm);
-        constexpr int sc = 1, sp = 2;  // + w below
-        const bool sm1 = w == 0 && i == 1;
-        const int pf = 1 + w, pp = 2 + w;   // local point indices f, f+1
-        double fv0[3], fv1[3];
-        point_flux(L.p[pf], L.u[pf], L.v[pf], L.rx[pf], L.ry[pf], beta, fv0);
-        point_flux(L.p[pp], L.u[pp], L.v[pp], L.rx[pp], L.ry[pp], beta, fv1);
+    for (int m = 0; m < 3; ++m) {
+        const double pc = dc[m], mc = dc[3 + m];
+        const double pn = dp[m], mn = dp[3 + m];
+        const double pm = f == 0 ? pc : dm[m], mm = f == 0 ? mc : dm[3 + m];
+        const double fmn = (pc + mc - pn - mn) * r6;
+        const double fpl = (pm + mm - pc - mc) * r6;
+        const double f3 = (pm - pc + mc - mn) * r6;
+        ff[m] = 0.5 * (fv1[m] + fv0[m]) +
+                cdis * ((double)(cp * cm) * f3 + (double)(cm * (1.f - cp)) * fpl +
+                        (double)(cp * (1.f - cm)) * fmn);
+    }
+}
+
+// a neighbouring lane's value: lane-1 (wave_shr) or lane+1 (wave_shl)
+template <bool UP> SMAC_DEV int from_lane(int v)
+{
+    return __builtin_amdgcn_update_dpp(0, v, UP ? 0x138 : 0x130, 0xf, 0xf, true);
+}
+template <bool UP> SMAC_DEV float from_lane(float v)
+{
+    return __builtin_bit_cast(float, from_lane<UP>(__builtin_bit_cast(int, v)));
+}
+template <bool UP> SMAC_DEV double from_lane(double v)
+{
+    const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+    const unsigned lo = (unsigned)from_lane<UP>((int)(unsigned)u);
+    const unsigned hi = (unsigned)from_lane<UP>((int)(unsigned)(u >> 32));
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+constexpr int ASM_COLS = 60;   // points of a row that a wave assembles
+
+// One wave assembles ASM_COLS points of `rows` rows, lane l at j = ASM_COLS bk.x + l - 2, and
+// marches in k.  A lane computes the xi face between its point and the next and one eta face
+// per row; what a point needs of its other faces comes from the lanes beside it (DPP moves; the
+// two outer lanes on each side only serve their neighbours) and from the rows
+// before (registers).  The row r's blocks need the eta faces r-1 and r; s of row r-1 needs the
+// fluxes of faces r-2 and r-1, which need face r: so s follows its blocks by one row, and a
+// strip starts two faces early and ends one late.
+template <typename LT>
+SMAC_DEV void b_assemble(const Blk &bk, int rows, const Dims &d, const DevParams &prm,
+                         const double *__restrict__ q, const double *__restrict__ met,
+                         const double *__restrict__ dj, double *__restrict__ s,
+                         LT *__restrict__ btc, LT *__restrict__ bjm, LT *__restrict__ bjp,
+                         LT *__restrict__ bkm, LT *__restrict__ bkp)
+{
+    const int lane = threadIdx.x & 63, jm = d.jm, km = d.km;
+    const int j = ASM_COLS * (int)bk.x + lane - 2;
+    const int r0 = rows * (int)bk.y, r1 = r0 + rows < km ? r0 + rows : km;   // rows [r0, r1)
+    const long N = d.N;
+    const int jc = j < 0 ? 0 : (j > jm - 1 ? jm - 1 : j);
+    const bool out = lane >= 2 && lane < 2 + ASM_COLS && j < jm;
+    const bool jin = j > 0 && j < jm - 1, jface = j >= 0 && j < jm - 1;
+    const double beta = prm.beta;
+    auto fetch = [&](int r, Pt &t) {
+        const int rc = r < 0 ? 0 : (r > km - 1 ? km - 1 : r);
+        load_pt(q, met, dj, N, (long)rc * jm, (unsigned)jc, t);
+    };
+    Pt cur, nxt, pre;        // rows r, r+1, r+2
+    fetch(r0 - 2, cur);
+    fetch(r0 - 1, nxt);
+    // of the faces and rows before: differences of faces r-2 and r-1, split of face r-1, flux
+    // of face r-2, physical flux of point r, point r-1's Jacobian operands, viscous faces r-2
+    // and r-1, and of row r-1 the xi terms of s
+    double d2[6] = {}, d1[6] = {}, ap0[9] = {}, am0[9] = {}, ff2[3] = {}, fv0[3] = {};
+    double pu = 0.0, pv = 0.0, prx = 0.0, pry = 0.0, sx[3] = {};
+    Visc v2{0.f, 0.f, 0.f}, v1{0.f, 0.f, 0.f};
+    float tx2 = 0.f, tx3 = 0.f;
+    for (int r = r0 - 2; r <= r1; ++r) {
+        fetch(r + 2, pre);
+        const bool mine = r >= r0 && r < r1, inner = r > 0 && r < km - 1;
+        // the planes' addresses are formed anew in each row (two scalar additions each): kept
+        // over the loop, 48 of them do not fit the scalar registers
+        long N = d.N;
+        asm volatile("" : "+s"(N));
+        const long o = (long)r * jm;
+        double vc[9], sxn[3];
+        Visc vr{0.f, 0.f, 0.f}, vl{0.f, 0.f, 0.f};
+        if (mine && inner) {
+            // ---- xi: the face to the next point, then what the lane before holds
+            // (ref/conup.f:216-271, ref/visc.f:95-113)
+            Pt right;
+            right.p = from_lane<false>(cur.p);
+            right.u = from_lane<false>(cur.u);
+            right.v = from_lane<false>(cur.v);
+            right.dj = from_lane<false>(cur.dj);
+            right.xix = from_lane<false>(cur.xix);
+            right.xiy = from_lane<false>(cur.xiy);
+            FaceVals x;
+            face_vals(cur, right, cur.xix, cur.xiy, right.xix, right.xiy, beta, x);
+#pragma unroll
+            for (int i = 0; i < 6; ++i) x.d[i] = jface ? x.d[i] : 0.0;
+            {
+                double dl[6], dr[6], fc[3], fr[3], fx[3];
+#pragma unroll
+                for (int i = 0; i < 6; ++i) {
+                    dl[i] = from_lane<true>(x.d[i]);
+                    dr[i] = from_lane<false>(x.d[i]);
+                }
+                point_flux(cur.p, cur.u, cur.v, cur.xix, cur.xiy, beta, fc);
+#pragma unroll
+                for (int m = 0; m < 3; ++m) fr[m] = from_lane<false>(fc[m]);
+                face_flux(j, jm, prm.cdis, fc, fr, dl, x.d, dr, fx);
+#pragma unroll
+                for (int m = 0; m < 3; ++m) sxn[m] = -(fx[m] - from_lane<true>(fx[m]));
+            }
+            double a4 = 0.0, b4 = 0.0;
+            if (prm.ivis == 1) {
+                vr = face_visc(cur, right, cur.xix, cur.xiy, right.xix, right.xiy, prm.vnu);
+                vl.vf = from_lane<true>(vr.vf);
+                vl.ud = from_lane<true>(vr.ud);
+                vl.vd = from_lane<true>(vr.vd);
+                a4 = vl.vf;
+                b4 = vr.vf;
+            }
+            double al[9], ar[9];
+            point_jac(from_lane<true>(cur.xix), from_lane<true>(cur.xiy), from_lane<true>(cur.u),
+                      from_lane<true>(cur.v), beta, al);
+            point_jac(right.xix, right.xiy, right.u, right.v, beta, ar);
+#pragma unroll
+            for (int i = 0; i < 9; ++i) {
+                const double apl = from_lane<true>(x.F.ap[i]), aml = from_lane<true>(x.F.am[i]);
+                double bm = 0.5 * (-al[i] - apl + aml);
+                double bp = 0.5 * (ar[i] - x.F.ap[i] + x.F.am[i]);
+                vc[i] = 0.5 * (x.F.ap[i] + apl - x.F.am[i] - aml);
+                if ((i == 4 || i == 8) && prm.ivis == 1) {
+                    bm = bm - a4;
+                    bp = bp - b4;
+                }
+                if (jin && out) {
+                    at_lane(bjm + i * N + o, (unsigned)j) = (LT)bm;
+                    at_lane(bjp + i * N + o, (unsigned)j) = (LT)bp;
+                }
+            }
+        }
+        // the eta face r, where it exists; elsewhere the reference reads it only as 0*stale
+        FaceVals e;
+        Visc ve{0.f, 0.f, 0.f};
+        if (r >= 0 && r < km - 1) {
+            face_vals(cur, nxt, cur.etx, cur.ety, nxt.etx, nxt.ety, beta, e);
+            if (prm.ivis == 1) ve = face_visc(cur, nxt, cur.etx, cur.ety, nxt.etx, nxt.ety, prm.vnu);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 6; ++i) e.d[i] = 0.0;
+#pragma unroll
+            for (int i = 0; i < 9; ++i) e.F.ap[i] = e.F.am[i] = 0.0;
+        }
+        double fv1[3];
+        point_flux(cur.p, cur.u, cur.v, cur.etx, cur.ety, beta, fv1);
+        // flux of face r-1, between points r-1 and r
+        double ff[3] = {0.0, 0.0, 0.0};
+        if (r >= r0 && r > 0) face_flux(r - 1, km, prm.cdis, fv0, fv1, d2, d1, e.d, ff);
+        // s of row r-1 (ref/conup.f:216-271, 377-457, ref/visc.f:95-140)
+        if (r > r0) {
+            double vs[3];
+#pragma unroll
+            for (int m = 0; m < 3; ++m) vs[m] = sx[m] - (ff[m] - ff2[m]);
+            if (prm.ivis == 1) {
+                vs[1] = vs[1] + (double)tx2;
+                vs[2] = vs[2] + (double)tx3;
+                const float t2 = v1.vf * v1.ud - v2.vf * v2.ud;
+                const float t3 = v1.vf * v1.vd - v2.vf * v2.vd;
+                vs[1] = vs[1] + (double)t2;
+                vs[2] = vs[2] + (double)t3;
+            }
+            const bool live = jin && r - 1 > 0 && r - 1 < km - 1;
+            if (out) {
+#pragma unroll
+                for (int m = 0; m < 3; ++m)
+                    at_lane(s + m * N + o - jm, (unsigned)j) = live ? vs[m] : 0.0;
+            }
+        }
+        if (mine && inner) {
+            // ---- eta: add (ref/conup.f:377-457, ref/visc.f:121-140)
+            double am_[9], ar[9];
+            point_jac(prx, pry, pu, pv, beta, am_);
+            point_jac(nxt.etx, nxt.ety, nxt.u, nxt.v, beta, ar);
+            // pseudo-time diagonal (ref/step.f:419-437), fib = 1
+            const double rdjdtau = 1.0 / (cur.dj * prm.dtau) + 1. - 1.0;
+            const double xa = vl.vf, xb = vr.vf, a = v1.vf, b = ve.vf;
+#pragma unroll
+            for (int i = 0; i < 9; ++i) {
+                double bm = 0.5 * (-am_[i] - ap0[i] + am0[i]);
+                double bp = 0.5 * (ar[i] - e.F.ap[i] + e.F.am[i]);
+                double c = vc[i] + 0.5 * (e.F.ap[i] + ap0[i] - e.F.am[i] - am0[i]);
+                if ((i == 4 || i == 8) && prm.ivis == 1) {
+                    bm = bm - a;
+                    bp = bp - b;
+                    c = c + xa + xb;
+                    c = c + a + b;
+                }
+                if (i == 0 || i == 4 || i == 8) c = c + rdjdtau;
+                if (jin && out) {
+                    at_lane(bkm + i * N + o, (unsigned)j) = (LT)bm;
+                    at_lane(bkp + i * N + o, (unsigned)j) = (LT)bp;
+                    at_lane(btc + i * N + o, (unsigned)j) = (LT)c;
+                }
+            }
+#pragma unroll
+            for (int m = 0; m < 3; ++m) sx[m] = sxn[m];
+            tx2 = vr.vf * vr.ud - vl.vf * vl.ud;
+            tx3 = vr.vf * vr.vd - vl.vf * vl.vd;
+        }
+        if (mine && out && !(jin && inner)) {
+            // blanked boundary row: all blocks zero, btc = identity (ref/step.f:386-437)
+#pragma unroll
+            for (int i = 0; i < 9; ++i) {
+                at_lane(btc + i * N + o, (unsigned)j) = (LT)((i == 0 || i == 4 || i == 8) ? 1.0 : 0.0);
+                at_lane(bjm + i * N + o, (unsigned)j) = (LT)0.0;
+                at_lane(bjp + i * N + o, (unsigned)j) = (LT)0.0;
+                at_lane(bkm + i * N + o, (unsigned)j) = (LT)0.0;
+                at_lane(bkp + i * N + o, (unsigned)j) = (LT)0.0;
+            }
+        }
+        // one row on
+#pragma unroll
+        for (int i = 0; i < 6; ++i) {
+            d2[i] = d1[i];
+            d1[i] = e.d[i];
+        }
+#pragma unroll
+        for (int i = 0; i < 9; ++i) {
+            ap0[i] = e.F.ap[i];
+            am0[i] = e.F.am[i];
+        }
 #pragma unroll
         for (int m = 0; m < 3; ++m) {
-            const double pc = dfp[sc + w][m], mc = dfm[sc + w][m];
-            const double pn = dfp[sp + w][m], mn = dfm[sp + w][m];
-            const double pm = sm1 ? dfp[1][m] : dfp[w][m], mm = sm1 ? dfm[1][m] : dfm[w][m];
-            double fmn = (pc + mc - pn - mn) * r6;
-            double fpl = (pm + mm - pc - mc) * r6;
-            double f3 = (pm - pc + mc - mn) * r6;
-            ff[w][m] = 0.5 * (fv1[m] + fv0[m]) +
-                       cdis * ((double)(cp * cm) * f3 + (double)(cm * (1.f - cp)) * fpl +
-                               (double)(cp * (1.f - cm)) * fmn);
+            ff2[m] = ff[m];
+            fv0[m] = fv1[m];
         }
+        v2 = v1;
+        v1 = ve;
+        pu = cur.u; pv = cur.v; prx = cur.etx; pry = cur.ety;
+        cur = nxt;
+        nxt = pre;
     }
-#pragma unroll
-    for (int m = 0; m < 3; ++m) dflux[m] = ff[1][m] - ff[0][m];
 }
 
-// viscous face coefficients of one direction at interior point i (ref/visc.f:95-113):
-// vf, udif, vdif of faces i-1 (index 0) and i (index 1), all default REAL
-SMAC_DEV void visc_dir(const Line5 &L, double vnu, float vf[2], float ud[2], float vd[2])
+// Rows per wave: marching saves faces (five a point for one row, 2.8 for four), one row each keeps
+// more waves running; four rows where that still leaves the chip's 1024 SIMDs a wave each, two
+// or one below.  1, 2, 4, 8 rows: 477x121 14.4, 19, 24, 40 us; 945x241 36, 30, 36, 50;
+// 1889x481 188, 154, 117, 149.  A wave's 300 registers leave room for one per SIMD; held to
+// two (256, a few spilled) it is the slower alone (120 us) and the faster in a batch (169 us
+// against 190), whose blocks are unequal.
+static int asm_rows(const Dims &d)
 {
-#pragma unroll
-    for (int w = 0; w < 2; ++w) {
-        int a = 1 + w, b = 2 + w;
-        double djv = 0.5 * (L.dj[a] * vnu + L.dj[b] * vnu);
-        ud[w] = (float)(L.u[b] - L.u[a]);
-        vd[w] = (float)(L.v[b] - L.v[a]);
-        double rx = 0.5 * (L.rx[a] + L.rx[b]);
-        double ry = 0.5 * (L.ry[a] + L.ry[b]);
-        vf[w] = (float)(djv * (rx * rx + ry * ry));
-    }
+    const long strips = (d.jm + ASM_COLS - 1) / ASM_COLS;
+    for (int rows = 4; rows > 1; rows /= 2)
+        if (strips * ((d.km + rows - 1) / rows) >= 1024) return rows;
+    return 1;
 }
 
 template <typename LT>
-SMAC_DEV void b_assemble(const Blk &bk, Dims d, DevParams prm, const double *__restrict__ q,
-                         const double *__restrict__ met, const double *__restrict__ dj,
-                         double *__restrict__ s, LT *__restrict__ btc, LT *__restrict__ bjm,
-                         LT *__restrict__ bjp, LT *__restrict__ bkm, LT *__restrict__ bkp)
-{
-    const int j = bk.x * blockDim.x + threadIdx.x;
-    const int k = bk.y;
-    if (j >= d.jm || k >= d.km) return;
-    const long N = d.N, p = P(d, j, k);
-    const bool interior = j > 0 && j < d.jm - 1 && k > 0 && k < d.km - 1;
-    if (!interior) {
-        // blanked boundary row: all blocks and s zero, btc = identity (ref/step.f:386-437)
-#pragma unroll
-        for (int m = 0; m < 3; ++m) s[m * N + p] = 0.0;
-#pragma unroll
-        for (int e = 0; e < 9; ++e) {
-            btc[e * N + p] = (LT)((e == 0 || e == 4 || e == 8) ? 1.0 : 0.0);
-            bjm[e * N + p] = (LT)0.0;
-            bjp[e * N + p] = (LT)0.0;
-            bkm[e * N + p] = (LT)0.0;
-            bkp[e * N + p] = (LT)0.0;
-        }
-        return;
-    }
-    // Each direction's neighbour blocks are final once that direction is done and are stored
-    // then; the centre block and s take their terms in the reference's order: xi convective,
-    // eta convective, xi viscous, eta viscous, pseudo-time diagonal.
-    const double *xix = met, *xiy = met + N, *etx = met + 2 * N, *ety = met + 3 * N;
-    double vs[3], vc[9], df[3];
-    float vfx[2], udx[2], vdx[2];
-    Line5 L, Le;
-    // xi: assign (ref/conup.f:216-271); the eta line's loads are issued first, so that their
-    // latency runs under the xi arithmetic
-    load_line(q, etx, ety, dj, N, (long)j, d.jm, k, d.km, Le);
-    load_line(q, xix, xiy, dj, N, (long)d.jm * k, 1, j, d.jm, L);
-    {
-        double bm[9], bp[9];
-        convect_dir(L, j, d.jm, prm.beta, prm.cdis, df, bm, bp, vc);
-#pragma unroll
-        for (int m = 0; m < 3; ++m) vs[m] = -df[m];
-        if (prm.ivis == 1) {
-            visc_dir(L, prm.vnu, vfx, udx, vdx);
-            // xi viscous blocks (ref/visc.f:95-113)
-            const double a = vfx[0], b = vfx[1];
-            bm[4] = bm[4] - a; bm[8] = bm[8] - a;
-            bp[4] = bp[4] - b; bp[8] = bp[8] - b;
-        }
-#pragma unroll
-        for (int e = 0; e < 9; ++e) {
-            bjm[e * N + p] = (LT)bm[e];
-            bjp[e * N + p] = (LT)bp[e];
-        }
-    }
-    // eta: add (ref/conup.f:377-457)
-    {
-        double bm[9], bp[9], bc[9];
-        convect_dir(Le, k, d.km, prm.beta, prm.cdis, df, bm, bp, bc);
-#pragma unroll
-        for (int e = 0; e < 9; ++e) vc[e] = vc[e] + bc[e];
-#pragma unroll
-        for (int m = 0; m < 3; ++m) vs[m] = vs[m] - df[m];
-        if (prm.ivis == 1) {
-            float vfy[2], udy[2], vdy[2];
-            visc_dir(Le, prm.vnu, vfy, udy, vdy);
-            // xi viscous terms of the centre and s (ref/visc.f:95-113), then eta (:121-140)
-            double a = vfx[0], b = vfx[1];
-            vc[4] = vc[4] + a + b; vc[8] = vc[8] + a + b;
-            float t2 = vfx[1] * udx[1] - vfx[0] * udx[0];
-            float t3 = vfx[1] * vdx[1] - vfx[0] * vdx[0];
-            vs[1] = vs[1] + (double)t2;
-            vs[2] = vs[2] + (double)t3;
-            a = vfy[0]; b = vfy[1];
-            bm[4] = bm[4] - a; bm[8] = bm[8] - a;
-            vc[4] = vc[4] + a + b; vc[8] = vc[8] + a + b;
-            bp[4] = bp[4] - b; bp[8] = bp[8] - b;
-            t2 = vfy[1] * udy[1] - vfy[0] * udy[0];
-            t3 = vfy[1] * vdy[1] - vfy[0] * vdy[0];
-            vs[1] = vs[1] + (double)t2;
-            vs[2] = vs[2] + (double)t3;
-        }
-#pragma unroll
-        for (int e = 0; e < 9; ++e) {
-            bkm[e * N + p] = (LT)bm[e];
-            bkp[e * N + p] = (LT)bp[e];
-        }
-    }
-    // pseudo-time diagonal (ref/step.f:419-437), fib = 1
-    double rdjdtau = 1.0 / (dj[p] * prm.dtau) + 1. - 1.0;
-    vc[0] = vc[0] + rdjdtau;
-    vc[4] = vc[4] + rdjdtau;
-    vc[8] = vc[8] + rdjdtau;
-#pragma unroll
-    for (int m = 0; m < 3; ++m) s[m * N + p] = vs[m];
-#pragma unroll
-    for (int e = 0; e < 9; ++e) btc[e * N + p] = (LT)vc[e];
-}
-
-template <typename LT>
-__global__ void __launch_bounds__(256)
-k_assemble(Dims d, DevParams prm, const double *__restrict__ q, const double *__restrict__ met,
-           const double *__restrict__ dj, double *__restrict__ s, LT *__restrict__ btc,
+__global__ void __launch_bounds__(64)
+k_assemble(Dims d, DevParams prm, int rows, const double *__restrict__ q,
+           const double *__restrict__ met, const double *__restrict__ dj, double *__restrict__ s, LT *__restrict__ btc,
            LT *__restrict__ bjm, LT *__restrict__ bjp, LT *__restrict__ bkm, LT *__restrict__ bkp)
 {
-    b_assemble<LT>(xcd_blk(), d, prm, q, met, dj, s, btc, bjm, bjp, bkm, bkp);
+    b_assemble<LT>(xcd_blk(), rows, d, prm, q, met, dj, s, btc, bjm, bjp, bkm, bkp);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -569,9 +669,10 @@ void launch_assemble(hipStream_t sm, const Dims &d, const DevParams &prm, const 
                      const double *met, const double *dj, double *s, LT *btc, LT *bjm, LT *bjp,
                      LT *bkm, LT *bkp)
 {
-    dim3 blk(64), grd((d.jm + 63) / 64, d.km);
-    hipLaunchKernelGGL(k_assemble<LT>, grd, blk, 0, sm, d, prm, q, met, dj, s, btc, bjm, bjp, bkm,
-                       bkp);
+    const int rows = asm_rows(d);
+    dim3 blk(64), grd((d.jm + ASM_COLS - 1) / ASM_COLS, (d.km + rows - 1) / rows);
+    hipLaunchKernelGGL(k_assemble<LT>, grd, blk, 0, sm, d, prm, rows, q, met, dj, s, btc, bjm, bjp,
+                       bkm, bkp);
 }
 
 template <typename LT>
@@ -612,8 +713,10 @@ template <typename LT>
 AsmArgs asm_args(const Dims &d, const DevParams &prm, const double *q, const double *met,
                  const double *dj, double *s, LT *btc, LT *bjm, LT *bjp, LT *bkm, LT *bkp)
 {
-    return AsmArgs{(unsigned)((d.jm + 63) / 64), (unsigned)d.km, d, prm, q, met, dj, s, btc, bjm,
-                   bjp, bkm, bkp};
+    // the cases of a batch fill the chip together
+    constexpr int rows = 4;
+    return AsmArgs{(unsigned)((d.jm + ASM_COLS - 1) / ASM_COLS), (unsigned)((d.km + rows - 1) / rows),
+                   d, prm, rows, q, met, dj, s, btc, bjm, bjp, bkm, bkp};
 }
 
 template <typename LT>
@@ -651,11 +754,12 @@ ResidFArgs residf_args(const Dims &d, int nt, double beta, const double *s, cons
 template <typename LT>
 struct CAssemble {
     using Args = AsmArgs;
-    static constexpr int THREADS = 64;
+    static constexpr int THREADS = 64, WAVES = 2;
     static SMAC_DEV void run(const Blk &b, const Args &a)
     {
-        b_assemble<LT>(b, a.d, a.prm, a.q, a.met, a.dj, a.s, (LT *)a.btc, (LT *)a.bjm,
-                       (LT *)a.bjp, (LT *)a.bkm, (LT *)a.bkp);
+        b_assemble<LT>(b, a.rows, a.d, a.prm, as_global(a.q), as_global(a.met), as_global(a.dj),
+                       as_global(a.s), (LT *)as_global(a.btc), (LT *)as_global(a.bjm),
+                       (LT *)as_global(a.bjp), (LT *)as_global(a.bkm), (LT *)as_global(a.bkp));
     }
 };
 

@@ -69,6 +69,15 @@ SMAC_DEV Blk xcd_blk()
     return Blk{lg % gridDim.x, lg / gridDim.x, gridDim.x, gridDim.y};
 }
 
+// A pointer that stands in a table in memory, read as one to device memory: its accesses are
+// global ones; read as a plain pointer they are flat, which also wait for the LDS.
+template <typename T> SMAC_DEV T *as_global(T *const &p)
+{
+    __attribute__((address_space(1))) T *g;
+    __builtin_memcpy(&g, &p, sizeof g);
+    return (T *)g;
+}
+
 // One launch for many items (cases, or a case's BC regions) of one kernel: item i's own grid
 // is args[i].gx x args[i].gy blocks, and the launch's blocks are those grids one after the
 // other (start[i] = the first block of item i, start[n] = the total).  Each block finds its
@@ -76,8 +85,12 @@ SMAC_DEV Blk xcd_blk()
 // item's grid, so every item gets exactly the work (and the arithmetic) of its own launch.
 // Blocks are taken in the XCD-aware order (xcd_lin), so that an item's neighbouring blocks
 // share an L2; no body waits on another block, so the order is free.
+// Waves per SIMD that a body's registers are to leave room for (C::WAVES, else one).
+template <class C> constexpr auto multi_waves(int) -> decltype(C::WAVES) { return C::WAVES; }
+template <class C> constexpr int multi_waves(long) { return 1; }
+
 template <class C>
-__global__ void __launch_bounds__(C::THREADS)
+__global__ void __launch_bounds__(C::THREADS, multi_waves<C>(0))
 k_multi(const typename C::Args *__restrict__ args, const int *__restrict__ start, int n,
         const int *__restrict__ item_case, const int *__restrict__ active)
 {

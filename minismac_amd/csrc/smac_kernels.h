@@ -246,6 +246,7 @@ struct AsmArgs {      // k_assemble
     unsigned gx, gy;
     Dims d;
     DevParams prm;
+    int rows;
     const double *q, *met, *dj;
     double *s;
     void *btc, *bjm, *bjp, *bkm, *bkp;   // LT
