@@ -769,8 +769,10 @@ struct CBc {
     static constexpr int THREADS = BC_THREADS;
     static SMAC_DEV void run(const Blk &, const Args &a)
     {
-        b_bc<LT>(a.d, a.t, a.pout, a.alpha, a.beta, a.st, a.x, a.y, a.met, a.q, a.s, (LT *)a.btc,
-                 (LT *)a.bjm, (LT *)a.bjp, (LT *)a.bkm, (LT *)a.bkp);
+        b_bc<LT>(a.d, a.t, a.pout, a.alpha, a.beta, as_global(a.st), as_global(a.x),
+                 as_global(a.y), as_global(a.met), as_global(a.q), as_global(a.s),
+                 (LT *)as_global(a.btc), (LT *)as_global(a.bjm), (LT *)as_global(a.bjp),
+                 (LT *)as_global(a.bkm), (LT *)as_global(a.bkp));
     }
 };
 
@@ -779,7 +781,8 @@ struct CResidP {
     static constexpr int THREADS = RED_THREADS;
     static SMAC_DEV void run(const Blk &b, const Args &a)
     {
-        b_resid_partial(b, a.d, a.s, a.dj, a.part_v, a.part_i, a.part_s);
+        b_resid_partial(b, a.d, as_global(a.s), as_global(a.dj), as_global(a.part_v),
+                        as_global(a.part_i), as_global(a.part_s));
     }
 };
 
@@ -788,8 +791,9 @@ struct CResidF {
     static constexpr int THREADS = RED_THREADS;
     static SMAC_DEV void run(const Blk &, const Args &a)
     {
-        b_resid_final(a.d, a.nparts, a.nt, a.beta, a.s, a.dj, a.part_v, a.part_i, a.part_s,
-                      a.st);
+        b_resid_final(a.d, a.nparts, a.nt, a.beta, as_global(a.s), as_global(a.dj),
+                      as_global(a.part_v), as_global(a.part_i), as_global(a.part_s),
+                      as_global(a.st));
     }
 };
 

@@ -215,14 +215,15 @@ ForceArgs force_args(const Dims &d, const DevParams &prm, const Walls &wl, const
 struct CUpdate {
     using Args = UpdArgs;
     static constexpr int THREADS = 256;
-    static SMAC_DEV void run(const Blk &b, const Args &a) { b_update(b, a.n3, a.q, a.dq, a.flag); }
+    static SMAC_DEV void run(const Blk &b, const Args &a) { b_update(b, a.n3, as_global(a.q), as_global(a.dq), as_global(a.flag)); }
 };
 struct CForce {
     using Args = ForceArgs;
     static constexpr int THREADS = FORCE_THREADS;
     static SMAC_DEV void run(const Blk &, const Args &a)
     {
-        b_force(a.d, a.prm, a.wl, a.x, a.y, a.met, a.dj, a.q, a.flag, a.st);
+        b_force(a.d, a.prm, a.wl, as_global(a.x), as_global(a.y), as_global(a.met),
+                as_global(a.dj), as_global(a.q), as_global(a.flag), as_global(a.st));
     }
 };
 

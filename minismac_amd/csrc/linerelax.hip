@@ -527,7 +527,8 @@ struct CWake {
     static constexpr int THREADS = 64;
     static SMAC_DEV void run(const Blk &b, const Args &a)
     {
-        b_wake(b, a.N, a.jm, a.neqs, a.npair, a.base, a.pairs, a.sq, a.ds, a.rhs);
+        b_wake(b, a.N, a.jm, a.neqs, a.npair, a.base, as_global(a.pairs), as_global(a.sq),
+               as_global(a.ds), as_global(a.rhs));
     }
 };
 

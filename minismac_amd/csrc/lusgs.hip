@@ -935,6 +935,16 @@ k_band(Dims d, LusgsWs w)
 // The bands of several cases in one launch: workgroup i runs band map[i].y of case map[i].x.
 // The map lists each case's bands contiguously in dispatch order, so every wait is on a
 // workgroup dispatched earlier.
+// a workspace out of a table in memory
+SMAC_DEV LusgsWs ws_global(const LusgsWs &t)
+{
+    LusgsWs w = t;
+    w.lhs = as_global(t.lhs);
+    w.edge = as_global(t.edge);
+    w.stall = as_global(t.stall);
+    return w;
+}
+
 template <int NEQ, bool FWD, typename T>
 __global__ void __launch_bounds__(BAND_LANES * BAND_WAVES)
 k_band_multi(const BandJob *__restrict__ jobs, const int2 *__restrict__ map,
@@ -944,7 +954,7 @@ k_band_multi(const BandJob *__restrict__ jobs, const int2 *__restrict__ map,
     // a stopped case: all of its bands leave, so none waits on another
     if (active && active[jobs[m.x].bcase] == 0) return;
     const Dims d = jobs[m.x].d;
-    const LusgsWs w = jobs[m.x].w;
+    const LusgsWs w = ws_global(jobs[m.x].w);
     band_run<NEQ, FWD, T>(d, w, m.y);
 }
 
@@ -1048,15 +1058,17 @@ struct CShear {
     static constexpr int THREADS = TILE_THREADS;
     static SMAC_DEV void run(const Blk &b, const Args &a)
     {
-        b_shear<LT, NEQ>(b, a.d, a.w, a.rhs, (const LT *)a.btc, (const LT *)a.bjm,
-                         (const LT *)a.bkm, (const LT *)a.bjp, (const LT *)a.bkp, (LT *)a.fac);
+        b_shear<LT, NEQ>(b, a.d, ws_global(a.w), as_global(a.rhs), (const LT *)as_global(a.btc),
+                         (const LT *)as_global(a.bjm), (const LT *)as_global(a.bkm),
+                         (const LT *)as_global(a.bjp), (const LT *)as_global(a.bkp),
+                         a.fac ? (LT *)as_global(a.fac) : nullptr);
     }
 };
 template <typename LT, int NEQ>
 struct CMid {
     using Args = MidArgs;
     static constexpr int THREADS = 256;
-    static SMAC_DEV void run(const Blk &b, const Args &a) { b_mid<LT, NEQ>(b, a.d, a.w); }
+    static SMAC_DEV void run(const Blk &b, const Args &a) { b_mid<LT, NEQ>(b, a.d, ws_global(a.w)); }
 };
 template <typename LT, int NEQ>
 struct CUnshear {
@@ -1064,7 +1076,7 @@ struct CUnshear {
     static constexpr int THREADS = TILE_THREADS;
     static SMAC_DEV void run(const Blk &b, const Args &a)
     {
-        b_unshear<NEQ, LT>(b, a.d, a.w, false, a.dst);
+        b_unshear<NEQ, LT>(b, a.d, ws_global(a.w), false, as_global(a.dst));
     }
 };
 

@@ -520,7 +520,8 @@ struct CSaDeriv {
     static constexpr int THREADS = 64;
     static SMAC_DEV void run(const Blk &b, const Args &a)
     {
-        b_sa_deriv(b, a.d, a.q, a.met, a.dj, a.vort, a.cu, a.ck, a.cv, a.fr);
+        b_sa_deriv(b, a.d, as_global(a.q), as_global(a.met), as_global(a.dj), as_global(a.vort),
+                   as_global(a.cu), as_global(a.ck), as_global(a.cv), as_global(a.fr));
     }
 };
 struct CSaAsm {
@@ -528,8 +529,11 @@ struct CSaAsm {
     static constexpr int THREADS = 64;
     static SMAC_DEV void run(const Blk &b, const Args &a)
     {
-        b_sa_assemble(b, a.d, a.prm, a.q, a.met, a.dj, a.anut, a.smin, a.use_smin, a.vort, a.cu,
-                      a.ck, a.cv, a.fr, a.sjm, a.sjp, a.skm, a.skp, a.stc, a.sf);
+        b_sa_assemble(b, a.d, a.prm, as_global(a.q), as_global(a.met), as_global(a.dj),
+                      as_global(a.anut), as_global(a.smin), a.use_smin, as_global(a.vort),
+                      as_global(a.cu), as_global(a.ck), as_global(a.cv), as_global(a.fr),
+                      as_global(a.sjm), as_global(a.sjp), as_global(a.skm), as_global(a.skp),
+                      as_global(a.stc), as_global(a.sf));
     }
 };
 struct CSaBc {
@@ -537,7 +541,8 @@ struct CSaBc {
     static constexpr int THREADS = 64;
     static SMAC_DEV void run(const Blk &b, const Args &a)
     {
-        b_sa_bc(b, a.d, a.r, a.anut, a.sjm, a.sjp, a.skm, a.skp, a.stc, a.sf);
+        b_sa_bc(b, a.d, a.r, as_global(a.anut), as_global(a.sjm), as_global(a.sjp),
+                as_global(a.skm), as_global(a.skp), as_global(a.stc), as_global(a.sf));
     }
 };
 struct CSaUpd {
@@ -545,13 +550,14 @@ struct CSaUpd {
     static constexpr int THREADS = 256;
     static SMAC_DEV void run(const Blk &b, const Args &a)
     {
-        b_sa_update(b, a.N, a.vnu, a.anut, a.ds, a.vnut, a.part);
+        b_sa_update(b, a.N, a.vnu, as_global(a.anut), as_global(a.ds), as_global(a.vnut),
+                    as_global(a.part));
     }
 };
 struct CSaTur {
     using Args = SaTurArgs;
     static constexpr int THREADS = 256;
-    static SMAC_DEV void run(const Blk &, const Args &a) { b_sa_turres(a.n, a.part, a.st); }
+    static SMAC_DEV void run(const Blk &, const Args &a) { b_sa_turres(a.n, as_global(a.part), as_global(a.st)); }
 };
 
 template <class C>
