@@ -235,7 +235,7 @@ struct MultiTab {
     int n = 0, nblk = 0;
 };
 
-constexpr int BC_THREADS = 256;
+constexpr int BC_THREADS = 64;
 constexpr int BC_MAX = 16;
 struct BcTable {
     int n;
