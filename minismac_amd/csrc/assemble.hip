@@ -568,7 +568,9 @@ k_bc(Dims d, BcTable t, double pout, double alpha, double beta, const DevStats *
 // ---------------------------------------------------------------------------------------
 // resid + rhsnorm: isamax over s*dj (ties to the first index, ref/blas.f:48-83) for all 3N
 // entries and for the first N, and sum of s^2; partials per block, then one final block.
-// The partition is fixed, so the result is the same on every run.
+// The partition is fixed, so the result is the same on every run.  945x241: 6 us for the partials
+// (1.2 TB/s; with a 64-bit remainder for every value 11-12 us beside the SA) and 4.6 us for the
+// final block, both mostly a launch and the latency of one round of loads.
 
 struct ArgMax {
     double v;
@@ -583,6 +585,36 @@ SMAC_DEV ArgMax amax_join(ArgMax a, ArgMax b)
 
 constexpr int RED_THREADS = 256;
 
+// Thread 0 gets the block's values: t joins t + w, w = 128, 64 .. 1, the last 64 in one wave.
+SMAC_DEV void red_tree(ArgMax &all, ArgMax &first, double &ss)
+{
+    constexpr int W = 64;
+    static_assert(RED_THREADS == 4 * W, "two steps through LDS");
+    __shared__ double v[2 * W][3];
+    __shared__ long id[2 * W][2];
+    const int t = threadIdx.x;
+    for (int w = RED_THREADS / 2; w >= W; w >>= 1) {
+        if (t >= w && t < 2 * w) {
+            v[t - w][0] = all.v; id[t - w][0] = all.i;
+            v[t - w][1] = first.v; id[t - w][1] = first.i;
+            v[t - w][2] = ss;
+        }
+        __syncthreads();
+        if (t < w) {
+            all = amax_join(all, {v[t][0], id[t][0]});
+            first = amax_join(first, {v[t][1], id[t][1]});
+            ss = ss + v[t][2];
+        }
+        __syncthreads();
+    }
+    if (t >= W) return;
+    for (int w = W / 2; w > 0; w >>= 1) {
+        all = amax_join(all, {__shfl_down(all.v, w), __shfl_down(all.i, w)});
+        first = amax_join(first, {__shfl_down(first.v, w), __shfl_down(first.i, w)});
+        ss = ss + __shfl_down(ss, w);
+    }
+}
+
 SMAC_DEV void b_resid_partial(const Blk &bk, Dims d, const double *__restrict__ s,
                               const double *__restrict__ dj, double *__restrict__ part_v,
                               long *__restrict__ part_i, double *__restrict__ part_s)
@@ -592,32 +624,19 @@ SMAC_DEV void b_resid_partial(const Blk &bk, Dims d, const double *__restrict__ 
     double ss = 0.0;
     for (long i = (long)bk.x * blockDim.x + threadIdx.x; i < n3;
          i += (long)bk.nx * blockDim.x) {
-        long p = i % N;
+        const long p = i < N ? i : i < 2 * N ? i - N : i - 2 * N;
         double sv = s[i];
         double a = fabs(sv * dj[p]);
         all = amax_join(all, {a, i});
         if (i < N) first = amax_join(first, {a, i});
         ss += sv * sv;
     }
-    __shared__ double sv_[RED_THREADS], fv_[RED_THREADS], sq_[RED_THREADS];
-    __shared__ long si_[RED_THREADS], fi_[RED_THREADS];
     const int t = threadIdx.x;
-    sv_[t] = all.v; si_[t] = all.i; fv_[t] = first.v; fi_[t] = first.i; sq_[t] = ss;
-    __syncthreads();
-    for (int w = RED_THREADS / 2; w > 0; w >>= 1) {
-        if (t < w) {
-            ArgMax a = amax_join({sv_[t], si_[t]}, {sv_[t + w], si_[t + w]});
-            sv_[t] = a.v; si_[t] = a.i;
-            ArgMax b = amax_join({fv_[t], fi_[t]}, {fv_[t + w], fi_[t + w]});
-            fv_[t] = b.v; fi_[t] = b.i;
-            sq_[t] = sq_[t] + sq_[t + w];
-        }
-        __syncthreads();
-    }
+    red_tree(all, first, ss);
     if (t == 0) {
-        part_v[2 * bk.x] = sv_[0]; part_i[2 * bk.x] = si_[0];
-        part_v[2 * bk.x + 1] = fv_[0]; part_i[2 * bk.x + 1] = fi_[0];
-        part_s[bk.x] = sq_[0];
+        part_v[2 * bk.x] = all.v; part_i[2 * bk.x] = all.i;
+        part_v[2 * bk.x + 1] = first.v; part_i[2 * bk.x + 1] = first.i;
+        part_s[bk.x] = ss;
     }
 }
 
@@ -641,24 +660,11 @@ SMAC_DEV void b_resid_final(const Dims &d, int nparts, int nt, double beta,
         first = amax_join(first, {part_v[2 * b + 1], part_i[2 * b + 1]});
         ss += part_s[b];
     }
-    __shared__ double sv_[RED_THREADS], fv_[RED_THREADS], sq_[RED_THREADS];
-    __shared__ long si_[RED_THREADS], fi_[RED_THREADS];
-    sv_[t] = all.v; si_[t] = all.i; fv_[t] = first.v; fi_[t] = first.i; sq_[t] = ss;
-    __syncthreads();
-    for (int w = RED_THREADS / 2; w > 0; w >>= 1) {
-        if (t < w) {
-            ArgMax a = amax_join({sv_[t], si_[t]}, {sv_[t + w], si_[t + w]});
-            sv_[t] = a.v; si_[t] = a.i;
-            ArgMax b = amax_join({fv_[t], fi_[t]}, {fv_[t + w], fi_[t + w]});
-            fv_[t] = b.v; fi_[t] = b.i;
-            sq_[t] = sq_[t] + sq_[t + w];
-        }
-        __syncthreads();
-    }
+    red_tree(all, first, ss);
     if (t == 0) {
         const long N = d.N;
-        long irmax = si_[0];                 // 0-based index into the 3N array
-        long id = fi_[0];
+        long irmax = all.i;                  // 0-based index into the 3N array
+        long id = first.i;
         int bad = 0;
         // an all-NaN residual leaves no candidate: report it instead of indexing with it
         if (irmax < 0 || irmax >= 3 * N) { irmax = 0; bad = 1; }
@@ -672,7 +678,7 @@ SMAC_DEV void b_resid_final(const Dims &d, int nparts, int nt, double beta,
             if (st->resmax0 < 1.) st->resmax0 = 1.0;
         }
         st->divmax = fabs(s[id] * dj[id] / beta);
-        st->rhsnorm = sqrt(sq_[0]);
+        st->rhsnorm = sqrt(ss);
         st->nonfinite = bad || !(st->rhsnorm <= 1.0e300);
     }
 }
