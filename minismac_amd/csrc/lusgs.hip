@@ -75,14 +75,20 @@ template <> struct Form<3, double> {
     static constexpr int RING = 24, FLY = 4;       // steps in the LDS ring; in flight per loader
     static constexpr int AHEAD = 2;                 // steps the LDS reads run ahead
     static constexpr bool Y_BWD = false;            // forward result into the backward chunk
+    static constexpr int SKEW = 0;                  // steps that four rows run behind the four before
+    static constexpr int EDGE = 4;                  // words of a step's hand-over values
 };
 template <> struct Form<3, float> {
     static constexpr int ROWS = 16, FB = 1536, BB = 1536;
     static constexpr int IMG = 1536, BOWN = 1536;
     static constexpr int RG = 0, RS = 48, RC = 16, RO = 12;
+    // more in flight (FLY) and the loaders, who count a step as landed FLY of their steps later,
+    // run out of ring: 11 323 -> 330 us a pass, 13 486; 7 or a longer ring gains nothing
     static constexpr int RING = 48, FLY = 9;
     static constexpr int AHEAD = 2;
     static constexpr bool Y_BWD = true;
+    static constexpr int SKEW = AHEAD;
+    static constexpr int EDGE = 20;
 };
 template <> struct Form<1, double> {
     static constexpr int ROWS = 64, FB = 2048, BB = 1024;
@@ -91,6 +97,8 @@ template <> struct Form<1, double> {
     static constexpr int RING = 36, FLY = 6;
     static constexpr int AHEAD = 2;
     static constexpr bool Y_BWD = false;
+    static constexpr int SKEW = 0;
+    static constexpr int EDGE = 4;
 };
 
 // the forward / backward chunk of rows tile*ROWS.. of hyperplane h
@@ -158,7 +166,7 @@ SMAC_DEV void lu_solve3_fma(const float f[9], float r1, float r2, float r3, floa
 // 464 bytes a point took 215 us), at 945x241 34 us (was 48).
 
 constexpr int TH = 16, TILE_THREADS = 256;
-constexpr int OVER = 8;
+template <class F> constexpr int OVER = 8 + 3 * F::SKEW;   // steps past a band's ends, at most
 constexpr int IMG_PAD = 16;      // bytes between the tile's chunks in LDS: the 16 hyperplanes of
                                  // one row land in different banks
 
@@ -195,7 +203,7 @@ SMAC_DEV void b_shear(const Blk &bk, const Dims &d, const LusgsWs &w,
     // the tiles the sweeps may touch: they run less than OVER steps past a band's ends (those
     // chunks are reset to zeros too), and a band of fewer rows may reach over a tile's edge
     const int tile = bk.y, k0 = tile * F::ROWS, h0 = (int)bk.x * TH - HP0;
-    const int over = OVER + (w.rows == F::ROWS ? 0 : F::ROWS);
+    const int over = OVER<F> + (w.rows == F::ROWS ? 0 : F::ROWS);
     if (h0 + TH <= k0 - over || h0 > d.jm + k0 + F::ROWS + over) return;
     const int nh = w.H + HP0 + 1 - h0 < TH ? w.H + HP0 + 1 - h0 : TH;   // hyperplanes of the tile
     const long fpitch = (long)(w.ks / F::ROWS) * F::FB, bpitch = (long)(w.ks / F::ROWS) * F::BB;
@@ -451,9 +459,22 @@ template <int NEQ> static unsigned mid_blocks(const LusgsWs &w)
 //
 // What bounds a sweep: its chain of jmax + kmax - 1 steps, each as long as the computing
 // wavefront takes to issue it -- a wavefront alone on its SIMD issues one VALU instruction
-// per 5 cycles (measured), so about 68 instructions FP64 make 144 ns, 31 FP32 70 ns -- and the
-// hand-over lag of 2 us per band beyond the 16 rows' own skew.  At 945x241 the forward sweep
-// takes 215 us FP64, 112 us FP32 and 64-80 us for the scalar system; with one row per lane,
+// per 5 cycles (measured), so about 68 instructions FP64 make 144 ns, 22 FP32 60 ns -- and the
+// hand-over lag of 2 us per band beyond the 16 rows' own skew.  The hand-over wavefront shares
+// the computing one's SIMD, which therefore runs at a higher priority (backward sweep 218 -> 209
+// us, an LU-SGS solve at 477x121 253.5 -> 250).
+//
+// The FP32 step has no 3x3 substitution, so what it issued was mostly moves: three results
+// broadcast in the quad, each passed to the next row by two moves (one inside a row of 16 lanes,
+// one across), and selects.  Its fused multiply-adds now take the quad's values themselves; a
+// lane passes its own equation on with one move; and across the rows of 16 lanes, which have no
+// such move for four lanes at once, a result goes through LDS with the hand-over values: four
+// rows run SKEW steps behind the four before, 90 more steps at 945x241.  A pass there 347 -> 324
+// us, each sweep 112 -> 105.  FP64 keeps the moves: it would save 4 of 68 instructions and pay
+// 8% more steps.
+//
+// At 945x241 the forward sweep takes 215 us FP64, 105 us FP32 and 64 us for the scalar system;
+// with one row per lane,
 // 64-row bands and an s_barrier per step it took 318, 215 and 130-150 us (whose step moved 15 KB
 // through one CU, next to 51 FP64 operations in every lane); at 1889x481 848 -> 438 us FP64.
 constexpr int SUB = 4;           // steps between two looks at the counters
@@ -561,12 +582,12 @@ SMAC_DEV void slot_value(unsigned long long e, float &v)
 // one lane's operands of a step
 template <int NEQ, typename T> struct Ops {
     T jn[3], kn[3], r, f[9];
-    T e[NEQ];           // the incoming hand-over values
+    T e[sizeof(T) == 4 ? 1 : NEQ];   // the incoming hand-over values (FP32: of this lane's equation)
 };
 
 // the shared state of a band's waves
 template <class F, typename T> struct BandLds {
-    __attribute__((aligned(16))) T edge[F::RING][4];   // the hand-over values
+    __attribute__((aligned(16))) T edge[F::RING][F::EDGE];   // the hand-over values
     __attribute__((aligned(16))) int cnt[4];   // steps landed (loaders), steps handed over
     int consumed;       // steps whose ring slots are free again
     __attribute__((aligned(16))) unsigned char ring[F::RING * F::IMG];
@@ -640,12 +661,7 @@ SMAC_DEV void read_ops(Ops<NEQ, T> &o, const unsigned char *b, const unsigned ch
         o.r = c.x;
         o.f[0] = c.y;
     }
-    if constexpr (NEQ == 3 && sizeof(T) == 4) {
-        typedef float v3 __attribute__((ext_vector_type(3)));
-        const v3 t = *(const v3 *)e;
-#pragma unroll
-        for (int n = 0; n < 3; ++n) o.e[n] = t[n];
-    } else if constexpr (NEQ == 3) {
+    if constexpr (NEQ == 3 && sizeof(T) == 8) {
         // no wider than the three words: a register loaded for nothing is reused at once, and
         // writing it would wait for every LDS read in flight
         typedef double v2 __attribute__((ext_vector_type(2)));
@@ -662,42 +678,75 @@ SMAC_DEV void read_ops(Ops<NEQ, T> &o, const unsigned char *b, const unsigned ch
 // 502-540: the j-term, then the k-term) or the backward part (ref/ilusol.f:353-469 and
 // 560-591: the k-term, then the j-term).  own: the row's result of the step before (in) and
 // of this one (out).  T = double: the reference's arithmetic; float: the scaled form.
-// first part: the sum of this lane's equation
+// first part: the sum of this lane's equation (v: that equation of `own`)
 template <int NEQ, bool FWD, typename T>
-SMAC_DEV T band_sum(const Ops<NEQ, T> &o, const T own[NEQ])
+SMAC_DEV T band_sum(const Ops<NEQ, T> &o, const T own[NEQ], T v)
 {
-    T nb[NEQ];
-#pragma unroll
-    for (int n = 0; n < NEQ; ++n) nb[n] = from_row_before<NEQ>(own[n], o.e[n]);
     T t = o.r;
-    auto part = [&](const T *b, const T *x) {
-#pragma unroll
-        for (int n = 0; n < NEQ; ++n) {
-            if constexpr (sizeof(T) == 4) t = __builtin_fmaf(-b[n], x[n], t);
-            else t = t - b[n] * x[n];
-        }
-    };
-    if constexpr (FWD) {
-        part(o.jn, own);
-        part(o.kn, nb);
+    if constexpr (NEQ == 3 && sizeof(T) == 4) {
+        // t += -b x.  A lane keeps its own equation only: the fused multiply-adds take the three
+        // equations' values from the quad, of the row's last result (v) and of the row before
+        // (x, which is the quad before's v, or e).  A DPP operand is read no sooner than two
+        // instructions after it was written.
+        T x = o.e[0];
+        if constexpr (FWD)
+            asm("s_nop 1\n\t"
+                "v_mov_b32_dpp %1, %2 row_shr:4 row_mask:0xf bank_mask:0xe\n\t"
+                "v_fmac_f32_dpp %0, %2, -%3 quad_perm:[0,0,0,0] row_mask:0xf bank_mask:0xf\n\t"
+                "v_fmac_f32_dpp %0, %2, -%4 quad_perm:[1,1,1,1] row_mask:0xf bank_mask:0xf\n\t"
+                "v_fmac_f32_dpp %0, %2, -%5 quad_perm:[2,2,2,2] row_mask:0xf bank_mask:0xf\n\t"
+                "v_fmac_f32_dpp %0, %1, -%6 quad_perm:[0,0,0,0] row_mask:0xf bank_mask:0xf\n\t"
+                "v_fmac_f32_dpp %0, %1, -%7 quad_perm:[1,1,1,1] row_mask:0xf bank_mask:0xf\n\t"
+                "v_fmac_f32_dpp %0, %1, -%8 quad_perm:[2,2,2,2] row_mask:0xf bank_mask:0xf"
+                : "+&v"(t), "+&v"(x)
+                : "v"(v), "v"(o.jn[0]), "v"(o.jn[1]), "v"(o.jn[2]), "v"(o.kn[0]), "v"(o.kn[1]),
+                  "v"(o.kn[2]));
+        else
+            asm("s_nop 1\n\t"
+                "v_mov_b32_dpp %1, %2 row_shr:4 row_mask:0xf bank_mask:0xe\n\t"
+                "s_nop 1\n\t"
+                "v_fmac_f32_dpp %0, %1, -%6 quad_perm:[0,0,0,0] row_mask:0xf bank_mask:0xf\n\t"
+                "v_fmac_f32_dpp %0, %1, -%7 quad_perm:[1,1,1,1] row_mask:0xf bank_mask:0xf\n\t"
+                "v_fmac_f32_dpp %0, %1, -%8 quad_perm:[2,2,2,2] row_mask:0xf bank_mask:0xf\n\t"
+                "v_fmac_f32_dpp %0, %2, -%3 quad_perm:[0,0,0,0] row_mask:0xf bank_mask:0xf\n\t"
+                "v_fmac_f32_dpp %0, %2, -%4 quad_perm:[1,1,1,1] row_mask:0xf bank_mask:0xf\n\t"
+                "v_fmac_f32_dpp %0, %2, -%5 quad_perm:[2,2,2,2] row_mask:0xf bank_mask:0xf"
+                : "+&v"(t), "+&v"(x)
+                : "v"(v), "v"(o.jn[0]), "v"(o.jn[1]), "v"(o.jn[2]), "v"(o.kn[0]), "v"(o.kn[1]),
+                  "v"(o.kn[2]));
     } else {
-        part(o.kn, nb);
-        part(o.jn, own);
+        T nb[NEQ];
+#pragma unroll
+        for (int n = 0; n < NEQ; ++n) nb[n] = from_row_before<NEQ>(own[n], o.e[n]);
+        auto part = [&](const T *b, const T *x) {
+#pragma unroll
+            for (int n = 0; n < NEQ; ++n) t = t - b[n] * x[n];
+        };
+        if constexpr (FWD) {
+            part(o.jn, own);
+            part(o.kn, nb);
+        } else {
+            part(o.kn, nb);
+            part(o.jn, own);
+        }
     }
     return t;
 }
-// second part: the row's result from its equations' sums r (3x3) or its sum (scalar)
+// second part: the row's result from the equations' sums, t that of this lane's; returns this
+// lane's equation of it (c0, c1: whether that is the first, the second)
 template <int NEQ, typename T>
-SMAC_DEV void band_solve(const Ops<NEQ, T> &o, const T *r, T own[NEQ])
+SMAC_DEV T band_solve(const Ops<NEQ, T> &o, T t, T own[NEQ], bool c0, bool c1)
 {
     if constexpr (NEQ == 3 && sizeof(T) == 8) {
-        lu_solve3<double>(o.f, r[0], r[1], r[2], own);
+        lu_solve3<double>(o.f, quad_lane<0>(t), quad_lane<1>(t), quad_lane<2>(t), own);
+        // kept as selects (not sunk into branches)
+        const T v = keep(c1 ? own[1] : own[2]);
+        return keep(c0 ? own[0] : v);
     } else if constexpr (NEQ == 3) {
         // scaled form: the blocks and the rhs already carry the inverse diagonal
-#pragma unroll
-        for (int n = 0; n < 3; ++n) own[n] = r[n];
+        return t;
     } else {
-        own[0] = o.f[0] * r[0];
+        return own[0] = o.f[0] * t;
     }
 }
 
@@ -718,7 +767,8 @@ SMAC_DEV void band_run(const Dims &d, const LusgsWs &w, int blk)
                   "ring");
     constexpr int NDMA = (F::IMG + 1023) / 1024;
     static_assert(F::FLY * NDMA <= 63, "vmcnt budget");
-    static_assert(SUB < OVER && OVER <= HP0, "the sweeps run past their ends within the padding");
+    static_assert(SUB + F::AHEAD + 3 * F::SKEW <= OVER<F> && OVER<F> <= HP0,
+                  "the sweeps run past their ends within the padding");
     __shared__ BandLds<F, T> L;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nband = w.nband;
     const int b = FWD ? blk : nband - 1 - blk;
@@ -727,7 +777,8 @@ SMAC_DEV void band_run(const Dims &d, const LusgsWs &w, int blk)
     const int nrow = klast - k0 + 1;
     const int dir = FWD ? 1 : -1;
     const int h0 = FWD ? k0 : d.jm - 1 + klast;
-    const int nsteps = d.jm - 1 + nrow;
+    const int nsteps = d.jm - 1 + nrow + (nrow - 1) / 4 * F::SKEW;
+    auto behind = [&](int q) { return q / 4 * F::SKEW; };   // steps that row slot q runs behind
     const int nexec = (nsteps + SUB - 1) / SUB * SUB, nload = nexec + F::AHEAD;
     // row slot q of the band, in sweep order: the row that takes the hand-over is slot 0; slots
     // without a row work on the padding row ks - 1
@@ -738,7 +789,8 @@ SMAC_DEV void band_run(const Dims &d, const LusgsWs &w, int blk)
     // edge regions: forward sweep bands 0..nband-1, backward sweep nband..2*nband-1
     unsigned long long *ebase = w.edge + (FWD ? 0 : (long)nband * w.epitch);
 
-    for (int i = threadIdx.x; i < F::RING * 4; i += BAND_LANES * BAND_WAVES) L.edge[i / 4][i % 4] = (T)0;
+    for (int i = threadIdx.x; i < F::RING * F::EDGE; i += BAND_LANES * BAND_WAVES)
+        L.edge[i / F::EDGE][i % F::EDGE] = (T)0;
     if (threadIdx.x < 4) L.cnt[threadIdx.x] = threadIdx.x == LOADERS && !has_in ? 0x7fffffff : 0;
     if (threadIdx.x == 4) L.consumed = 0;
     __syncthreads();
@@ -765,6 +817,7 @@ SMAC_DEV void band_run(const Dims &d, const LusgsWs &w, int blk)
             const bool own = FWD || o >= F::BOWN;
             src[i] = (own ? fwd_chunk<F>(w, h0, tile) : bwd_chunk<F>(w, h0, tile)) + off;
             pitch[i] = own ? fpitch : bpitch;
+            src[i] -= behind(q) * pitch[i];
         }
         const int first = wave - 1;
         const unsigned landed = lds_addr(&L.cnt[first]), consumed = lds_addr(&L.consumed);
@@ -850,6 +903,7 @@ SMAC_DEV void band_run(const Dims &d, const LusgsWs &w, int blk)
         return;
     }
     // ---- the computing wavefront
+    __builtin_amdgcn_s_setprio(3);
     const int c = NEQ == 3 ? ((lane & 3) < 2 ? lane & 3 : 2) : 0, q = NEQ == 3 ? lane >> 2 : lane;
     const bool c0 = c == 0, c1 = c == 1;
     const int krow = row_of(q), ktile = krow / F::ROWS, kk = krow % F::ROWS;
@@ -857,9 +911,10 @@ SMAC_DEV void band_run(const Dims &d, const LusgsWs &w, int blk)
     constexpr bool YB = FWD && F::Y_BWD;
     char *out = r_of<F>(YB ? bwd_chunk<F>(w, h0, ktile) : fwd_chunk<F>(w, h0, ktile), kk, c);
     const long opitch = YB ? bpitch : fpitch;
+    out -= behind(q) * opitch;
     const rsrc_t rE = mk_rsrc(ebase + (long)b * w.epitch, (unsigned)w.epitch * 8u);
     const unsigned eo = has_out && q == nrow - 1 ? 8u * c : 0x80000000u;
-    unsigned es = (unsigned)(h0 - kout + EPAD) * 32u;
+    unsigned es = (unsigned)(h0 - dir * behind(nrow - 1) - kout + EPAD) * 32u;
 
     // the least of the four counters (three loaders, the hand-over), in every lane
     static_assert(LOADERS == 3, "four counters in one read");
@@ -877,12 +932,17 @@ SMAC_DEV void band_run(const Dims &d, const LusgsWs &w, int blk)
     T own[NEQ];
 #pragma unroll
     for (int n = 0; n < NEQ; ++n) own[n] = (T)0;
+    T v = (T)0;                   // this lane's equation of the row's last result
+    // skewed rows: a step's hand-over values of row slots 0, 4, 8 and 12, four words each; the
+    // lanes of slots 3, 7 and 11 pass theirs on, the others write a word that is not read
+    const int take = F::SKEW > 0 ? lane / 16 * 4 + c : 0;
+    const int pass = lane < 48 && lane % 16 >= 12 ? lane / 16 * 4 + 4 + lane % 4 : 16 + lane % 4;
     constexpr int A = F::AHEAD;
     Ops<NEQ, T> s[A + 1];
     await(A);
 #pragma unroll
     for (int u = 0; u < A; ++u)
-        read_ops<NEQ, T>(s[u], lb + u * F::IMG, rb + u * F::IMG, L.edge[u]);
+        read_ops<NEQ, T>(s[u], lb + u * F::IMG, rb + u * F::IMG, L.edge[u] + take);
     v4i last = {0, 0, 0, 0};
     int st = 0;
     // the step in ring slot u; false once the band is done (looked at every SUB steps)
@@ -898,21 +958,12 @@ SMAC_DEV void band_run(const Dims &d, const LusgsWs &w, int blk)
         }
         if constexpr (u % SUB == SUB / 2) last = counts();
         constexpr int un = (u + A) % R;
-        read_ops<NEQ, T>(s[un % (A + 1)], lb + un * F::IMG, rb + un * F::IMG, L.edge[un]);
-        const T t = band_sum<NEQ, FWD, T>(s[u % (A + 1)], own);
-        T r[3] = {t, t, t};
-        if constexpr (NEQ == 3) {
-            r[0] = quad_lane<0>(t);
-            r[1] = quad_lane<1>(t);
-            r[2] = quad_lane<2>(t);
-        }
-        band_solve<NEQ, T>(s[u % (A + 1)], r, own);
-        T v = own[0];
-        if constexpr (NEQ == 3) {
-            // kept as selects (not sunk into branches)
-            v = keep(c1 ? own[1] : own[2]);
-            v = keep(c0 ? own[0] : v);
-        }
+        read_ops<NEQ, T>(s[un % (A + 1)], lb + un * F::IMG, rb + un * F::IMG, L.edge[un] + take);
+        const T t = band_sum<NEQ, FWD, T>(s[u % (A + 1)], own, v);
+        v = band_solve<NEQ, T>(s[u % (A + 1)], t, own, c0, c1);
+        // to the four rows that run SKEW steps behind: they read it in the next step, for the
+        // step AHEAD of that
+        if constexpr (F::SKEW > 0) L.edge[(u + A + 1) % R][pass] = v;
         *(T *)out = v;                       // slots without a row: padding
         out += opitch;
         unsigned lo, hi;
