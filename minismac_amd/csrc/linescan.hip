@@ -807,7 +807,7 @@ k_lr_sweep(int nline, int len, long N, int count, int first, int step, double un
 // their 128 registers do not hold them, and each line loads its own: FP64 1201x241 31 ms a pass
 // against 53 with the spilled prefetch).  FP32-LHS 945x241: an eta line (241 points) 3.2 us, 5.7
 // without prefetch and with crossbar scans, a xi line (945 points) 6.6, before 12.1; FP64 passes
-// 20.0 ms, before 24.9.
+// 20.0 ms, before 24.9.  (3x3 lines of up to 256 points, FP64 128, take k_lr_walk_ahead.)
 template <typename LT, int NEQ, int NT, int PP>
 __global__ void __launch_bounds__(NT)
 k_lr_walk(int nline, int len, long N, int count, int first, int step, double underr, int assign,
@@ -957,6 +957,275 @@ k_lr_walk(int nline, int len, long N, int count, int first, int step, double und
     }
 }
 
+// The walk of lines of up to NT points with three times the threads.  The matrices of a scan's
+// steps, 27 of a step's 36 multiply-adds and 9 of its 12 exchanges, follow from the operands
+// alone, so two more groups of waves, one for each direction, form them a line ahead and pass
+// them through LDS, and the chain of lines is left with the vectors.  The forward matrices of line
+// l + 1 are written between the barriers S1 and S2 of line l (one in each of its scans), the
+// backward ones between S2 of line l and S1 of line l + 1, while the other direction's are read.
+// FP32-LHS 945x241: an eta line (241 points) 2.4 us instead of 3.2, with one group for both
+// directions 3.0.  The matrices of both directions take 432 bytes (FP64: 864) of LDS a point, so
+// lines of up to 256 (128) points go this way, longer ones that of k_lr_walk.
+template <typename T> struct ScanMats {   // one step's matrix of a lane, in 16-byte pieces
+    static constexpr int W = 16 / sizeof(T), K = 9 / W;
+    typedef T V __attribute__((ext_vector_type(W)));
+};
+
+template <typename LT, int NT> struct ScanLds {
+    using S = ScanMats<LT>;
+    typename S::V v[2][6][S::K][NT];   // direction, step (before step 1..5; after the last)
+    LT x[2][6][NT];
+};
+template <typename LT, int NT>
+SMAC_DEV void mats_put(ScanLds<LT, NT> &L, int dir, int step, int t, const LT *m)
+{
+    using S = ScanMats<LT>;
+#pragma unroll
+    for (int k = 0; k < S::K; ++k) {
+        typename S::V p;
+#pragma unroll
+        for (int e = 0; e < S::W; ++e) p[e] = m[k * S::W + e];
+        L.v[dir][step][k][t] = p;
+    }
+    L.x[dir][step][t] = m[8];
+}
+template <typename LT, int NT>
+SMAC_DEV void mats_get(const ScanLds<LT, NT> &L, int dir, int step, int t, LT *m)
+{
+    using S = ScanMats<LT>;
+#pragma unroll
+    for (int k = 0; k < S::K; ++k) {
+        const typename S::V p = L.v[dir][step][k][t];
+#pragma unroll
+        for (int e = 0; e < S::W; ++e) m[k * S::W + e] = p[e];
+    }
+    m[8] = L.x[dir][step][t];
+}
+
+// a step of the matrices; of the vectors, whose matrix of this lane is m
+template <typename AT, bool FWD, int OFF>
+SMAC_DEV void mats_level(AT *m, int lane)
+{
+    Aff<AT, 3> n, o;
+#pragma unroll
+    for (int e = 0; e < 9; ++e) {
+        n.m[e] = m[e];
+        o.m[e] = lane_shift<OFF, FWD>(m[e], lane);
+    }
+#pragma unroll
+    for (int e = 0; e < 3; ++e) n.v[e] = o.v[e] = (AT)0;
+    aff_after(n, o);
+    const bool has = FWD ? lane >= OFF : lane + OFF < 64;
+#pragma unroll
+    for (int e = 0; e < 9; ++e) m[e] = has ? n.m[e] : m[e];
+}
+template <typename AT, bool FWD, int OFF>
+SMAC_DEV void vec_level(const AT *m, AT *v, int lane)
+{
+    AT o[3], n[3];
+#pragma unroll
+    for (int e = 0; e < 3; ++e) o[e] = lane_shift<OFF, FWD>(v[e], lane);
+    aff_apply<AT, 3>(m, v, o, n);
+    const bool has = FWD ? lane >= OFF : lane + OFF < 64;
+#pragma unroll
+    for (int e = 0; e < 3; ++e) v[e] = has ? n[e] : v[e];
+}
+
+// line_scan of one point a thread with the steps' matrices from LDS: point map (m, v), x the
+// value after it
+template <typename AT, int NT, bool FWD>
+SMAC_DEV void line_scan_ahead(const AT *m, const AT *v0, AT *x, const ScanLds<AT, NT> &L, AT (*tot)[12],
+                              int t)
+{
+    constexpr int NW = NT / 64, D = FWD ? 0 : 1;
+    const int lane = t & 63, wv = t >> 6;
+    AT a[6][9], v[3];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) mats_get(L, D, k, t, a[k]);
+#pragma unroll
+    for (int n = 0; n < 3; ++n) v[n] = v0[n];
+    vec_level<AT, FWD, 1>(m, v, lane);
+    vec_level<AT, FWD, 2>(a[0], v, lane);
+    vec_level<AT, FWD, 4>(a[1], v, lane);
+    vec_level<AT, FWD, 8>(a[2], v, lane);
+    vec_level<AT, FWD, 16>(a[3], v, lane);
+    vec_level<AT, FWD, 32>(a[4], v, lane);
+    if (lane == (FWD ? 63 : 0)) {
+#pragma unroll
+        for (int e = 0; e < 9; ++e) tot[wv][e] = a[5][e];
+#pragma unroll
+        for (int n = 0; n < 3; ++n) tot[wv][9 + n] = v[n];
+    }
+    __syncthreads();
+    AT Y[3], ye[3], cur[3];
+    wave_entry<AT, 3, NW, FWD>(tot, wv, Y);
+    aff_apply<AT, 3>(a[5], v, Y, ye);
+#pragma unroll
+    for (int n = 0; n < 3; ++n) {
+        const AT nb = lane_shift<1, FWD>(ye[n], lane);
+        cur[n] = lane == (FWD ? 0 : 63) ? Y[n] : nb;
+    }
+    aff_apply<AT, 3>(m, v0, cur, x);
+}
+
+template <typename LT, int NT>
+__global__ void __launch_bounds__(3 * NT)
+k_lr_walk_ahead(int nline, int len, long N, int count, int first, int step, double underr,
+                double *__restrict__ dq, const double *__restrict__ s, const LT *__restrict__ op)
+{
+    constexpr int NB = 9, NW = NT / 64;
+    __shared__ ScanLds<LT, NT> L;
+    __shared__ LT lf[NW][12], lb[NW][12];
+    const bool up = step > 0;
+    const int t = threadIdx.x & (NT - 1), lane = t & 63;
+    const bool in = t < len;
+    const LT *pB = op, *pM = op + NB * N, *pC = op + 2 * NB * N,
+             *pNear = op + (up ? 3 : 4) * NB * N, *pFar = op + (up ? 4 : 3) * NB * N;
+    auto line = [&](int idx) {
+        const int l = (first + (idx < count ? idx : count - 1) * step) % nline;
+        return l < 0 ? l + nline : l;
+    };
+    // past the line's end in-range addresses stand, whose values nothing uses
+    const int at0 = in ? t : len - 1;
+    auto load = [&](LT *x, const LT *pl, int l) {
+#pragma unroll
+        for (int e = 0; e < NB; ++e) x[e] = pl[e * N + (long)l * len + at0];
+    };
+    // a point's map: past the line the identity
+    auto map = [&](LT *x) {
+#pragma unroll
+        for (int e = 0; e < NB; ++e) x[e] = in ? x[e] : e % 4 == 0 ? (LT)1 : (LT)0;
+    };
+    // a direction's matrices, formed in registers while that direction's of the line before are
+    // in use, then written to LDS
+    auto produce = [&](auto fwd) {
+        constexpr bool FWD = decltype(fwd)::value;
+        constexpr int D = FWD ? 0 : 1;
+        const LT *pl = FWD ? pM : pC;
+        LT m[NB], a[6][NB];
+        auto form = [&](int next) {
+            map(m);
+            auto keep = [&](int k) {
+#pragma unroll
+                for (int e = 0; e < NB; ++e) a[k][e] = m[e];
+            };
+            mats_level<LT, FWD, 1>(m, lane);
+            keep(0);
+            mats_level<LT, FWD, 2>(m, lane);
+            keep(1);
+            mats_level<LT, FWD, 4>(m, lane);
+            keep(2);
+            mats_level<LT, FWD, 8>(m, lane);
+            keep(3);
+            mats_level<LT, FWD, 16>(m, lane);
+            keep(4);
+            mats_level<LT, FWD, 32>(m, lane);
+            keep(5);
+            load(m, pl, line(next));
+        };
+        auto put = [&]() {
+#pragma unroll
+            for (int k = 0; k < 6; ++k) mats_put(L, D, k, t, a[k]);
+        };
+        load(m, pl, line(0));
+        form(1);
+        if (FWD) put();
+        __syncthreads();   // S0
+        for (int idx = 0; idx < count; ++idx) {
+            if (FWD) form(idx + 2);
+            else put();
+            __syncthreads();   // S1
+            if (FWD) put();
+            else form(idx + 2);
+            __syncthreads();   // S2
+        }
+    };
+    const int group = __builtin_amdgcn_readfirstlane(threadIdx.x / NT);
+    if (group == 1) return produce(std::true_type{});
+    if (group == 2) return produce(std::false_type{});
+    __builtin_amdgcn_s_setprio(3);
+    LT B[NB], M[NB], C[NB], near[NB], far[NB];
+    double rhs[3], fx[3], own[3], done[3];
+    auto loadv = [&](double *x, const double *pl, int l) {
+#pragma unroll
+        for (int n = 0; n < 3; ++n) x[n] = pl[n * N + (long)l * len + at0];
+    };
+    // what a line needs before its scans
+    auto fetch = [&](int l) {
+        const int beyond = up ? l + 1 : l - 1;
+        load(B, pB, l);
+        load(near, pNear, l);
+        load(far, pFar, l);
+        loadv(rhs, s, l);
+        loadv(fx, dq, beyond >= 0 && beyond < nline ? beyond : l);
+    };
+    fetch(line(0));
+    load(M, pM, line(0));
+    load(C, pC, line(0));
+    int lprev = -2;
+    __syncthreads();   // S0
+    for (int idx = 0; idx < count; ++idx) {
+        const int l = line(idx), ln = line(idx + 1);
+        const bool hm = l > 0, hp = l < nline - 1;
+        const bool regm = lprev == l - 1, regp = lprev == l + 1;
+        double r[3];
+        LT bv[3], w[3], x[3];
+#pragma unroll
+        for (int n = 0; n < 3; ++n) r[n] = rhs[n];
+        if (hm) {
+#pragma unroll
+            for (int m = 0; m < 3; ++m) {
+                double y[3];
+#pragma unroll
+                for (int n = 0; n < 3; ++n) y[n] = regm ? done[n] : fx[n];
+                double b = (double)(up ? near : far)[m] * y[0];
+#pragma unroll
+                for (int n = 1; n < 3; ++n) b = b + (double)(up ? near : far)[m + 3 * n] * y[n];
+                r[m] = r[m] - b;
+            }
+        }
+        if (hp) {
+#pragma unroll
+            for (int m = 0; m < 3; ++m) {
+                double y[3];
+#pragma unroll
+                for (int n = 0; n < 3; ++n) y[n] = regp ? done[n] : fx[n];
+                double b = (double)(up ? far : near)[m] * y[0];
+#pragma unroll
+                for (int n = 1; n < 3; ++n) b = b + (double)(up ? far : near)[m + 3 * n] * y[n];
+                r[m] = r[m] - b;
+            }
+        }
+        LT rr[3];
+#pragma unroll
+        for (int n = 0; n < 3; ++n) rr[n] = (LT)r[n];
+#pragma unroll
+        for (int m = 0; m < 3; ++m) {
+            LT acc = B[m] * rr[0];
+#pragma unroll
+            for (int n = 1; n < 3; ++n) acc = acc + B[m + 3 * n] * rr[n];
+            bv[m] = in ? acc : (LT)0;
+        }
+        loadv(own, dq, l);
+        fetch(ln);
+        map(M);
+        line_scan_ahead<LT, NT, true>(M, bv, w, L, lf, t);    // S1
+        load(M, pM, ln);
+        map(C);
+#pragma unroll
+        for (int n = 0; n < 3; ++n) w[n] = in ? w[n] : (LT)0;
+        line_scan_ahead<LT, NT, false>(C, w, x, L, lb, t);    // S2
+        load(C, pC, ln);
+#pragma unroll
+        for (int n = 0; n < 3; ++n) {
+            const double nv = own[n] + underr * ((double)x[n] - own[n]);
+            if (in) dq[n * N + (long)l * len + t] = nv;
+            done[n] = nv;
+        }
+        lprev = l;
+    }
+}
+
 // ------------------------------------------------------------------------------------------
 // natural (j fastest) <-> eta-major (k fastest) transposition of `planes` planes of N
 
@@ -1038,13 +1307,27 @@ static void sweep_launch(hipStream_t sm, int nline, int len, long N, int count, 
 #define WALK(NT, PPV)                                                                           \
     hipLaunchKernelGGL((k_lr_walk<LT, NEQ, NT, PPV>), dim3(1), dim3(NT), 0, sm, nline, len, N,  \
                        count, first, step, underr, assign, dq, s, op)
+#define AHEAD(NT)                                                                               \
+    hipLaunchKernelGGL((k_lr_walk_ahead<LT, NT>), dim3(1), dim3(3 * NT), 0, sm, nline, len, N,  \
+                       count, first, step, underr, dq, s, op)
 #define COLOUR(NT, PPV, TW, TR)                                                                 \
     hipLaunchKernelGGL((k_lr_sweep<LT, NEQ, NT, PPV, TW, TR>), dim3(count), dim3(NT), 0, sm,    \
                        nline, len, N, count, first, step, underr, assign, couple, dq, s, op, ts)
 #define TWISTED(NT, PPV) COLOUR(NT, PPV, true, false)
 #define PLAIN(NT, PPV) COLOUR(NT, PPV, false, false)
 #define TRANSPOSED(NT, PPV) COLOUR(NT, PPV, false, true)
-    if constexpr (FORM == SWEEP_WALK) SWT(WALK);
+    if constexpr (FORM == SWEEP_WALK) {
+        if constexpr (NEQ == 3) {
+            constexpr int MOST = sizeof(LT) == 4 ? 256 : 128;
+            if (len <= 64) AHEAD(64);
+            else if (len <= MOST) AHEAD(MOST);
+            else if (len <= 256) {
+                if constexpr (MOST < 256) WALK(256, 1);
+            } else if (len <= 512) WALK(512, 1);
+            else if (len <= 1024) WALK(512, 2);
+            else WALK(1024, 2);
+        } else SWT(WALK);
+    }
     else if constexpr (FORM == SWEEP_TRANSPOSED) SWT(TRANSPOSED);
     else if (twist) SWT(TWISTED);
     else SWT(PLAIN);
@@ -1052,6 +1335,7 @@ static void sweep_launch(hipStream_t sm, int nline, int len, long N, int count, 
 #undef PLAIN
 #undef TWISTED
 #undef COLOUR
+#undef AHEAD
 #undef WALK
 #undef SWT
 }
