@@ -340,11 +340,21 @@ template <typename LT, int NEQ> static dim3 shear_grid(const Dims &d, const Lusg
                 (unsigned)((d.km + F::ROWS - 1) / F::ROWS));
 }
 
+// The wake-cut injection (bcimpds, ref/bc.f:571-591) of the points that a workgroup of k_unshear
+// writes, on the way: a cut point's new value follows from its pair's dq on the second row, which
+// the workspace holds.  A launch of its own behind k_unshear cost 4 us: 945x241 FP32-LHS passes 323
+// -> 319 us, 119x31 laminar steps 113 -> 111.
+struct WakeIn {
+    WakePairs pairs;
+    const double *sq;
+    double *rhs;          // gets the cut points' values too
+};
+
 // r's place in the forward chunks (dq after the backward sweep, the middle-step rhs before
 // it; FP32-LHS has the latter in the backward chunks) -> natural FP64 planes
 template <int NEQ, typename T>
 SMAC_DEV void b_unshear(const Blk &bk, const Dims &d, const LusgsWs &w, bool mid,
-                        double *__restrict__ dst)
+                        double *__restrict__ dst, const WakeIn &wk)
 {
     using F = Form<NEQ, T>;
     constexpr int UK = 16;                  // rows per workgroup
@@ -357,11 +367,38 @@ SMAC_DEV void b_unshear(const Blk &bk, const Dims &d, const LusgsWs &w, bool mid
         char *ch = mid && F::Y_BWD ? bwd_chunk<F>(w, h0 + hh, tile) : fwd_chunk<F>(w, h0 + hh, tile);
         lds[c][kk][hh] = *(const T *)r_of<F>(ch, kt + kk, c);
     }
+    // the pair of each point on the first row
+    const bool cut = k0 == 0 && wk.pairs.n > 0;
+    __shared__ int pair[TH];
+    if (cut) {
+        if (threadIdx.x < TH) pair[threadIdx.x] = -1;
+        __syncthreads();
+        for (int i = threadIdx.x; i < wk.pairs.n; i += TILE_THREADS) {
+            const long jt = wk.pairs.pairs[2 * i] - wk.pairs.base, jb = wk.pairs.pairs[2 * i + 1] - wk.pairs.base;
+            if (jt < 0 || jt >= d.jm || jb < 0 || jb >= d.jm) continue;
+            if (jt >= h0 && jt < h0 + TH) pair[jt - h0] = (int)jb;
+        }
+    }
     __syncthreads();
     for (int e = threadIdx.x; e < TH * UK; e += TILE_THREADS) {
         const int kk = e / TH, hh = e % TH, k = k0 + kk, j = h0 + hh - k;
         if (j < 0 || j >= d.jm || k >= d.km) continue;
         const long p = P(d, j, k);
+        const int jb = cut && k == 0 ? pair[hh] : -1;
+        if (jb >= 0) {
+            // the second row's points of columns j and jb
+            char *ct = fwd_chunk<F>(w, j + 1, 0), *cb = fwd_chunk<F>(w, jb + 1, 0);
+#pragma unroll
+            for (int m = 0; m < NEQ; ++m) {
+                const double snew = 0.5 * (wk.sq[m * d.N + j + d.jm] + wk.sq[m * d.N + jb + d.jm]);
+                const double dsnew = 0.5 * ((double)*(const T *)r_of<F>(ct, 1, m) +
+                                            (double)*(const T *)r_of<F>(cb, 1, m));
+                const double v = snew + dsnew - wk.sq[m * d.N + j];
+                dst[m * d.N + p] = v;
+                wk.rhs[m * d.N + p] = v;
+            }
+            continue;
+        }
 #pragma unroll
         for (int m = 0; m < NEQ; ++m) dst[m * d.N + p] = (double)lds[m][kk][hh];
     }
@@ -369,9 +406,9 @@ SMAC_DEV void b_unshear(const Blk &bk, const Dims &d, const LusgsWs &w, bool mid
 
 template <int NEQ, typename T>
 __global__ void __launch_bounds__(TILE_THREADS)
-k_unshear(Dims d, LusgsWs w, bool mid, double *__restrict__ dst)
+k_unshear(Dims d, LusgsWs w, bool mid, double *__restrict__ dst, WakeIn wk)
 {
-    b_unshear<NEQ, T>(xcd_blk(), d, w, mid, dst);
+    b_unshear<NEQ, T>(xcd_blk(), d, w, mid, dst, wk);
 }
 
 static dim3 unshear_grid(const Dims &d, const LusgsWs &w)
@@ -1076,8 +1113,7 @@ void lusgs_post(hipStream_t sm, const Dims &d, const LusgsWs &w, const WakePairs
                 const double *q, double *dq, double *rhs)
 {
     hipLaunchKernelGGL((k_unshear<NEQ, LT>), unshear_grid(d, w), dim3(TILE_THREADS), 0, sm, d, w,
-                       false, dq);
-    launch_wake(sm, d, NEQ, wk, q, dq, rhs);
+                       false, dq, WakeIn{wk, q, rhs});
 }
 
 // ---- multi-case launches ------------------------------------------------------------------
@@ -1127,7 +1163,7 @@ struct CUnshear {
     static constexpr int THREADS = TILE_THREADS;
     static SMAC_DEV void run(const Blk &b, const Args &a)
     {
-        b_unshear<NEQ, LT>(b, a.d, ws_global(a.w), false, as_global(a.dst));
+        b_unshear<NEQ, LT>(b, a.d, ws_global(a.w), false, as_global(a.dst), WakeIn{});
     }
 };
 
@@ -1186,7 +1222,7 @@ static void launch_lusgs(hipStream_t sm, const Dims &d, const LusgsWs &w, const 
     lusgs_mid<LT, NEQ>(sm, d, w);
     if (rhs_out)   // before the backward sweep writes dq in its place
         hipLaunchKernelGGL((k_unshear<NEQ, LT>), unshear_grid(d, w), dim3(TILE_THREADS), 0, sm, d, w,
-                           true, rhs);
+                           true, rhs, WakeIn{});
     lusgs_band<LT, NEQ>(sm, d, w, false);
     lusgs_post<LT, NEQ>(sm, d, w, wk, q, dq, rhs);
 }
