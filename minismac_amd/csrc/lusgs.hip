@@ -101,6 +101,18 @@ template <> struct Form<1, double> {
     static constexpr int EDGE = 4;
 };
 
+// The forms of a launch whose bands are more than two per compute unit, as a large batch's are:
+// a shorter ring, of which more fit a compute unit's 160 KB (FP32 four instead of two, scalar
+// three).  64 cases FP32-LHS, 632 bands: forward sweep 0.69 -> 0.585 ms, a pass of all 3.383 -> 3.331 ms;
+// up to two per compute unit the longer ring is the better (12 cases, 112 bands: the single case's).
+template <int NEQ, typename T> struct FormMany : Form<NEQ, T> {};
+template <> struct FormMany<3, float> : Form<3, float> {
+    static constexpr int RING = 24, FLY = 4;
+};
+template <> struct FormMany<1, double> : Form<1, double> {
+    static constexpr int RING = 24, FLY = 5;
+};
+
 // the forward / backward chunk of rows tile*ROWS.. of hyperplane h
 template <class F> SMAC_DEV char *fwd_chunk(const LusgsWs &w, int h, int tile)
 {
@@ -796,10 +808,9 @@ static __device__ __forceinline__ bool ring_round(Fn &f, std::integer_sequence<i
 
 // One band of one case: blk is the band's place in dispatch order (forward bands bottom up,
 // backward bands top down, so that every band is dispatched after the band it waits for).
-template <int NEQ, bool FWD, typename T>
+template <int NEQ, bool FWD, typename T, class F = Form<NEQ, T>>
 SMAC_DEV void band_run(const Dims &d, const LusgsWs &w, int blk)
 {
-    using F = Form<NEQ, T>;
     static_assert(F::RING % SUB == 0 && F::RING % LOADERS == 0 && F::RING % (F::AHEAD + 1) == 0 && F::RING - F::FLY * LOADERS > 2 * SUB,
                   "ring");
     constexpr int NDMA = (F::IMG + 1023) / 1024;
@@ -1033,7 +1044,7 @@ SMAC_DEV LusgsWs ws_global(const LusgsWs &t)
     return w;
 }
 
-template <int NEQ, bool FWD, typename T>
+template <int NEQ, bool FWD, typename T, class F>
 __global__ void __launch_bounds__(BAND_LANES * BAND_WAVES)
 k_band_multi(const BandJob *__restrict__ jobs, const int2 *__restrict__ map,
              const int *__restrict__ active)
@@ -1043,7 +1054,7 @@ k_band_multi(const BandJob *__restrict__ jobs, const int2 *__restrict__ map,
     if (active && active[jobs[m.x].bcase] == 0) return;
     const Dims d = jobs[m.x].d;
     const LusgsWs w = ws_global(jobs[m.x].w);
-    band_run<NEQ, FWD, T>(d, w, m.y);
+    band_run<NEQ, FWD, T, F>(d, w, m.y);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1095,10 +1106,16 @@ void lusgs_band_multi(hipStream_t sm, const BandJob *jobs, const int2 *map, int 
 {
     if (nblk <= 0) return;
     const dim3 blk(BAND_LANES * BAND_WAVES);
-    if (fwd)
-        hipLaunchKernelGGL((k_band_multi<NEQ, true, LT>), dim3(nblk), blk, 0, sm, jobs, map, active);
-    else
-        hipLaunchKernelGGL((k_band_multi<NEQ, false, LT>), dim3(nblk), blk, 0, sm, jobs, map, active);
+    constexpr int FULL = 2 * 256;   // two bands on each compute unit
+    auto launch = [&](auto form) {
+        using F = decltype(form);
+        if (fwd)
+            hipLaunchKernelGGL((k_band_multi<NEQ, true, LT, F>), dim3(nblk), blk, 0, sm, jobs, map, active);
+        else
+            hipLaunchKernelGGL((k_band_multi<NEQ, false, LT, F>), dim3(nblk), blk, 0, sm, jobs, map, active);
+    };
+    if (FormMany<NEQ, LT>::RING < Form<NEQ, LT>::RING && nblk > FULL) launch(FormMany<NEQ, LT>{});
+    else launch(Form<NEQ, LT>{});
 }
 
 template <typename LT, int NEQ>
