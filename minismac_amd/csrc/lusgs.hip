@@ -101,16 +101,14 @@ template <> struct Form<1, double> {
     static constexpr int EDGE = 4;
 };
 
-// The forms of a launch whose bands are more than two per compute unit, as a large batch's are:
-// a shorter ring, of which more fit a compute unit's 160 KB (FP32 four instead of two, scalar
-// three).  64 cases FP32-LHS, 632 bands: forward sweep 0.69 -> 0.585 ms, a pass of all 3.383 -> 3.331 ms;
-// up to two per compute unit the longer ring is the better (12 cases, 112 bands: the single case's).
+// The FP32 form of a launch whose bands are more than two per compute unit, as a large batch's
+// are: a shorter ring, of which four fit a compute unit's 160 KB instead of two.  64 cases
+// FP32-LHS, 632 bands: forward sweep 0.69 -> 0.585 ms, a pass of all 3.383 -> 3.331 ms.  Where the
+// long rings fit they are the better: 112 bands (12 cases) 687 us a pass against 750, 224 bands
+// 1070 against 1100, 448 bands 2005 against 2009.
 template <int NEQ, typename T> struct FormMany : Form<NEQ, T> {};
 template <> struct FormMany<3, float> : Form<3, float> {
     static constexpr int RING = 24, FLY = 4;
-};
-template <> struct FormMany<1, double> : Form<1, double> {
-    static constexpr int RING = 24, FLY = 5;
 };
 
 // the forward / backward chunk of rows tile*ROWS.. of hyperplane h
@@ -1114,8 +1112,9 @@ void lusgs_band_multi(hipStream_t sm, const BandJob *jobs, const int2 *map, int 
         else
             hipLaunchKernelGGL((k_band_multi<NEQ, false, LT, F>), dim3(nblk), blk, 0, sm, jobs, map, active);
     };
-    if (FormMany<NEQ, LT>::RING < Form<NEQ, LT>::RING && nblk > FULL) launch(FormMany<NEQ, LT>{});
-    else launch(Form<NEQ, LT>{});
+    if constexpr (FormMany<NEQ, LT>::RING < Form<NEQ, LT>::RING)
+        if (nblk > FULL) return launch(FormMany<NEQ, LT>{});
+    launch(Form<NEQ, LT>{});
 }
 
 template <typename LT, int NEQ>
