@@ -1227,16 +1227,21 @@ k_lr_walk_ahead(int nline, int len, long N, int count, int first, int step, doub
 }
 
 // ------------------------------------------------------------------------------------------
-// natural (j fastest) <-> eta-major (k fastest) transposition of `planes` planes of N
+// natural (j fastest) <-> eta-major (k fastest) transposition of the three planes of N of one
+// array, or of two in one launch: at these sizes a launch costs as much as its traffic (945x241
+// 5.5 us for 11 MB)
 
 constexpr int TT = 32;
 
 __global__ void __launch_bounds__(256)
-k_transpose(const double *__restrict__ src, double *__restrict__ dst, int rows, int cols, long N)
+k_transpose(const double *__restrict__ src0, double *__restrict__ dst0,
+            const double *__restrict__ src1, double *__restrict__ dst1, int rows, int cols, long N)
 {
     // src plane: rows x cols, cols fastest; dst plane: cols x rows, rows fastest
     __shared__ double tile[TT][TT + 1];
-    const long base = (long)blockIdx.z * N;
+    const long base = (long)(blockIdx.z % 3) * N;
+    const double *src = blockIdx.z < 3 ? src0 : src1;
+    double *dst = blockIdx.z < 3 ? dst0 : dst1;
     const int c0 = blockIdx.x * TT, r0 = blockIdx.y * TT;
     for (int rr = threadIdx.y; rr < TT; rr += 8) {
         const int r = r0 + rr, c = c0 + threadIdx.x;
@@ -1249,18 +1254,20 @@ k_transpose(const double *__restrict__ src, double *__restrict__ dst, int rows, 
     }
 }
 
-static void transpose(hipStream_t sm, const double *src, double *dst, int rows, int cols, long N,
-                      int planes)
+static void transpose(hipStream_t sm, int rows, int cols, long N, const double *src, double *dst,
+                      const double *src1 = nullptr, double *dst1 = nullptr)
 {
-    dim3 g((cols + TT - 1) / TT, (rows + TT - 1) / TT, planes);
-    hipLaunchKernelGGL(k_transpose, g, dim3(TT, 8), 0, sm, src, dst, rows, cols, N);
+    dim3 g((cols + TT - 1) / TT, (rows + TT - 1) / TT, src1 ? 6 : 3);
+    hipLaunchKernelGGL(k_transpose, g, dim3(TT, 8), 0, sm, src, dst, src1, dst1, rows, cols, N);
 }
 
 // wake-cut injection (bcimpds single-rank branch, ref/bc.f:571-591) with ds and rhs in the
-// eta-major layout; q stays natural.  Pairs outside the row are skipped.
+// eta-major layout; q stays natural, and the natural rhs, which differs from the eta-major one in
+// these points only, gets their values too.  Pairs outside the row are skipped.
 __global__ void k_wake_eta(long N, int jm, int km, int neqs, int npair, int base,
                            const int *__restrict__ pairs, const double *__restrict__ sq,
-                           double *__restrict__ ds, double *__restrict__ rhs)
+                           double *__restrict__ ds, double *__restrict__ rhs,
+                           double *__restrict__ rhs_nat)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= npair) return;
@@ -1271,7 +1278,7 @@ __global__ void k_wake_eta(long N, int jm, int km, int neqs, int npair, int base
         double snew = 0.5 * (sq[n * N + jt + jm] + sq[n * N + jb + jm]);
         double dsnew = 0.5 * (ds[n * N + t1] + ds[n * N + b1]);
         ds[n * N + t0] = snew + dsnew - sq[n * N + jt];
-        rhs[n * N + t0] = ds[n * N + t0];
+        rhs[n * N + t0] = rhs_nat[n * N + jt] = ds[n * N + t0];
     }
 }
 
@@ -1396,16 +1403,14 @@ void launch_lrelax_scan(hipStream_t sm, const Dims &d, const DevParams &prm, int
         if ((nj / nbcimp) * nbcimp == nj) launch_wake(sm, d, 3, w, q, dq, s);
     }
     if (nksp > 0) {
-        transpose(sm, s, ws.s_t, d.km, d.jm, N, 3);
-        transpose(sm, dq, ws.dq_t, d.km, d.jm, N, 3);
+        transpose(sm, d.km, d.jm, N, s, ws.s_t, dq, ws.dq_t);
         for (int nk = 1; nk <= nksp; ++nk) {
             sweep<LT, 3>(sm, d.jm, d.km, N, nk, zebra, tw, prm.underr, ws.dq_t, ws.s_t, ope);
             if ((nk / nbcimp) * nbcimp == nk && w.n > 0)
                 hipLaunchKernelGGL(k_wake_eta, dim3((w.n + 63) / 64), dim3(64), 0, sm, N, d.jm,
-                                   d.km, 3, w.n, w.base, w.pairs, q, ws.dq_t, ws.s_t);
+                                   d.km, 3, w.n, w.base, w.pairs, q, ws.dq_t, ws.s_t, s);
         }
-        transpose(sm, ws.dq_t, dq, d.jm, d.km, N, 3);
-        transpose(sm, ws.s_t, s, d.jm, d.km, N, 3);
+        transpose(sm, d.jm, d.km, N, ws.dq_t, dq);
     }
 }
 

@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 
 import pyoracle
-from minismac_amd._abi import SMAC_FP32_LHS, SMAC_FP64
+from minismac_amd._abi import SMAC_FP32_LHS, SMAC_FP64, SMAC_ORDER_REFERENCE, SMAC_ORDER_ZEBRA
 from minismac_amd.case import naca_case
 from minismac_amd.solver import Solver
 
@@ -51,3 +51,22 @@ def test_walk_follows_the_sequential_form(jm, km):
     ref, tol = _dq(case, False), 1000 * _sens(case)
     assert np.abs(_dq(case, True) - ref).max() <= tol * 2.0 ** -29
     assert np.abs(_dq(_case(jm, km, SMAC_FP32_LHS), True) - ref).max() <= tol
+
+
+@pytest.mark.parametrize("precision", [SMAC_FP64, SMAC_FP32_LHS])
+@pytest.mark.parametrize("order", [SMAC_ORDER_REFERENCE, SMAC_ORDER_ZEBRA])
+def test_cut_rows_of_the_rhs(order, precision):
+    """After a pass whose last sweeps are eta ones the natural right-hand side holds the injected
+    values in the cut's points, as dq does, and the assembled ones everywhere else."""
+    case = naca_case(63, 17, impsch=1, alpha=3.0, reynum=1e3, wall_spacing=1e-3, dtau=0.1, underr=0.3,
+                     iturb=0, precision=precision, line_order=order)
+    o = pyoracle.Oracle(case)
+    o.step()
+    with Solver(case, options={"lr_solve": 1}) as g:
+        g.step()
+        s, dq = g.array("s"), g.array("dq")
+    cut = np.unique(case.wake_pairs()[:, 0]) - 1
+    assert np.array_equal(s[cut, 0], dq[cut, 0])
+    rest = np.ones(s.shape[:2], bool)
+    rest[cut, 0] = False
+    assert np.array_equal(s[rest], o.array("s")[rest])
