@@ -1145,7 +1145,7 @@ struct smac_batch {
     MultiTab<SaUpdArgs> sa_upd;
     MultiTab<SaTurArgs> sa_tur;
     MultiTab<AsmArgs> asm_[2];       // [0] FP64 cases, [1] FP32-LHS cases
-    MultiTab<BcArgs> bc[2];
+    std::vector<MultiTab<BcArgs>> bc[2];   // one launch after the other, see build_multi
     MultiTab<ResidPArgs> resp;
     MultiTab<ResidFArgs> resf;
     MultiTab<ShearArgs> shear[2];
@@ -1215,8 +1215,9 @@ static void free_multi(smac_batch *b)
     mt_free(b->sa_tur); mt_free(b->resp); mt_free(b->resf); mt_free(b->wake); mt_free(b->upd);
     mt_free(b->force);
     for (int g = 0; g < 2; ++g) {
-        mt_free(b->asm_[g]); mt_free(b->bc[g]); mt_free(b->shear[g]); mt_free(b->mid[g]);
-        mt_free(b->unshear[g]);
+        mt_free(b->asm_[g]); mt_free(b->shear[g]); mt_free(b->mid[g]); mt_free(b->unshear[g]);
+        for (MultiTab<BcArgs> &t : b->bc[g]) mt_free(t);
+        b->bc[g].clear();
     }
 }
 
@@ -1301,7 +1302,10 @@ static smac_status build_multi(smac_batch *b)
     Items<SaUpdArgs> sup;
     Items<SaTurArgs> stu;
     Items<AsmArgs> as[2];
-    Items<BcArgs> bc[2];
+    // A case's regions go BC_MAX to an item, and a point that regions of two items share takes
+    // the rows of the later one: so a case's first items are one launch, its second ones the next.
+    std::vector<Items<BcArgs>> bc[2];
+    std::vector<BcArgs> bc_case;
     Items<ResidPArgs> rp;
     Items<ResidFArgs> rf;
     Items<UpdArgs> up;
@@ -1330,7 +1334,7 @@ static smac_status build_multi(smac_batch *b)
             as[g].v.push_back(asm_args<float>(d, dp, h->q, h->met, h->dj, h->s, fb[0], fb[1], fb[2],
                                             fb[3], fb[4]));
             bc_args<float>(d, dp, h->regs.data(), (int)h->regs.size(), h->st, h->x, h->y, h->met,
-                           h->q, h->s, fb[0], fb[1], fb[2], fb[3], fb[4], bc[g].v);
+                           h->q, h->s, fb[0], fb[1], fb[2], fb[3], fb[4], bc_case);
             sh[g].v.push_back(shear_args<float, 3>(d, h->lws, h->s, fb[0], fb[1], fb[2], fb[3], fb[4],
                                               (float *)nullptr));
             mid[g].v.push_back(mid_args<float, 3>(d, h->lws));
@@ -1339,7 +1343,7 @@ static smac_status build_multi(smac_batch *b)
             as[g].v.push_back(asm_args<double>(d, dp, h->q, h->met, h->dj, h->s, db[0], db[1],
                                              db[2], db[3], db[4]));
             bc_args<double>(d, dp, h->regs.data(), (int)h->regs.size(), h->st, h->x, h->y,
-                            h->met, h->q, h->s, db[0], db[1], db[2], db[3], db[4], bc[g].v);
+                            h->met, h->q, h->s, db[0], db[1], db[2], db[3], db[4], bc_case);
             sh[g].v.push_back(shear_args<double, 3>(d, h->lws, h->s, db[0], db[1], db[2], db[3], db[4],
                                                (double *)nullptr));
             mid[g].v.push_back(mid_args<double, 3>(d, h->lws));
@@ -1354,8 +1358,14 @@ static smac_status build_multi(smac_batch *b)
         sd.tag(i); sas.tag(i); sbc.tag(i); ssh.tag(i); smid.tag(i); sun.tag(i); swk.tag(i);
         sup.tag(i); stu.tag(i); rp.tag(i); rf.tag(i); wk.tag(i); up.tag(i); fo.tag(i);
         for (int gg = 0; gg < 2; ++gg) {
-            as[gg].tag(i); bc[gg].tag(i); sh[gg].tag(i); mid[gg].tag(i); un[gg].tag(i);
+            as[gg].tag(i); sh[gg].tag(i); mid[gg].tag(i); un[gg].tag(i);
         }
+        if (bc[g].size() < bc_case.size()) bc[g].resize(bc_case.size());
+        for (size_t r = 0; r < bc_case.size(); ++r) {
+            bc[g][r].v.push_back(bc_case[r]);
+            bc[g][r].tag(i);
+        }
+        bc_case.clear();
     }
     B_TRY(mt_build(b->sa_deriv, sd, b->active));
     B_TRY(mt_build(b->sa_asm, sas, b->active));
@@ -1368,7 +1378,8 @@ static smac_status build_multi(smac_batch *b)
     B_TRY(mt_build(b->sa_tur, stu, b->active));
     for (int g = 0; g < 2; ++g) {
         B_TRY(mt_build(b->asm_[g], as[g], b->active));
-        B_TRY(mt_build(b->bc[g], bc[g], b->active));
+        b->bc[g].resize(bc[g].size());
+        for (size_t r = 0; r < bc[g].size(); ++r) B_TRY(mt_build(b->bc[g][r], bc[g][r], b->active));
         B_TRY(mt_build(b->shear[g], sh[g], b->active));
         B_TRY(mt_build(b->mid[g], mid[g], b->active));
         B_TRY(mt_build(b->unshear[g], un[g], b->active));
@@ -1475,8 +1486,8 @@ static smac_status enqueue_batch_pass_multi(smac_batch *b, bool time_band)
     // mean flow up to its band sweeps
     multi_assemble<double>(sm, b->asm_[0]);
     multi_assemble<float>(sm, b->asm_[1]);
-    multi_bc<double>(sm, b->bc[0]);
-    multi_bc<float>(sm, b->bc[1]);
+    for (const MultiTab<BcArgs> &t : b->bc[0]) multi_bc<double>(sm, t);
+    for (const MultiTab<BcArgs> &t : b->bc[1]) multi_bc<float>(sm, t);
     multi_resid_partial(sm, b->resp);
     multi_resid_final(sm, b->resf);
     multi_shear<double, 3>(sm, b->shear[0]);

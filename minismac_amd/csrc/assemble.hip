@@ -431,10 +431,11 @@ k_assemble(Dims d, DevParams prm, int rows, const double *__restrict__ q,
 }
 
 // ---------------------------------------------------------------------------------------
-// BC rows (ref/bc.f): every region of the case in one launch.  A region writes only its own
-// points' rows and reads nothing that a region writes, so regions meet only in the points they
-// share: one thread does all of a point's regions, in file order, and a later region's rows win
-// as in the reference's sequence of calls.
+// BC rows (ref/bc.f): BC_MAX regions of the case in one launch, more in further ones in file
+// order (in a batch too).  A region writes only its own points' rows and reads nothing that a
+// region writes, so regions meet only in the points they share: one thread does all of a point's
+// regions in the launch, in file order, and a later region's rows win as in the reference's
+// sequence of calls.
 //
 // Bound by the latency of one point's chain of loads and of the far field's cosine, sine and
 // divisions: 4.8 us at 945x241 and 10.5 at 1889x481 beside the SA,
