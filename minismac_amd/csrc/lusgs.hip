@@ -105,7 +105,10 @@ template <> struct Form<1, double> {
 // are: a shorter ring, of which four fit a compute unit's 160 KB instead of two.  64 cases
 // FP32-LHS, 632 bands: forward sweep 0.69 -> 0.585 ms, a pass of all 3.383 -> 3.331 ms.  Where the
 // long rings fit they are the better: 112 bands (12 cases) 687 us a pass against 750, 224 bands
-// 1070 against 1100, 448 bands 2005 against 2009.
+// 1070 against 1100, 448 bands 2005 against 2009.  (One row per lane in 64-row bands, of which
+// these cases had 158, took 0.32 ms for this sweep and 3.54 for the pass: where the chip is full
+// of bands the sixteen-row ones lose in the sweeps what their hand-overs cost, and the pass gains
+// from the other kernels.)
 template <int NEQ, typename T> struct FormMany : Form<NEQ, T> {};
 template <> struct FormMany<3, float> : Form<3, float> {
     static constexpr int RING = 24, FLY = 4;
@@ -899,51 +902,41 @@ SMAC_DEV void band_run(const Dims &d, const LusgsWs &w, int blk)
     }
     if (wave == LOADERS + 1) {
         // ---- hand-over: the words of BS steps per poll, one word per lane; the prefix of them
-        // that has been written goes to LDS.  POLLS polls are in flight one after another, so
-        // that a slot is seen a fraction of a memory round trip after it was written.
+        // that has been written goes to LDS.  One poll at a time: with four in flight a slot is
+        // seen sooner, but the waves' polls (each up to 63 words in as many sectors, past the
+        // caches) hold up one another and the operands: 945x241 alone FP64 558 us a pass instead
+        // of 548, a batch of 64 cases 5.16 ms instead of 5.10, FP32-LHS 3.39 instead of 3.36.
         if (!has_in) return;
-        constexpr int BS = F::RING < 21 ? F::RING : (NEQ == 3 ? 21 : F::RING), POLLS = 4;
+        constexpr int BS = F::RING < 21 ? F::RING : (NEQ == 3 ? 21 : F::RING);
         const int i = lane / NEQ, word = lane % NEQ;
         // the slot of column j = h - kin
         const unsigned long long *p0 = ebase + (long)(b - dir) * w.epitch +
                                        (long)(h0 - kin + EPAD) * 4 + word;
-        unsigned long long v[POLLS];
-        int from[POLLS];               // the first step of each poll
         int base = 0, lim = F::RING, spin = 0;
         bool broken = false;
-        auto poll = [&](int d) {
-            const int st = base + i < nload ? base + i : nload - 1;
-            from[d] = base;
-            v[d] = __hip_atomic_load(p0 + (long)dir * st * 4, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        };
-#pragma unroll
-        for (int d = 0; d < POLLS; ++d) poll(d);
         while (base < nload) {
-#pragma unroll
-            for (int d = 0; d < POLLS; ++d) {
-                if (base + BS > lim) lim = cnt_ld(&L.consumed) + F::RING;
-                const int st = from[d] + i;
-                const int top = from[d] + BS < lim ? from[d] + BS : lim;
-                const int end = top < nload ? top : nload;    // steps this poll may hand over
-                const bool none = edge_empty(v[d]) && !broken;
-                const unsigned long long missing =
-                    __builtin_amdgcn_ballot_w64(none && i < BS && st >= base && st < end);
-                const int upto = missing ? from[d] + __builtin_ctzll(missing) / NEQ : end;
-                if (upto > base) {
-                    if (i < BS && st >= base && st < upto) {
-                        T x;
-                        slot_value(edge_empty(v[d]) ? 0ull : v[d], x);
-                        L.edge[st % F::RING][word] = x;
-                    }
-                    asm volatile("" ::: "memory");
-                    base = upto;
-                    if (lane == 0) cnt_st(&L.cnt[LOADERS], base < nload ? base : 0x7fffffff);
-                    spin = 0;
-                } else if (base < lim && ++spin > EDGE_SPIN_MAX) {
-                    broken = true;
-                    if (lane == 0) atomicOr(w.stall, 1);
+            const int st = base + i;
+            const unsigned long long v = __hip_atomic_load(
+                p0 + (long)dir * (st < nload ? st : nload - 1) * 4, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (base + BS > lim) lim = cnt_ld(&L.consumed) + F::RING;
+            const int top = base + BS < lim ? base + BS : lim;
+            const int end = top < nload ? top : nload;    // steps this poll may hand over
+            const bool none = edge_empty(v) && !broken;
+            const unsigned long long missing = __builtin_amdgcn_ballot_w64(none && i < BS && st < end);
+            const int upto = missing ? base + __builtin_ctzll(missing) / NEQ : end;
+            if (upto > base) {
+                if (i < BS && st < upto) {
+                    T x;
+                    slot_value(edge_empty(v) ? 0ull : v, x);
+                    L.edge[st % F::RING][word] = x;
                 }
-                poll(d);
+                asm volatile("" ::: "memory");
+                base = upto;
+                if (lane == 0) cnt_st(&L.cnt[LOADERS], base < nload ? base : 0x7fffffff);
+                spin = 0;
+            } else if (base < lim && ++spin > EDGE_SPIN_MAX) {
+                broken = true;
+                if (lane == 0) atomicOr(w.stall, 1);
             }
         }
         return;
