@@ -3,6 +3,7 @@
 // the reference's lrelax / lusgs call sites.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <chrono>
 #include <cmath>
 #include <cstdio>
@@ -218,6 +219,8 @@ static smac_status alloc_one_ws(smac_handle *h, int rows, int neqs, LusgsWs &w)
     return SMAC_OK;
 }
 
+static bool has_sa(const smac_handle *h) { return h->dp.ivis == 1 && h->dp.iturb == 1; }
+
 // LU-SGS workspaces: the mean flow (neqs = 3) and the SA (neqs = 1), which may run at once
 static smac_status alloc_lusgs_ws(smac_handle *h, int rows)
 {
@@ -229,6 +232,10 @@ static smac_status alloc_lusgs_ws(smac_handle *h, int rows)
     if (rc) return rc;
     rc = alloc_one_ws(h, rows, 1, h->lws_sa);
     if (rc) return rc;
+    if (has_sa(h)) {
+        h->lws.beside = h->lws_sa.nband;
+        h->lws_sa.beside = h->lws.nband;
+    }
     h->lusgs_rows = rows;
     return SMAC_OK;
 }
@@ -1055,9 +1062,14 @@ smac_status smac_adjoint(smac_handle *h, int nshape, const double *dx, const dou
         c2.ws = h->adj_ws2;
     }
     HIP_TRY(hipStreamSynchronize(h->stream));   // the operator and factors are built
-    std::thread cd([&]() { its[1] = adj_gmres(c2, c.g[1], c.lam[1], maxit, tol, &rel[1]); });
+    auto solve_cd = [&]() { its[1] = adj_gmres(c2, c.g[1], c.lam[1], maxit, tol, &rel[1]); };
+    // both solves' bands on the chip at once, or (1920 rows and more) one solve after the other
+    const bool both = h->p.impsch == 1 || lusgs_bands_fit(2 * h->adj_ws.nband);
+    std::thread cd;
+    if (both) cd = std::thread(solve_cd);
     its[0] = adj_gmres(c, c.g[0], c.lam[0], maxit, tol, &rel[0]);
-    cd.join();
+    if (both) cd.join();
+    else solve_cd();
     HIP_TRY(hipStreamSynchronize(h->stream_sa));
     adj_gradients(c, nshape, dx, dy, dcl, dcd);
     HIP_TRY(hipGetLastError());
@@ -1228,7 +1240,6 @@ static void free_multi(smac_batch *b)
     } while (0)
 
 static bool is_lusgs(const smac_handle *h) { return h->p.impsch == 2; }
-static bool has_sa(const smac_handle *h) { return h->dp.ivis == 1 && h->dp.iturb == 1; }
 
 // frees the device tables (the member list stays)
 static void free_group(BandGroup &g)
@@ -1474,9 +1485,10 @@ static smac_status enqueue_batch_pass_multi(smac_batch *b, bool time_band)
     multi_shear<double, 1>(ss, b->sa_shear);
     BandGroup &gs = b->sa;
     if (gs.nblk) {
-        lusgs_band_multi<double, 1>(ss, gs.jobs, gs.map, gs.nblk, true, b->active);
+        const int beside = std::max(b->mean[0].nblk, b->mean[1].nblk);
+        lusgs_band_multi<double, 1>(ss, gs.jobs, gs.map, gs.nblk, beside, true, b->active);
         multi_mid<double, 1>(ss, b->sa_mid);
-        lusgs_band_multi<double, 1>(ss, gs.jobs, gs.map, gs.nblk, false, b->active);
+        lusgs_band_multi<double, 1>(ss, gs.jobs, gs.map, gs.nblk, beside, false, b->active);
     }
     multi_unshear<double, 1>(ss, b->sa_unshear);
     multi_wake(ss, b->sa_wake);
@@ -1498,15 +1510,15 @@ static smac_status enqueue_batch_pass_multi(smac_batch *b, bool time_band)
         const bool rec = time_band && g == b->band_group;
         if (rec) HIP_TRY(hipEventRecord(b->ev_band[0], sm));
         if (g == 0)
-            lusgs_band_multi<double, 3>(sm, gm.jobs, gm.map, gm.nblk, true, b->active);
+            lusgs_band_multi<double, 3>(sm, gm.jobs, gm.map, gm.nblk, gs.nblk, true, b->active);
         else
-            lusgs_band_multi<float, 3>(sm, gm.jobs, gm.map, gm.nblk, true, b->active);
+            lusgs_band_multi<float, 3>(sm, gm.jobs, gm.map, gm.nblk, gs.nblk, true, b->active);
         if (rec) HIP_TRY(hipEventRecord(b->ev_band[1], sm));
         if (g == 0) {
             multi_mid<double, 3>(sm, b->mid[0]);
-            lusgs_band_multi<double, 3>(sm, gm.jobs, gm.map, gm.nblk, false, b->active);
+            lusgs_band_multi<double, 3>(sm, gm.jobs, gm.map, gm.nblk, gs.nblk, false, b->active);
         } else {
-            lusgs_band_multi<float, 3>(sm, gm.jobs, gm.map, gm.nblk, false, b->active);
+            lusgs_band_multi<float, 3>(sm, gm.jobs, gm.map, gm.nblk, gs.nblk, false, b->active);
         }
     }
     multi_unshear<double, 3>(sm, b->unshear[0]);
@@ -1562,7 +1574,7 @@ static smac_status enqueue_batch_pass(smac_batch *b, bool time_band,
     B_TRY(join_lanes(b));
     BandGroup &gs = b->sa;
     if (gs.nblk) {
-        lusgs_band_multi<double, 1>(sm, gs.jobs, gs.map, gs.nblk, true, act);
+        lusgs_band_multi<double, 1>(sm, gs.jobs, gs.map, gs.nblk, 0, true, act);
         B_TRY(fork_lanes(b));
         for (size_t n = 0; n < gs.members.size(); ++n) {
             if (!runs(gs.members[n])) continue;
@@ -1570,7 +1582,7 @@ static smac_status enqueue_batch_pass(smac_batch *b, bool time_band,
             lusgs_mid<double, 1>(lane_of(gs.members[n]), h->d, h->lws_sa);
         }
         B_TRY(join_lanes(b));
-        lusgs_band_multi<double, 1>(sm, gs.jobs, gs.map, gs.nblk, false, act);
+        lusgs_band_multi<double, 1>(sm, gs.jobs, gs.map, gs.nblk, 0, false, act);
     }
     // SA after its sweeps; mean flow up to its band sweeps (line relaxation: the whole solve)
     B_TRY(fork_lanes(b));
@@ -1615,9 +1627,9 @@ static smac_status enqueue_batch_pass(smac_batch *b, bool time_band,
         const bool rec = time_band && g == b->band_group;
         if (rec) HIP_TRY(hipEventRecord(b->ev_band[0], sm));
         if (g == 0)
-            lusgs_band_multi<double, 3>(sm, gm.jobs, gm.map, gm.nblk, true, act);
+            lusgs_band_multi<double, 3>(sm, gm.jobs, gm.map, gm.nblk, 0, true, act);
         else
-            lusgs_band_multi<float, 3>(sm, gm.jobs, gm.map, gm.nblk, true, act);
+            lusgs_band_multi<float, 3>(sm, gm.jobs, gm.map, gm.nblk, 0, true, act);
         if (rec) HIP_TRY(hipEventRecord(b->ev_band[1], sm));
         B_TRY(fork_lanes(b));
         for (int i : gm.members) {
@@ -1629,9 +1641,9 @@ static smac_status enqueue_batch_pass(smac_batch *b, bool time_band,
         }
         B_TRY(join_lanes(b));
         if (g == 0)
-            lusgs_band_multi<double, 3>(sm, gm.jobs, gm.map, gm.nblk, false, act);
+            lusgs_band_multi<double, 3>(sm, gm.jobs, gm.map, gm.nblk, 0, false, act);
         else
-            lusgs_band_multi<float, 3>(sm, gm.jobs, gm.map, gm.nblk, false, act);
+            lusgs_band_multi<float, 3>(sm, gm.jobs, gm.map, gm.nblk, 0, false, act);
     }
     B_TRY(fork_lanes(b));
     for (int i = 0; i < nc; ++i) {

@@ -73,6 +73,7 @@ template <> struct Form<3, double> {
     static constexpr int IMG = 4096, BOWN = 2304;   // a step's operands; those of the bwd chunk
     static constexpr int RG = 2304, RS = 48, RC = 16, RO = 0;   // r_c of row q: RG + q*RS + c*RC + RO
     static constexpr int RING = 24, FLY = 4;       // steps in the LDS ring; in flight per loader
+    static constexpr int SUB = 4;                   // steps between two looks at the counters
     static constexpr int AHEAD = 2;                 // steps the LDS reads run ahead
     static constexpr bool Y_BWD = false;            // forward result into the backward chunk
     static constexpr int SKEW = 0;                  // steps that four rows run behind the four before
@@ -85,6 +86,7 @@ template <> struct Form<3, float> {
     // more in flight (FLY) and the loaders, who count a step as landed FLY of their steps later,
     // run out of ring: 11 323 -> 330 us a pass, 13 486; 7 or a longer ring gains nothing
     static constexpr int RING = 48, FLY = 9;
+    static constexpr int SUB = 4;
     static constexpr int AHEAD = 2;
     static constexpr bool Y_BWD = true;
     static constexpr int SKEW = AHEAD;
@@ -95,22 +97,23 @@ template <> struct Form<1, double> {
     static constexpr int IMG = 2048, BOWN = 1024;
     static constexpr int RG = 1024, RS = 16, RC = 0, RO = 0;
     static constexpr int RING = 36, FLY = 6;
+    static constexpr int SUB = 4;
     static constexpr int AHEAD = 2;
     static constexpr bool Y_BWD = false;
     static constexpr int SKEW = 0;
-    static constexpr int EDGE = 4;
+    static constexpr int EDGE = 1;
 };
 
-// The FP32 form of a launch whose bands are more than two per compute unit, as a large batch's
-// are: a shorter ring, of which four fit a compute unit's 160 KB instead of two.  64 cases
-// FP32-LHS, 632 bands: forward sweep 0.69 -> 0.585 ms, a pass of all 3.383 -> 3.331 ms.  Where the
-// long rings fit they are the better: 112 bands (12 cases) 687 us a pass against 750, 224 bands
-// 1070 against 1100, 448 bands 2005 against 2009.  (One row per lane in 64-row bands, of which
-// these cases had 158, took 0.32 ms for this sweep and 3.54 for the pass: where the chip is full
-// of bands the sixteen-row ones lose in the sweeps what their hand-overs cost, and the pass gains
-// from the other kernels.)
-template <int NEQ, typename T> struct FormMany : Form<NEQ, T> {};
+// The forms of large launches (see band_form for the rule).  FormMost: a shorter ring, of which
+// four fit a compute unit's 160 KB instead of two.
+template <int NEQ, typename T> struct FormMany;
 template <> struct FormMany<3, float> : Form<3, float> {
+    static constexpr int RING = 36, FLY = 6;
+};
+template <> struct FormMany<1, double> : Form<1, double> {
+    static constexpr int RING = 18, FLY = 4, SUB = 2;
+};
+struct FormMost : Form<3, float> {
     static constexpr int RING = 24, FLY = 4;
 };
 
@@ -527,7 +530,6 @@ template <int NEQ> static unsigned mid_blocks(const LusgsWs &w)
 // with one row per lane,
 // 64-row bands and an s_barrier per step it took 318, 215 and 130-150 us (whose step moved 15 KB
 // through one CU, next to 51 FP64 operations in every lane); at 1889x481 848 -> 438 us FP64.
-constexpr int SUB = 4;           // steps between two looks at the counters
 constexpr int LOADERS = 3;       // loader wavefronts, each taking every third step
 constexpr int BAND_WAVES = 2 + LOADERS;
 
@@ -812,11 +814,12 @@ static __device__ __forceinline__ bool ring_round(Fn &f, std::integer_sequence<i
 template <int NEQ, bool FWD, typename T, class F = Form<NEQ, T>>
 SMAC_DEV void band_run(const Dims &d, const LusgsWs &w, int blk)
 {
-    static_assert(F::RING % SUB == 0 && F::RING % LOADERS == 0 && F::RING % (F::AHEAD + 1) == 0 && F::RING - F::FLY * LOADERS > 2 * SUB,
+    static_assert(F::RING % F::SUB == 0 && F::RING % LOADERS == 0 && F::RING % (F::AHEAD + 1) == 0 &&
+                      F::RING - F::FLY * LOADERS > 2 * F::SUB,
                   "ring");
     constexpr int NDMA = (F::IMG + 1023) / 1024;
     static_assert(F::FLY * NDMA <= 63, "vmcnt budget");
-    static_assert(SUB + F::AHEAD + 3 * F::SKEW <= OVER<F> && OVER<F> <= HP0,
+    static_assert(F::SUB + F::AHEAD + 3 * F::SKEW <= OVER<F> && OVER<F> <= HP0,
                   "the sweeps run past their ends within the padding");
     __shared__ BandLds<F, T> L;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nband = w.nband;
@@ -828,6 +831,7 @@ SMAC_DEV void band_run(const Dims &d, const LusgsWs &w, int blk)
     const int h0 = FWD ? k0 : d.jm - 1 + klast;
     const int nsteps = d.jm - 1 + nrow + (nrow - 1) / 4 * F::SKEW;
     auto behind = [&](int q) { return q / 4 * F::SKEW; };   // steps that row slot q runs behind
+    constexpr int SUB = F::SUB;
     const int nexec = (nsteps + SUB - 1) / SUB * SUB, nload = nexec + F::AHEAD;
     // row slot q of the band, in sweep order: the row that takes the hand-over is slot 0; slots
     // without a row work on the padding row ks - 1
@@ -1015,11 +1019,11 @@ SMAC_DEV void band_run(const Dims &d, const LusgsWs &w, int blk)
     while (ring_round(one, std::make_integer_sequence<int, F::RING>{})) {}
 }
 
-template <int NEQ, bool FWD, typename T>
+template <int NEQ, bool FWD, typename T, class F>
 __global__ void __launch_bounds__(BAND_LANES * BAND_WAVES)
 k_band(Dims d, LusgsWs w)
 {
-    band_run<NEQ, FWD, T>(d, w, (int)blockIdx.x);
+    band_run<NEQ, FWD, T, F>(d, w, (int)blockIdx.x);
 }
 
 // The bands of several cases in one launch: workgroup i runs band map[i].y of case map[i].x.
@@ -1081,33 +1085,78 @@ void lusgs_pre(hipStream_t sm, const Dims &d, const LusgsWs &w, const double *rh
                        d, w, rhs, btc, bjm, bkm, bjp, bkp, fac);
 }
 
+// The form of a launch of nblk bands beside which a launch of `beside` bands of the other system
+// may run (launch gets it, and LDS to ask for beyond the kernel's own).
+//
+// A band waits for the band before it, which its launch dispatched earlier.  That one makes its
+// way as long as the bands of the other launch, which wait for one another too, do not hold every
+// place it could take.  As long as lusgs_bands_fit none does.  Beyond that the scalar system's bands take a ring small enough, and the
+// mean flow's one large enough (FormMost asks for more LDS than it uses), that the units which
+// hold all the mean-flow bands they can have room for one of the scalar system's: those end then,
+// and with them what holds up the others.  In the other forms a unit with a scalar band has no
+// room for an FP64 one, and one full of FP32 bands none for a scalar one.
+//
+// A pass, in the forms of a single case and in these: 26 cases FP64 (276 + 69 bands) 2270 and 2290
+// us, 64 cases (632 + 158) 5089 and 5095; FP32-LHS 16 of 945x241 (256 + 64) 1722 and 1696, 32 of
+// them (512 + 128) 3301 and 3298, 32 cases (340 + 85) 1958 and 1973, 64 cases 3396 and 3334; below,
+// 12 cases (124 + 31) 825 and 856.  Alone, FP32 past two bands a unit takes the shortest ring: 64
+// cases without the SA 2580 and 2541 us.  (One row per lane in 64-row bands, of which the 64 cases
+// had 158, took 0.32 ms for a forward sweep of theirs beside the SA, and 3.54 for a pass.  It takes
+// 0.48 now: on a chip full of bands the sixteen-row ones lose their gain to hand-overs.)
+constexpr int LDS_UNIT = 160 * 1024, LDS_GRAIN = 1280;
+constexpr int lds_grains(int bytes) { return (bytes + LDS_GRAIN - 1) / LDS_GRAIN * LDS_GRAIN; }
+template <class F, typename T> constexpr int lds_of(int room = 0)
+{
+    return lds_grains((int)sizeof(BandLds<F, T>) + room);
+}
+constexpr int MOST_ROOM = LDS_UNIT / 4 + 16 - (int)sizeof(BandLds<FormMost, float>);
+constexpr bool leaves_room(int mean)
+{
+    return LDS_UNIT % mean >= lds_of<FormMany<1, double>, double>();
+}
+static_assert(leaves_room(lds_of<Form<3, double>, double>()), "FP64");
+static_assert(leaves_room(lds_of<FormMany<3, float>, float>()), "FP32");
+static_assert(leaves_room(lds_of<FormMost, float>(MOST_ROOM)), "FP32, many");
+
+template <typename LT, int NEQ, class Launch>
+static void band_form(int nblk, int beside, Launch launch)
+{
+    const bool crowd = beside > 0 && !lusgs_bands_fit(nblk + beside);
+    if constexpr (NEQ == 3 && sizeof(LT) == 4) {
+        if (nblk > 2 * LUSGS_UNITS) return launch(FormMost{}, crowd ? MOST_ROOM : 0);
+    }
+    if constexpr (NEQ == 1 || sizeof(LT) == 4) {
+        if (crowd) return launch(FormMany<NEQ, LT>{}, 0);
+    }
+    launch(Form<NEQ, LT>{}, 0);
+}
+
 template <typename LT, int NEQ>
 void lusgs_band(hipStream_t sm, const Dims &d, const LusgsWs &w, bool fwd)
 {
     const dim3 blk(BAND_LANES * BAND_WAVES);
-    if (fwd)
-        hipLaunchKernelGGL((k_band<NEQ, true, LT>), dim3(w.nband), blk, 0, sm, d, w);
-    else
-        hipLaunchKernelGGL((k_band<NEQ, false, LT>), dim3(w.nband), blk, 0, sm, d, w);
+    band_form<LT, NEQ>(w.nband, w.beside, [&](auto form, int room) {
+        using F = decltype(form);
+        if (fwd)
+            hipLaunchKernelGGL((k_band<NEQ, true, LT, F>), dim3(w.nband), blk, room, sm, d, w);
+        else
+            hipLaunchKernelGGL((k_band<NEQ, false, LT, F>), dim3(w.nband), blk, room, sm, d, w);
+    });
 }
 
 template <typename LT, int NEQ>
-void lusgs_band_multi(hipStream_t sm, const BandJob *jobs, const int2 *map, int nblk, bool fwd,
-                      const int *active)
+void lusgs_band_multi(hipStream_t sm, const BandJob *jobs, const int2 *map, int nblk, int beside,
+                      bool fwd, const int *active)
 {
     if (nblk <= 0) return;
     const dim3 blk(BAND_LANES * BAND_WAVES);
-    constexpr int FULL = 2 * 256;   // two bands on each compute unit
-    auto launch = [&](auto form) {
+    band_form<LT, NEQ>(nblk, beside, [&](auto form, int room) {
         using F = decltype(form);
         if (fwd)
-            hipLaunchKernelGGL((k_band_multi<NEQ, true, LT, F>), dim3(nblk), blk, 0, sm, jobs, map, active);
+            hipLaunchKernelGGL((k_band_multi<NEQ, true, LT, F>), dim3(nblk), blk, room, sm, jobs, map, active);
         else
-            hipLaunchKernelGGL((k_band_multi<NEQ, false, LT, F>), dim3(nblk), blk, 0, sm, jobs, map, active);
-    };
-    if constexpr (FormMany<NEQ, LT>::RING < Form<NEQ, LT>::RING)
-        if (nblk > FULL) return launch(FormMany<NEQ, LT>{});
-    launch(Form<NEQ, LT>{});
+            hipLaunchKernelGGL((k_band_multi<NEQ, false, LT, F>), dim3(nblk), blk, room, sm, jobs, map, active);
+    });
 }
 
 template <typename LT, int NEQ>
@@ -1258,7 +1307,7 @@ void launch_lusgs1(hipStream_t sm, const Dims &d, const LusgsWs &w, const WakePa
                                      LT *);                                                    \
     template void lusgs_band<LT, NEQ>(hipStream_t, const Dims &, const LusgsWs &, bool);       \
     template void lusgs_band_multi<LT, NEQ>(hipStream_t, const BandJob *, const int2 *, int,   \
-                                            bool, const int *);                                \
+                                            int, bool, const int *);                                \
     template void lusgs_mid<LT, NEQ>(hipStream_t, const Dims &, const LusgsWs &);              \
     template void lusgs_post<LT, NEQ>(hipStream_t, const Dims &, const LusgsWs &,              \
                                       const WakePairs &, const double *, double *, double *);

@@ -91,6 +91,7 @@ void launch_lrelax_scan_t(hipStream_t, const Dims &, int njsp, int nksp, double 
 struct LusgsWs {
     int rows;                    // rows per band: 1..16 (3x3 system), 1..64 (scalar)
     int nband;                   // bands covering k = 0..km-1
+    int beside;                  // bands of another launch that may run at the same time
     int ks;                      // rows of one hyperplane, padded to whole chunks
     int H;                       // last hyperplane, jm + km - 2
     int epitch;                  // slots per band region: (jm + 2*128 padding)*4
@@ -100,6 +101,11 @@ struct LusgsWs {
     int *stall;                  // raised when a hand-over wait times out
     hipEvent_t ev_fwd[2];        // when set: recorded around the forward band sweep
 };
+// Whether n bands, of launches that may run at the same time, leave each XCD (of 8, dealt a launch's
+// workgroups in turn, with 32 compute units each) a unit without one: then the next band of each
+// launch finds its place whatever the others do.
+constexpr int LUSGS_UNITS = 256;
+inline bool lusgs_bands_fit(int n) { return n <= LUSGS_UNITS - 2 * 8; }
 // one case's part of a multi-case band launch
 struct BandJob {
     Dims d;
@@ -116,8 +122,8 @@ template <typename LT, int NEQ>
 void lusgs_band(hipStream_t, const Dims &, const LusgsWs &, bool fwd);
 // jobs and map in device memory; map[i] = (job, band in dispatch order), nblk entries
 template <typename LT, int NEQ>
-void lusgs_band_multi(hipStream_t, const BandJob *jobs, const int2 *map, int nblk, bool fwd,
-                      const int *active);
+void lusgs_band_multi(hipStream_t, const BandJob *jobs, const int2 *map, int nblk, int beside,
+                      bool fwd, const int *active);
 template <typename LT, int NEQ>
 void lusgs_mid(hipStream_t, const Dims &, const LusgsWs &);
 template <typename LT, int NEQ>

@@ -28,3 +28,18 @@ def test_many_bands_equal_alone(n, precision, iturb):
         for a, b in zip(s.get_state(), ref):
             assert np.array_equal(a, b)
         s.close()
+
+
+@pytest.mark.parametrize("precision", [SMAC_FP64, SMAC_FP32_LHS])
+@pytest.mark.parametrize("km", [119, 121, 521])
+def test_one_case_of_many_bands(km, precision):
+    # bands of one row, beside the SA's: 238, 242 and 1042 of both systems
+    case = naca_case(63, km, impsch=2, alpha=3.0, reynum=1e4, wall_spacing=1e-3, dtau=0.001,
+                     precision=precision)
+    out = []
+    for rows in (1, 64):
+        with Solver(case, options={"lusgs_rows": rows}) as s:
+            s.run(4)
+            out.append(s.get_state())
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
