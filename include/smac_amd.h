@@ -168,10 +168,9 @@ smac_status smac_timings(smac_handle *h, double out[7]);
  * smac_get_array), "timing" (1: time kernel families with HIP events on the handle's
  * stream), "lusgs_rows" (1..64, default 64: grid rows per wavefront band of the LU-SGS
  * sweeps; the 3x3 sweeps take at most 16), "lusgs_prefetch" / "lusgs_prefetch_sa" (1, 2, 3, 4,
- * 6 or 8) and "lusgs_ring" (0 or 1) (accepted, without effect: the sweeps have one form, fed
- * through an LDS ring),
- * "lr_lines" (1..64, default 64: lines per workgroup of the line-relaxation
- * factorisations), "adj_restart" (4..400, default 100: GMRES restart length of
+ * 6 or 8), "lusgs_ring" (0 or 1) and "lr_lines" (1..64) (accepted, without effect: the sweeps are
+ * fed through an LDS ring, and the lines per workgroup of the line-relaxation factorisations
+ * follow from the grid), "adj_restart" (4..400, default 100: GMRES restart length of
  * smac_adjoint), "adj_prec_steps" (1..8, default 3: steps of the transposed update per
  * application of its GMRES preconditioner, with the operator between them; more steps, fewer
  * iterations), "adj_reorth" (0..1000, default 100: its Gram-Schmidt projects a vector a

@@ -3,12 +3,13 @@
 The tunable knobs change how the work is cut into workgroups, never the arithmetic (results
 are bit-identical for every setting):
 
-* ``lusgs_rows``        grid rows per wavefront band of the LU-SGS hyperplane sweeps;
-* ``lusgs_prefetch``, ``lusgs_prefetch_sa``, ``lusgs_ring``
-                        accepted by the library without effect (the sweeps have one form), so
-                        each has one value here;
-* ``lr_lines``          lines per workgroup of the line-relaxation factorisations.
+* ``lusgs_rows``        grid rows per wavefront band of the LU-SGS hyperplane sweeps.  The 3x3
+                        sweeps take at most 16, so values from there on differ only for the
+                        scalar sweeps, and a case without them has one value;
+* ``lusgs_prefetch``, ``lusgs_prefetch_sa``, ``lusgs_ring``, ``lr_lines``
+                        accepted by the library without effect, so each has one value here.
 
+A case whose knobs have one value each is not timed.
 ``tune(case)`` times candidate settings on a private copy of the case (its own device
 state, so the caller's solver is untouched), by wall clock around ``smac_run`` (which ends
 with a device synchronisation), coordinate by coordinate, and caches the winner per device,
@@ -27,10 +28,11 @@ from .solver import Solver
 CACHE_ENV = "MINISMAC_AMD_TUNE_CACHE"
 
 LUSGS_ROWS = (16, 32, 64)
+LUSGS_ROWS_3X3 = (64,)
 LUSGS_PREFETCH = (4,)
 LUSGS_PREFETCH_SA = (8,)
 LUSGS_RING = (1,)
-LR_LINES = (8, 16, 32, 64)
+LR_LINES = (64,)
 # a setting replaces the current one only when it is faster by more than this fraction
 # (wall-clock noise of a few passes)
 MIN_GAIN = 0.02
@@ -101,7 +103,7 @@ def _space(case: Case) -> list[tuple[str, tuple]]:
     p = case.params
     sa = p.ivis == 1 and p.iturb == 1
     if p.impsch == 2:
-        dims = [("lusgs_ring", LUSGS_RING), ("lusgs_rows", LUSGS_ROWS),
+        dims = [("lusgs_ring", LUSGS_RING), ("lusgs_rows", LUSGS_ROWS if sa else LUSGS_ROWS_3X3),
                 ("lusgs_prefetch", LUSGS_PREFETCH)]
         if sa:
             dims.append(("lusgs_prefetch_sa", LUSGS_PREFETCH_SA))
@@ -123,6 +125,10 @@ def tune(case: Case, passes: int = 10, repeats: int = 2, sweeps: int = 2,
     defaults = {"lusgs_ring": 1, "lusgs_rows": 64, "lusgs_prefetch": 4, "lusgs_prefetch_sa": 8,
                 "lr_lines": 64}
     cur = {name: defaults[name] for name, _ in dims}
+    if all(len(vals) == 1 for _, vals in dims):
+        if use_cache:
+            _store(path, {**_load(path), k: {"options": cur}})
+        return dict(cur)
     probe = _Probe(case)
     try:
         t_cur = t_default = probe.time(cur, passes, repeats)

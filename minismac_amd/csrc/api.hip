@@ -72,7 +72,6 @@ struct smac_handle {
     WakePairs wake = {};
     LusgsWs lws = {};          // LU-SGS sheared workspace (impsch = 2)
     int lusgs_rows = 64;
-    int lr_lines = 64;     // lines per workgroup of the line-relaxation factor kernels
     int lr_refactor = 1;   // scan/zebra forms: factor the lines every this many passes
     long lr_factored = -1; // the pass whose blocks the line operands hold (-1: none)
     // line relaxation with each line solved by prefix scans inside the line (1), or by the
@@ -516,8 +515,7 @@ smac_status smac_set_option(smac_handle *h, const char *name, int value)
     }
     if (!std::strcmp(name, "lr_lines")) {
         if (value < 1 || value > 64) return fail(SMAC_ERR_ARG, "lr_lines must be in [1, 64]");
-        h->lr_lines = value;
-        return SMAC_OK;
+        return SMAC_OK;   // as above: the lines per workgroup follow from the grid
     }
     if (!std::strcmp(name, "adj_reorth")) {
         if (value < 0 || value > 1000) return fail(SMAC_ERR_ARG, "adj_reorth must be in [0, 1000]");
@@ -595,7 +593,7 @@ static void enqueue_lrelax(smac_handle *h, hipStream_t sm)
     h->lr_factored = !h->lr_solve ? -1 : (factor ? h->nt : h->lr_factored);
     if (!h->lr_solve)
         launch_lrelax_ref(sm, d, h->dp, h->p.njsp, h->p.nksp, h->p.nbcimp, h->wake, h->q, h->dq,
-                          h->s, btc, bjm, bjp, bkm, bkp, h->lrs.opx, h->lr_lines);
+                          h->s, btc, bjm, bjp, bkm, bkp, h->lrs.opx);
     else if (h->p.precision == SMAC_FP32_LHS)
         launch_lrelax_scan<float>(sm, d, h->dp, h->p.njsp, h->p.nksp, h->p.nbcimp, zebra, h->wake,
                                   h->q, h->dq, h->s, (const float *)btc, (const float *)bjm,

@@ -550,21 +550,15 @@ void launch_wake(hipStream_t sm, const Dims &d, int neqs, const WakePairs &w, co
 void launch_lrelax_ref(hipStream_t sm, const Dims &d, const DevParams &prm, int njsp, int nksp,
                        int nbcimp, const WakePairs &w, const double *q, double *dq, double *s,
                        double *btc, const double *bjm, double *bjp, const double *bkm,
-                       const double *bkp, void *pack, int lpb)
+                       const double *bkp, void *pack)
 {
     const long N = d.N;
     char *pk = (char *)pack;
     // lines per workgroup of the factor kernels (one lane per line): as few as leave a wave per
-    // SIMD, at most lpb -- the lanes of a wave load from as many cache lines (31 lines of 119
-    // points: 160 us in one wave, 103 us in 31)
-    auto groups = [&](int nline) {
-        const int few = (nline + 1023) / 1024, n = lpb < 1 ? 1 : (lpb < few ? lpb : few);
-        return dim3((unsigned)((nline + n - 1) / n));
-    };
-    auto lines = [&](int nline) {
-        const int few = (nline + 1023) / 1024;
-        return dim3((unsigned)(lpb < 1 ? 1 : (lpb < few ? lpb : few)));
-    };
+    // SIMD -- the lanes of a wave load from as many cache lines (31 lines of 119 points: 160 us
+    // in one wave, 103 us in 31)
+    auto lines = [](int nline) { return (unsigned)((nline + 1023) / 1024); };
+    auto groups = [&](int nline) { return (nline + lines(nline) - 1) / lines(nline); };
     auto sweep = [&](int eta, int ns, const double *om, const double *op) {
         const int len = eta ? d.km : d.jm;
         const size_t lds = sizeof(double) * 3 * ((len + RB - 1) / RB * RB) + 4 * (1 + (len + 63) / 64);
@@ -574,14 +568,14 @@ void launch_lrelax_ref(hipStream_t sm, const Dims &d, const DevParams &prm, int 
     };
     hipLaunchKernelGGL(k_fill, dim3(256), dim3(256), 0, sm, dq, 3 * N, 0.0);
     if (njsp > 0)
-        hipLaunchKernelGGL(k_btlu3<double>, groups(d.km), lines(d.km), 0, sm, N, d.km,
+        hipLaunchKernelGGL(k_btlu3<double>, dim3(groups(d.km)), dim3(lines(d.km)), 0, sm, N, d.km,
                            d.jm, 1L, (long)d.jm, bjm, btc, bjp, pk);
     for (int nj = 1; nj <= njsp; ++nj) sweep(0, nj, bkm, bkp);
     if (njsp > 0)
         hipLaunchKernelGGL(k_btund3<double>, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, sm, N,
                            d.jm, bjm, btc, bjp, pk);
     if (nksp > 0)
-        hipLaunchKernelGGL(k_btlu3<double>, groups(d.jm), lines(d.jm), 0, sm, N, d.jm,
+        hipLaunchKernelGGL(k_btlu3<double>, dim3(groups(d.jm)), dim3(lines(d.jm)), 0, sm, N, d.jm,
                            d.km, (long)d.jm, 1L, bkm, btc, bkp, pk);
     for (int nk = 1; nk <= nksp; ++nk) sweep(1, nk, bjm, bjp);
 }

@@ -51,7 +51,7 @@ long lr_ref_bytes(const Dims &);
 void launch_lrelax_ref(hipStream_t, const Dims &, const DevParams &, int njsp, int nksp,
                        int nbcimp, const WakePairs &, const double *q, double *dq, double *s,
                        double *btc, const double *bjm, double *bjp, const double *bkm,
-                       const double *bkp, void *pack, int lines_per_block = 64);
+                       const double *bkp, void *pack);
 void launch_wake(hipStream_t, const Dims &, int neqs, const WakePairs &, const double *sq,
                  double *ds, double *rhs);
 

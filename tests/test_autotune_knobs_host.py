@@ -1,0 +1,25 @@
+"""The autotuner's choices (no GPU): a knob has several values only where they differ, and a case
+with nothing to choose starts no timing run."""
+import pytest
+
+from minismac_amd import autotune
+from minismac_amd._abi import SMAC_FP32_LHS, SMAC_ORDER_ZEBRA
+from minismac_amd.case import config_case
+
+
+@pytest.mark.parametrize("kw", [dict(impsch=2, iturb=0), dict(impsch=2, ivis=0),
+                                dict(impsch=2, iturb=0, precision=SMAC_FP32_LHS), dict(impsch=1),
+                                dict(impsch=1, line_order=SMAC_ORDER_ZEBRA)])
+def test_nothing_to_choose_is_not_timed(tmp_path, monkeypatch, kw):
+    def no_probe(*a, **k):
+        raise AssertionError("a timing run of settings that launch the same kernels")
+
+    monkeypatch.setattr(autotune, "_Probe", no_probe)
+    case, path = config_case(0, **kw), str(tmp_path / "tune.json")
+    opts = autotune.tune(case, path=path)
+    assert opts == {name: vals[0] for name, vals in autotune._space(case)}
+    assert autotune._load(path)[autotune.key(case)]["options"] == opts
+
+
+def test_scalar_sweeps_have_rows_to_choose():
+    assert len(dict(autotune._space(config_case(0, impsch=2)))["lusgs_rows"]) > 1
