@@ -13,17 +13,20 @@ A case whose knobs have one value each is not timed.
 ``tune(case)`` times candidate settings on a private copy of the case (its own device
 state, so the caller's solver is untouched), by wall clock around ``smac_run`` (which ends
 with a device synchronisation), coordinate by coordinate, and caches the winner per device,
-grid size, scheme and precision in a JSON file.  ``tune_cases`` tunes each distinct
+library build, grid size, scheme and precision in a JSON file: another build's kernels may
+have other best settings, so its entries are left alone.  ``tune_cases`` tunes each distinct
 (size, scheme, precision) of a list once; ``apply`` sets the options on a solver.
 """
 from __future__ import annotations
 
+import functools
+import hashlib
 import json
 import os
 import time
 
 from .case import Case
-from .solver import Solver
+from .solver import LIB_PATH, Solver
 
 CACHE_ENV = "MINISMAC_AMD_TUNE_CACHE"
 
@@ -51,10 +54,20 @@ def _device_name() -> str:
         return "unknown"
 
 
+@functools.lru_cache(maxsize=None)
+def _build_of(path: str) -> str:
+    # a process loads the library once, so its bytes are read once too
+    try:
+        with open(path, "rb") as f:
+            return hashlib.sha256(f.read()).hexdigest()[:12]
+    except OSError:
+        return "unknown"
+
+
 def key(case: Case) -> str:
     p = case.params
     sa = int(p.ivis == 1 and p.iturb == 1)
-    return f"{_device_name()}|{case.jmax}x{case.kmax}|impsch{p.impsch}|prec{p.precision}|sa{sa}"
+    return f"{_device_name()}|build {_build_of(LIB_PATH)}|{case.jmax}x{case.kmax}|impsch{p.impsch}|prec{p.precision}|sa{sa}"
 
 
 def _load(path: str) -> dict:

@@ -23,3 +23,17 @@ def test_nothing_to_choose_is_not_timed(tmp_path, monkeypatch, kw):
 
 def test_scalar_sweeps_have_rows_to_choose():
     assert len(dict(autotune._space(config_case(0, impsch=2)))["lusgs_rows"]) > 1
+
+
+def test_settings_of_another_build_are_not_taken(tmp_path, monkeypatch):
+    case = config_case(0, impsch=2)
+    builds = [tmp_path / "a.so", tmp_path / "b.so"]
+    keys = []
+    for i, b in enumerate(builds):
+        b.write_bytes(b"build %d" % i)
+        monkeypatch.setattr(autotune, "LIB_PATH", str(b))
+        keys.append(autotune.key(case))
+    assert keys[0] != keys[1] and all("119x31" in k for k in keys)
+    # an entry of a version whose keys did not name the build
+    sa = int(case.params.ivis == 1 and case.params.iturb == 1)
+    assert f"{autotune._device_name()}|119x31|impsch2|prec0|sa{sa}" not in keys
