@@ -300,8 +300,8 @@ k_sweep_ref(Dims d, int eta, int nsweep, double underr, double *__restrict__ dq,
 
     if (wave > 0) {
         const double half = 0.5;
-        // the right-hand side of line l at point i, with dq of the line solved before it (lnew,
-        // -1: none) in xn
+        // the update of the line just solved (l, -1: none yet), then the right-hand side of the next
+        // (ln, -1: none), with x and y the dq of the lines on its two sides
         for (int ll = -1; ll < nline; ++ll) {
             const int l = ll < 0 ? -1 : line_of(ll), ln = ll + 1 < nline ? line_of(ll + 1) : -1;
             const int lmn = ln - 1 > 0 ? ln - 1 : 0;

@@ -409,8 +409,7 @@ static int lines_per_group(int nline, bool twist) { return nline * (twist ? 2 : 
 // the sweep: lines count of them, line l = (first + idx*step) mod nline, one workgroup per line
 // (lines of one colour); k_lr_walk below takes them in order in one workgroup.
 // s, dq: NEQ planes, line-major; op: the factor kernel's planes.  assign: dq = x (the SA's
-// lreltur); otherwise dq += underr (x - dq) (ref/lrelax.f:377-381).  couple = 0 leaves out
-// the neighbouring lines' terms: a plain solve of each line (the transposed sweeps).
+// lreltur); otherwise dq += underr (x - dq) (ref/lrelax.f:377-381).
 //
 // The solve follows the twisted factorisation (mid = len/2):
 //   phase 1  y_i = M_i y_(i-1) + T_i^-1 r_i  forward over i < mid, and
@@ -587,7 +586,7 @@ struct LrTStep {
 template <typename LT, int NEQ, int NT, int PP, bool TWIST, bool TRANS>
 __global__ void __launch_bounds__(NT)
 k_lr_sweep(int nline, int len, long N, int count, int first, int step, double underr,
-           int assign, int couple, double *__restrict__ dq, const double *__restrict__ s,
+           int assign, double *__restrict__ dq, const double *__restrict__ s,
            const LT *__restrict__ op, LrTStep ts)
 {
     using AT = LT;
@@ -612,7 +611,7 @@ k_lr_sweep(int nline, int len, long N, int count, int first, int step, double un
     };
     for (int idx = (int)blockIdx.x; idx < count; idx += (int)gridDim.x) {
         const int l = (first + idx * step) % nline;
-        const bool hm = (TRANS || couple) && l > 0, hp = (TRANS || couple) && l < nline - 1;
+        const bool hm = l > 0, hp = l < nline - 1;
         AT mmat[PP][NB];               // M (Ma at mid)
         AT bv[PP][NEQ];                // T^-1 r
         AT w[PP][NEQ];                 // y (i < mid) or z (i > mid); z_(mid+1), then x_mid, at
@@ -632,7 +631,7 @@ k_lr_sweep(int nline, int len, long N, int count, int first, int step, double un
                 r[u][n] = (TRANS ? ts.a : s)[n * N + nat(l, u)];
                 if constexpr (TRANS) sb[u][n] = ts.begin ? 0.0 : ts.sbar[n * N + nat(l, u)];
             }
-        if (TRANS ? ts.spread : couple) {
+        if (!TRANS || ts.spread) {
             AT om[PP][NB], op_[PP][NB];
             double xm[PP][NEQ], xp[PP][NEQ];
             load_planes(om, pOm + lo, N);
@@ -1301,7 +1300,7 @@ enum SweepForm { SWEEP_COLOUR, SWEEP_WALK, SWEEP_TRANSPOSED };
 template <typename LT, int NEQ, SweepForm FORM>
 static void sweep_launch(hipStream_t sm, int nline, int len, long N, int count, int first,
                          int step, double underr, int assign, double *dq, const double *s,
-                         const LT *op, int couple, bool twist, const LrTStep &ts = {})
+                         const LT *op, bool twist, const LrTStep &ts = {})
 {
 #define SWT(LAUNCH)                                                                             \
     do {                                                                                       \
@@ -1319,7 +1318,7 @@ static void sweep_launch(hipStream_t sm, int nline, int len, long N, int count, 
                        count, first, step, underr, dq, s, op)
 #define COLOUR(NT, PPV, TW, TR)                                                                 \
     hipLaunchKernelGGL((k_lr_sweep<LT, NEQ, NT, PPV, TW, TR>), dim3(count), dim3(NT), 0, sm,    \
-                       nline, len, N, count, first, step, underr, assign, couple, dq, s, op, ts)
+                       nline, len, N, count, first, step, underr, assign, dq, s, op, ts)
 #define TWISTED(NT, PPV) COLOUR(NT, PPV, true, false)
 #define PLAIN(NT, PPV) COLOUR(NT, PPV, false, false)
 #define TRANSPOSED(NT, PPV) COLOUR(NT, PPV, false, true)
@@ -1355,14 +1354,14 @@ static void sweep(hipStream_t sm, int nline, int len, long N, int nsweep, bool z
 {
     if (zebra) {
         sweep_launch<LT, NEQ, SWEEP_COLOUR>(sm, nline, len, N, (nline + 1) / 2, 0, 2, underr, 0, dq, s,
-                                     op, 1, twist);
-        sweep_launch<LT, NEQ, SWEEP_COLOUR>(sm, nline, len, N, nline / 2, 1, 2, underr, 0, dq, s, op, 1,
+                                     op, twist);
+        sweep_launch<LT, NEQ, SWEEP_COLOUR>(sm, nline, len, N, nline / 2, 1, 2, underr, 0, dq, s, op,
                                      twist);
         return;
     }
     const bool rev = (nsweep / 2) * 2 == nsweep;
     sweep_launch<LT, NEQ, SWEEP_WALK>(sm, nline, len, N, nline, rev ? nline - 1 : 0, rev ? -1 : 1,
-                                underr, 0, dq, s, op, 1, false);
+                                underr, 0, dq, s, op, false);
 }
 
 long lr_scan_bytes(const Dims &d)
@@ -1483,7 +1482,7 @@ static void tsweep(hipStream_t sm, int nline, int len, long N, int nsweep, doubl
             const int count = par ? nline / 2 : (nline + 1) / 2;
             if (count > 0)
                 sweep_launch<LT, 3, SWEEP_TRANSPOSED>(sm, nline, len, N, count, par, 2, 1.0, 1, z,
-                                                      nullptr, op, 0, false, ts);
+                                                      nullptr, op, false, ts);
         }
 }
 
@@ -1521,14 +1520,14 @@ void launch_sa_lreltur_scan(hipStream_t sm, const Dims &d, int ntjsp, const Wake
     for (int pass = 1; pass <= ntjsp; ++pass) {
         if (ws.zebra) {
             sweep_launch<double, 1, SWEEP_COLOUR>(sm, d.km, d.jm, d.N, (d.km + 1) / 2, 0, 2, 1.0, 1,
-                                           a.ds, a.sf, ws.sa_op, 1, true);
+                                           a.ds, a.sf, ws.sa_op, true);
             sweep_launch<double, 1, SWEEP_COLOUR>(sm, d.km, d.jm, d.N, d.km / 2, 1, 2, 1.0, 1, a.ds,
-                                           a.sf, ws.sa_op, 1, true);
+                                           a.sf, ws.sa_op, true);
             sweep_launch<double, 1, SWEEP_COLOUR>(sm, d.km, d.jm, d.N, 1, 0, 1, 1.0, 1, a.ds, a.sf,
-                                           ws.sa_op, 1, true);
+                                           ws.sa_op, true);
         } else {
             sweep_launch<double, 1, SWEEP_WALK>(sm, d.km, d.jm, d.N, d.km + 1, 0, 1, 1.0, 1, a.ds, a.sf,
-                                          ws.sa_op, 1, false);
+                                          ws.sa_op, false);
         }
         launch_wake(sm, d, 1, w, a.anut, a.ds, a.sf);
     }
