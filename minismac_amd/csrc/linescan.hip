@@ -130,7 +130,7 @@ template <int OFF, bool UP> SMAC_DEV double lane_shift(double v, int lane)
 // The bound is the issue of those instructions, one per 5 cycles for a wave alone on its SIMD,
 // over half the longest line.  Broadcasting every point's blocks through LDS to a recurrence
 // that all lanes form alike took 238 us at 945x241 in FP64 and 116 at 705x173 in FP32; this
-// takes 160 and 92 (reference-order FP32 945x241, whole lines: 287 and 255).
+// takes 152 and 91 (reference-order FP32 945x241, whole lines: 287 and 255).
 // (The reference keeps T_i as LU factors; the explicit inverse makes the sweeps' T_i^-1 r_i a
 // parallel product.)  The blocks to the neighbouring lines pass through to the operand planes.
 

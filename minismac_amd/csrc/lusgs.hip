@@ -508,14 +508,14 @@ template <int NEQ> static unsigned mid_blocks(const LusgsWs &w)
 // does not wait back, so they end: a loader waits for the computing wave's progress, the
 // computing wave for the counters, and the hand-over wave, whose polls are bounded (on
 // time-out it raises the stall flag and hands zeros on), for the band before, which was
-// dispatched earlier.
+// dispatched earlier and finds a place whatever other launches hold (band_form).
 //
 // What bounds a sweep: its chain of jmax + kmax - 1 steps, each as long as the computing
 // wavefront takes to issue it -- a wavefront alone on its SIMD issues one VALU instruction
 // per 5 cycles (measured), so about 68 instructions FP64 make 144 ns, 22 FP32 60 ns -- and the
 // hand-over lag of 2 us per band beyond the 16 rows' own skew.  The hand-over wavefront shares
-// the computing one's SIMD, which therefore runs at a higher priority (backward sweep 218 -> 209
-// us, an LU-SGS solve at 477x121 253.5 -> 250).
+// the computing one's SIMD, which therefore runs at a higher priority (with four polls in flight,
+// as once: backward sweep 218 -> 209 us, an LU-SGS solve at 477x121 253.5 -> 250; now 204 and 242).
 //
 // The FP32 step has no 3x3 substitution, so what it issued was mostly moves: three results
 // broadcast in the quad, each passed to the next row by two moves (one inside a row of 16 lanes,
@@ -526,9 +526,8 @@ template <int NEQ> static unsigned mid_blocks(const LusgsWs &w)
 // us, each sweep 112 -> 105.  FP64 keeps the moves: it would save 4 of 68 instructions and pay
 // 8% more steps.
 //
-// At 945x241 the forward sweep takes 215 us FP64, 105 us FP32 and 64 us for the scalar system;
-// with one row per lane,
-// 64-row bands and an s_barrier per step it took 318, 215 and 130-150 us (whose step moved 15 KB
+// At 945x241 the forward sweep takes 211 us FP64, 105 us FP32 and 64 us for the scalar system;
+// with one row per lane, 64-row bands and an s_barrier per step it took 318, 215 and 130-150 us (whose step moved 15 KB
 // through one CU, next to 51 FP64 operations in every lane); at 1889x481 848 -> 438 us FP64.
 constexpr int LOADERS = 3;       // loader wavefronts, each taking every third step
 constexpr int BAND_WAVES = 2 + LOADERS;
