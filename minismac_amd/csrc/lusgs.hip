@@ -1087,13 +1087,14 @@ void lusgs_pre(hipStream_t sm, const Dims &d, const LusgsWs &w, const double *rh
 // The form of a launch of nblk bands beside which a launch of `beside` bands of the other system
 // may run (launch gets it, and LDS to ask for beyond the kernel's own).
 //
-// A band waits for the band before it, which its launch dispatched earlier.  That one makes its
-// way as long as the bands of the other launch, which wait for one another too, do not hold every
-// place it could take.  As long as lusgs_bands_fit none does.  Beyond that the scalar system's bands take a ring small enough, and the
-// mean flow's one large enough (FormMost asks for more LDS than it uses), that the units which
-// hold all the mean-flow bands they can have room for one of the scalar system's: those end then,
-// and with them what holds up the others.  In the other forms a unit with a scalar band has no
-// room for an FP64 one, and one full of FP32 bands none for a scalar one.
+// A band waits for the band before it, which its launch dispatched earlier.  That one makes its way
+// as long as the bands of the other launch, which wait for one another too, do not hold every place
+// it could take.  As long as lusgs_bands_fit none does.  Beyond that the scalar system's bands take
+// a ring small enough, and the mean flow's one large enough (FormMost asks for more LDS than it
+// uses), that the units which hold all the mean-flow bands they can have room (and registers) for
+// one of the scalar system's: those end then, and with them what holds up the others.  In the other
+// forms a unit with a scalar band has no room for an FP64 one, and one full of FP32 bands none for a
+// scalar one.
 //
 // A pass, in the forms of a single case and in these: 26 cases FP64 (276 + 69 bands) 2270 and 2290
 // us, 64 cases (632 + 158) 5089 and 5095; FP32-LHS 16 of 945x241 (256 + 64) 1722 and 1696, 32 of
