@@ -1098,9 +1098,9 @@ void lusgs_pre(hipStream_t sm, const Dims &d, const LusgsWs &w, const double *rh
 //
 // A pass, in the forms of a single case and in these: 26 cases FP64 (276 + 69 bands) 2270 and 2290
 // us, 64 cases (632 + 158) 5089 and 5095; FP32-LHS 16 of 945x241 (256 + 64) 1722 and 1696, 32 of
-// them (512 + 128) 3301 and 3298, 32 cases (340 + 85) 1958 and 1973, 64 cases 3396 and 3334; below,
-// 12 cases (124 + 31) 825 and 856.  Alone, FP32 past two bands a unit takes the shortest ring: 64
-// cases without the SA 2580 and 2541 us.  (One row per lane in 64-row bands, of which the 64 cases
+// them (512 + 128) 3301 and 3298, 32 cases (340 + 85) 1958 and 1973, 64 cases 3344 (the shortest
+// ring, four bands a unit) and 3334; below, 12 cases (124 + 31) 825 and 856.  Alone, FP32 past two
+// bands a unit takes the shortest ring: 64 cases without the SA 2580 and 2541 us.  (One row per lane in 64-row bands, of which the 64 cases
 // had 158, took 0.32 ms for a forward sweep of theirs beside the SA, and 3.54 for a pass.  It takes
 // 0.48 now: on a chip full of bands the sixteen-row ones lose their gain to hand-overs.)
 constexpr int LDS_UNIT = 160 * 1024, LDS_GRAIN = 1280;
